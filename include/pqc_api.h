@@ -75,20 +75,24 @@ int pqc_ctx_set_tuning(pqc_ctx *ctx, int fused_waves_per_cu, int fused_grid);
 typedef struct pqc_tuning {
   int32_t plain_block;        /* threads per workgroup, plain per-op Kyber kernels: 64..1024, multiple of 64 */
   int32_t newhope_block;      /* same for the NewHope-1024 kernels */
-  int32_t fused_waves_per_cu; /* fused persistent grid = CUs x this: 1..4 (LDS holds 4) */
+  int32_t fused_waves_per_cu; /* fused persistent grid = CUs x this: 1..4 (LDS holds 4); staged kernels: this
+                                 many sponge waves per SIMD and half as many product workgroups per CU */
   int32_t mixed_order;        /* mixed-batch tile order: 0 = K 4,3,2; 1 = K 2,3,4; 2 = round-robin over K;
                                  3 = K 4,3,2 with 32-request tiles for K = 4 and K = 2 */
   int32_t frodo_stream_block; /* threads per workgroup of the Frodo noise-stream kernel: 64, 128 or 256 */
   int32_t lowlat_max;         /* Kyber batches of at most this many requests run one four-wave
-                                 workgroup per request (latency) instead of 64-request tiles
-                                 (throughput): 0 = library defaults (8192 decapsulations, 4096
-                                 encapsulations), -1 = never, else 1..65536 for both */
+                                 workgroup per request (latency) instead of the throughput forms
+                                 below: 0 = library defaults (1024 decapsulations of one parameter
+                                 set, 8192 mixed, 4096 encapsulations), -1 = never, else 1..65536
+                                 for all */
   int32_t frodo_chunk;        /* FrodoKEM-976 batches under one key above this many requests are cut
                                  into chunks of this many, run on four streams: 0 = library default
                                  (no split up to 65536), else a multiple of 32 in 32..65536 */
-  int32_t fused_dec_tile;     /* requests per tile of the fused Kyber decapsulation: 32 (two waves per
-                                 SIMD, A^T in a global scratch) or 64 (one wave per SIMD, A^T in an LDS
-                                 ring); 0 = library default (32) */
+  int32_t fused_dec_tile;     /* fused Kyber decapsulation: 64 = one persistent kernel over 64-request tiles
+                                 (one wave per SIMD, A^T in an LDS ring); 32 = the throughput form, whose
+                                 entries A^T go through a global scratch: sponge and matrix-core stages
+                                 (one parameter set) or 32-request tiles at two waves per SIMD (mixed
+                                 batches); 0 = library default (32) */
   int32_t fused_enc_tile;     /* the same for the fused Kyber encapsulation */
   int32_t fused_key_tile;     /* the same for the fused Kyber key generation */
   int32_t frodo_lane_min;     /* Keccak lane layout of the FrodoKEM-976 noise stream and F prefix in

@@ -81,6 +81,9 @@ struct pqc_ctx {
   int16_t* kat = nullptr;
   size_t kat_waves = 0;
   size_t kat_region = 0;  // int16 per wave region (sized for the largest K held)
+  // staged Kyber path: 128 bytes per request between the stages; requests per pass
+  uint8_t* krow = nullptr;
+  size_t kstage_max = 0;
   void* tuner = nullptr;  // autotuner samples and the learned cost model (tuner.cpp)
 };
 
@@ -110,6 +113,10 @@ int kyber_fused_enc(pqc_ctx* c, int k, size_t n, uint8_t* ct, uint8_t* ss, const
                     const uint8_t* coins, hipStream_t s);
 int kyber_fused_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct, const uint8_t* sk,
                     hipStream_t s);
+
+// the same in stages (kyber_staged.hip): throughput path of larger batches
+size_t kyber_stage_at_bytes(int k);  // sampled matrix entries of one request
+int kyber_staged_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct, const uint8_t* sk, hipStream_t s);
 
 // mixed Kyber-512/768/1024 batch through the fused kernels (kyber_fused.hip)
 int kyber_fused_mixed(pqc_ctx* c, int dec, size_t n, const pqc_kem_req* reqs, uint8_t* ct, size_t ct_bytes,

@@ -136,6 +136,46 @@ __device__ __forceinline__ void keccakf1600(uint64_t (&A64)[25]) {
   for (int i = 0; i < 25; ++i) A64[i] = (uint64_t)A[i].lo | ((uint64_t)A[i].hi << 32);
 }
 
+// The same permutation for kernels that keep several waves on a SIMD: two rounds per
+// trip, the next round constant loaded a round ahead.  Measured on MI355X, G state
+// permutations/s of the whole GPU at 1 / 2 / 4 waves per SIMD: 7.1 / 9.4 / 10.1, against
+// 6.7 / 9.0 / 9.8 for the loop above (a taken branch costs a lone wave ~200 cycles).
+__device__ __forceinline__ void keccakf1600_dense(uint64_t (&A64)[25]) {
+  Lane2 A[25];
+#pragma unroll
+  for (int i = 0; i < 25; ++i) A[i] = Lane2{(uint32_t)A64[i], (uint32_t)(A64[i] >> 32)};
+  uint64_t rc = c_keccak_rc[0];
+#pragma unroll 2
+  for (int round = 0; round < 24; ++round) {
+    const uint64_t rc_next = c_keccak_rc[round < 23 ? round + 1 : 0];
+    Lane2 C[5], Cm[5], Rp[5], B[25];
+#pragma unroll
+    for (int x = 0; x < 5; ++x) {
+      C[x].lo = xor3_32(xor3_32(A[x].lo, A[x + 5].lo, A[x + 10].lo), A[x + 15].lo, A[x + 20].lo);
+      C[x].hi = xor3_32(xor3_32(A[x].hi, A[x + 5].hi, A[x + 10].hi), A[x + 15].hi, A[x + 20].hi);
+    }
+#pragma unroll
+    for (int x = 0; x < 5; ++x) {
+      Cm[x] = C[(x + 4) % 5];
+      Rp[x] = rotl_2<1>(C[(x + 1) % 5]);
+    }
+    keccak_theta_rho_pi<0>(B, A, Cm, Rp);
+#pragma unroll
+    for (int y = 0; y < 5; ++y) {
+#pragma unroll
+      for (int x = 0; x < 5; ++x) {
+        const Lane2 a = B[x + 5 * y], b = B[(x + 1) % 5 + 5 * y], c = B[(x + 2) % 5 + 5 * y];
+        A[x + 5 * y] = Lane2{chi_32(a.lo, b.lo, c.lo), chi_32(a.hi, b.hi, c.hi)};
+      }
+    }
+    A[0].lo ^= (uint32_t)rc;
+    A[0].hi ^= (uint32_t)(rc >> 32);
+    rc = rc_next;
+  }
+#pragma unroll
+  for (int i = 0; i < 25; ++i) A64[i] = (uint64_t)A[i].lo | ((uint64_t)A[i].hi << 32);
+}
+
 // ---- split state: one sponge per pair of adjacent lanes ------------------------
 // The even lane holds the low 32-bit halves of the 25 state words, the odd lane
 // the high halves.  A 64-bit rotation needs the partner's half: one DPP

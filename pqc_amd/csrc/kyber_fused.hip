@@ -25,6 +25,7 @@
 
 #include "internal.h"
 #include "req_check.h"
+#include "kyber_src.cuh"
 #include "kyber_wave.cuh"
 #include "kyber_wavef.cuh"
 #include "sponge.cuh"
@@ -308,53 +309,6 @@ __device__ __forceinline__ int sample_entry(int16_t* dst, const uint64_t (&rho)[
   }
   return (int)(p - dst);
 }
-
-// Where the requests of a tile live.  DenseSrc: element-contiguous arrays of
-// one parameter set (element r at r * size).  MixedSrc: requests of mixed
-// parameter sets named by descriptors (pqc_kem_req: alg + byte offsets into
-// four arenas), bucketed by K into `order` by k_mixed_classify; index r of the
-// K bucket is request order[(K - 2) * cap + r].
-struct ReqP {
-  uint8_t* ss;
-  uint8_t* ct;
-  const uint8_t* key;
-  const uint8_t* coins;
-  uint8_t* prf;
-};
-
-struct DenseSrc {
-  uint8_t* ss;
-  uint8_t* ct;
-  const uint8_t* key;
-  const uint8_t* coins;
-  uint8_t* prf;
-  template <int K, bool DEC>
-  __device__ __forceinline__ ReqP req(int r) const {
-    using P = Params<K>;
-    return ReqP{ss + (size_t)r * 32, ct + (size_t)r * P::ct_bytes,
-                key + (size_t)r * (DEC ? P::sk_bytes : P::pk_bytes), coins ? coins + (size_t)r * 32 : nullptr,
-                prf + (size_t)r * Tile<K>::PRFB};
-  }
-};
-
-struct MixedSrc {
-  const pqc_kem_req* reqs;
-  const uint32_t* order;
-  int cap;
-  uint8_t* ss;
-  uint8_t* ct;
-  const uint8_t* key;
-  const uint8_t* coins;
-  uint8_t* prf;       // prf_stride bytes per request index
-  size_t prf_stride;  // >= Tile<K>::PRFB of every K the context holds
-  template <int K, bool DEC>
-  __device__ __forceinline__ ReqP req(int r) const {
-    const uint32_t idx = order[(size_t)(K - 2) * cap + r];
-    const pqc_kem_req d = reqs[idx];
-    return ReqP{ss + d.ss_off, ct + d.ct_off, key + d.key_off, coins ? coins + d.coins_off : nullptr,
-                prf + (size_t)idx * prf_stride};
-  }
-};
 
 // Request t of the tile, from the lane that holds it (t wave-uniform): no
 // descriptor reload for the cooperative phases.
@@ -946,16 +900,6 @@ __device__ __forceinline__ void enc_tile32(const Src& src, int base, int n, Lds3
     }
   }
   __syncthreads();
-}
-
-template <int K>
-__global__ __launch_bounds__(64, 2) void k_fused_dec32(int n, int ntiles, DenseSrc src, int16_t* at_scratch,
-                                                       uint32_t* __restrict__ status) {
-  __shared__ Lds32 sh;
-  LaneZF z;
-  load_lane_zf(z, &c_lane_twf);
-  global_t<int16_t>* at = (global_t<int16_t>*)(at_scratch + (size_t)blockIdx.x * Tile32<K>::ENTRIES * kAtStride);
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) dec_tile32<K>(src, tile * 32, n, sh, at, z, status);
 }
 
 template <int K>
@@ -1775,16 +1719,17 @@ static int launch_fused(pqc_ctx* c, size_t n, uint8_t* ss, uint8_t* ct, const ui
   return hip_err(hipGetLastError());
 }
 
-// Kyber batches (dense or mixed) of at most this many requests take the
-// one-workgroup-per-request kernels.  Measured on MI355X (Kyber-768): a tile
-// launch takes ~1.0 ms for any batch up to 65536; the per-request kernels run
-// ~10.6 M decaps/s and ~5.4 M encaps/s with ~0.12 / 0.2 ms latency, so they win
-// below ~10 K decapsulations and ~5 K encapsulations.  tuning.lowlat_max
-// overrides both (-1 = never).
-constexpr int kLowLatDefaultDec = 8192, kLowLatDefaultEnc = 4096;
+// Kyber batches of at most this many requests take the one-workgroup-per-request
+// kernels.  Dense decapsulation goes to the staged path above that (kyber_staged.hip):
+// measured on MI355X (Kyber-768), the per-request kernel takes 123 us at 761 requests,
+// 145 at 1024 and 219 at 2048, the stages 158 us at 761 and 163 at 2048.  For the other
+// operations a 32-request tile launch is the alternative, and the per-request kernels
+// win below ~10 K (mixed decapsulation) and ~5 K requests (encapsulation).
+// tuning.lowlat_max overrides them all (-1 = never).
+constexpr int kLowLatDenseDec = 1024, kLowLatDefaultDec = 8192, kLowLatDefaultEnc = 4096;
 
-inline bool use_lowlat(const pqc_ctx* c, size_t n, bool dec) {
-  const int lim = c->tune.lowlat_max != 0 ? c->tune.lowlat_max : dec ? kLowLatDefaultDec : kLowLatDefaultEnc;
+inline bool use_lowlat(const pqc_ctx* c, size_t n, int dflt) {
+  const int lim = c->tune.lowlat_max != 0 ? c->tune.lowlat_max : dflt;
   return n > 0 && (long long)n <= (long long)lim;
 }
 
@@ -1792,19 +1737,6 @@ template <int K, bool DEC>
 static int launch_lowlat(pqc_ctx* c, size_t n, uint8_t* ss, uint8_t* ct, const uint8_t* key, const uint8_t* coins,
                          hipStream_t s) {
   hipLaunchKernelGGL((k_lowlat<K, DEC>), dim3((unsigned)n), dim3(256), 0, s, (int)n, ss, ct, key, coins, c->status);
-  return hip_err(hipGetLastError());
-}
-
-template <int K>
-static int launch_dec32(pqc_ctx* c, size_t n, uint8_t* ss, uint8_t* ct, const uint8_t* sk, hipStream_t s) {
-  const int ntiles = (int)((n + Tile32<K>::T - 1) / Tile32<K>::T);
-  // two waves per SIMD at the default tuning (fused_waves_per_cu 4 -> 8 waves per CU)
-  int grid = c->fused_grid_override > 0 ? c->fused_grid_override : c->cu_count * 2 * c->tune.fused_waves_per_cu;
-  grid = std::min(grid, ntiles);
-  grid = std::min<long long>(grid, (long long)c->kat_waves);  // one scratch region per wave
-  if (grid < 1) return PQC_ERR_INVALID_ARG;
-  const DenseSrc src{ss, ct, sk, nullptr, c->kprf};
-  hipLaunchKernelGGL((k_fused_dec32<K>), dim3(grid), dim3(64), 0, s, (int)n, ntiles, src, c->kat, c->status);
   return hip_err(hipGetLastError());
 }
 
@@ -1864,15 +1796,9 @@ size_t tile32_scratch_bytes(int k) {
 
 int kyber_fused_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct, const uint8_t* sk, hipStream_t s) {
   uint8_t* ctm = const_cast<uint8_t*>(ct);  // read-only in the decaps instantiation
-  if (n > 0 && !kyber::fused::use_lowlat(c, n, true) && c->tune.fused_dec_tile != 64 && c->kat) {
-    switch (k) {
-      case 2: return kyber::fused::launch_dec32<2>(c, n, ss, ctm, sk, s);
-      case 3: return kyber::fused::launch_dec32<3>(c, n, ss, ctm, sk, s);
-      case 4: return kyber::fused::launch_dec32<4>(c, n, ss, ctm, sk, s);
-      default: return PQC_ERR_UNSUPPORTED;
-    }
-  }
-  if (kyber::fused::use_lowlat(c, n, true)) {
+  if (n > 0 && !kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDenseDec) && c->tune.fused_dec_tile != 64 && c->kat)
+    return kyber_staged_dec(c, k, n, ss, ct, sk, s);
+  if (kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDenseDec)) {
     switch (k) {
       case 2: return kyber::fused::launch_lowlat<2, true>(c, n, ss, ctm, sk, nullptr, s);
       case 3: return kyber::fused::launch_lowlat<3, true>(c, n, ss, ctm, sk, nullptr, s);
@@ -1890,7 +1816,7 @@ int kyber_fused_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct,
 
 int kyber_fused_enc(pqc_ctx* c, int k, size_t n, uint8_t* ct, uint8_t* ss, const uint8_t* pk, const uint8_t* coins,
                     hipStream_t s) {
-  if (n > 0 && !kyber::fused::use_lowlat(c, n, false) && c->tune.fused_enc_tile != 64 && c->kat) {
+  if (n > 0 && !kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDefaultEnc) && c->tune.fused_enc_tile != 64 && c->kat) {
     switch (k) {
       case 2: return kyber::fused::launch_enc32<2>(c, n, ss, ct, pk, coins, s);
       case 3: return kyber::fused::launch_enc32<3>(c, n, ss, ct, pk, coins, s);
@@ -1898,7 +1824,7 @@ int kyber_fused_enc(pqc_ctx* c, int k, size_t n, uint8_t* ct, uint8_t* ss, const
       default: return PQC_ERR_UNSUPPORTED;
     }
   }
-  if (kyber::fused::use_lowlat(c, n, false)) {
+  if (kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDefaultEnc)) {
     switch (k) {
       case 2: return kyber::fused::launch_lowlat<2, false>(c, n, ss, ct, pk, coins, s);
       case 3: return kyber::fused::launch_lowlat<3, false>(c, n, ss, ct, pk, coins, s);
@@ -1923,7 +1849,7 @@ int kyber_fused_mixed(pqc_ctx* c, int dec, size_t n, const pqc_kem_req* reqs, ui
   using namespace kyber::fused;
   if (n == 0) return PQC_OK;
   if (!c->kmix_order || !c->kprf) return PQC_ERR_UNSUPPORTED;
-  if (use_lowlat(c, n, dec != 0)) {  // one workgroup per descriptor, no bucketing
+  if (use_lowlat(c, n, dec ? kLowLatDefaultDec : kLowLatDefaultEnc)) {  // one workgroup per descriptor, no bucketing
     if (dec)
       hipLaunchKernelGGL(k_lowlat_mixed<true>, dim3((unsigned)n), dim3(256), 0, s, (int)n, c->alg_mask, reqs, ct,
                          (uint64_t)ct_bytes, key, (uint64_t)key_bytes, ss, (uint64_t)ss_bytes, coins,
@@ -1941,7 +1867,7 @@ int kyber_fused_mixed(pqc_ctx* c, int dec, size_t n, const pqc_kem_req* reqs, ui
                      c->alg_mask, reqs,
                      (uint64_t)ct_bytes, (uint64_t)key_bytes, (uint64_t)ss_bytes, (uint64_t)coins_bytes,
                      c->kmix_order, c->kmix_counts, c->status);
-  const MixedSrc src{reqs, c->kmix_order, cap, ss, ct, key, coins, c->kprf, c->kprf_per_elem};
+  const kyber::MixedSrc src{reqs, c->kmix_order, cap, ss, ct, key, coins, c->kprf, c->kprf_per_elem};
   const int max_tiles = (int)((n + 31) / 32) + 2;  // half tiles at most; buckets round up separately
   if (c->kat && (dec ? c->tune.fused_dec_tile : c->tune.fused_enc_tile) != 64) {
     // 32-request tiles, two waves per SIMD, one A^T scratch region per wave
@@ -2025,7 +1951,7 @@ int noalloc_dec(const NoAllocDev& d, size_t n, uint8_t* ss, uint8_t* ct, const u
   } else {
     const int ntiles = (int)((n + Tile<K>::T - 1) / Tile<K>::T);
     const int grid = std::max(1, std::min(ntiles, d.cus * 4));  // the default fused_waves_per_cu
-    const DenseSrc src{ss, ct, sk, nullptr, d.ptr + 256};
+    const kyber::DenseSrc src{ss, ct, sk, nullptr, d.ptr + 256};
     hipLaunchKernelGGL((k_fused<K, true>), dim3(grid), dim3(64), 0, s, (int)n, ntiles, src, status);
   }
   return hip_err(hipGetLastError());

@@ -1,0 +1,588 @@
+// Batched Kyber encapsulation, decapsulation and key generation in stages.
+//
+// A batch runs as a short chain of launches, each with the shape its work wants:
+//   sponge stages   one sponge chain per lane (H, G, PRF, KDF and the matrix entries
+//                   A_ij, K^2 lanes per request), about 100 VGPRs and little LDS, so
+//                   four waves share a SIMD and Keccak issues at its best rate;
+//   product stages  16 requests per wave: transforms on the matrix cores, the rest of
+//                   the polynomial arithmetic on FP32 values (kyber_mfma.cuh).
+// Between them: the noise bytes, the sampled entries and 96 bytes per request, in the
+// layouts the next stage reads (below).
+//
+//   decapsulation  k_open (indcpa_dec) -> k_sponge (H(ct); G, PRF; A^T)
+//                  -> k_reencrypt (indcpa_enc, verify, KDF)
+//   encapsulation  k_sponge (H(pk), m, G; A^T) -> k_prf -> k_reencrypt -> k_final
+//                  (H(ct), KDF)
+//   key generation k_key_seed (G) -> k_sponge (PRF; A) -> k_key_mul -> k_final (H(pk))
+//
+// Scratch, by group of 16 requests (request r of a bucket: group r / 16, slot r % 16;
+// dense batches have one bucket, mixed batches three whose groups follow each other):
+//   prf  [group][polynomial][chunk c][slot] 4 bytes: a wave's read of a chunk column is
+//        4 x 64 contiguous bytes, the writing lanes' stores too
+//   at   [group][entry][chunk c][slot] 16 bytes (8 coefficients)
+//   row  [group][slot] 128 bytes: m, Kbar, H(ct) or H(pk)
+//
+// The data flow and the reference functions are those of the 64-request tiles
+// (kyber_fused.hip); every path gives the same bytes.
+//
+// Measured on MI355X, us per call, this path and the 32-request tiles (two waves per
+// SIMD, butterfly transforms) or per-request workgroups it replaced:
+//   Kyber-768 decapsulation, 65536 requests    623    714
+//   Kyber-1024 decapsulation, 6000 requests    233    675 (a workgroup per request)
+// At 65536 the sponge stage takes ~370 us (53 permutations per request at 9.4 G/s, the
+// rate of the VALU on this mix), the product stages ~65 and ~140, the KDF ~15.
+#include <algorithm>
+
+#include "internal.h"
+#include "kyber_mfma.cuh"
+#include "kyber_src.cuh"
+#include "sponge.cuh"
+
+namespace pqc {
+namespace kyber {
+namespace staged {
+
+using namespace mfma;
+
+__device__ const DftTables c_dft = make_dft_tables();
+
+constexpr int kMaxBlocks = 32;  // SHAKE128 blocks per entry before giving up (never reached)
+
+struct Scratch {
+  uint8_t* prf;
+  size_t prf_group;  // bytes per group
+  uint8_t* at;
+  size_t at_group;  // bytes per group
+  uint8_t* row;
+  uint32_t* status;
+  // chunk column (poly, 4 t + g) of a wave's group: uniform base + 32-bit lane offset
+  __device__ __forceinline__ uint32_t prf_load(int grp, int poly, int t, uint32_t lane_off) const {
+    const uint8_t* p = prf + (size_t)grp * prf_group + (poly * 32 + 4 * t) * 64;
+    return *(const __attribute__((address_space(1))) uint32_t*)(p + lane_off);
+  }
+  __device__ __forceinline__ uint32_t* prf_word(int grp, int slot, int poly, int c) const {
+    return reinterpret_cast<uint32_t*>(prf + (size_t)grp * prf_group) + (poly * 32 + c) * 16 + slot;
+  }
+  __device__ __forceinline__ uint8_t* at_chunk(int grp, int slot, int entry, int c) const {
+    return at + (size_t)grp * at_group + ((size_t)(entry * 32 + c) * 16 + slot) * 16;
+  }
+  __device__ __forceinline__ uint8_t* row_of(int grp, int slot) const {
+    return row + ((size_t)grp * 16 + slot) * 128;
+  }
+};
+constexpr int kRowM = 0, kRowKbar = 32, kRowH = 64, kRowFail = 96;  // offsets inside a row
+
+// One bucket of a batch: n requests of one parameter set, its groups from grp0 on.
+struct Bucket {
+  int n, grp0;
+};
+
+// ---- sponge pieces ---------------------------------------------------------------
+
+__device__ __forceinline__ void load_words4(uint64_t (&w)[4], const uint8_t* p) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = load_u64_global(p + 8 * i);
+}
+
+__device__ __forceinline__ void store_words4(uint8_t* p, const uint64_t* w) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) store_u64(p + 8 * i, w[i]);
+}
+
+// PRF(seed, nonce): SHAKE256(seed || nonce), 128 bytes into the group's noise words
+__device__ __forceinline__ void prf_store(const Scratch& sc, int grp, int slot, const uint64_t (&seed)[4], int nonce) {
+  uint64_t A[25];
+  absorb_fixed<kRateShake256, 4, true>(A, seed, (uint64_t)nonce | (0x1Full << 8));
+  uint32_t* o = sc.prf_word(grp, slot, nonce, 0);
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    o[32 * w] = (uint32_t)A[w];
+    o[32 * w + 16] = (uint32_t)(A[w] >> 32);
+  }
+}
+
+// ---- matrix entries ----------------------------------------------------------------
+// Sampling stage: one LDS row of 40 coefficients per lane.  A third of a block (28
+// candidates) is written at the running position without a branch (an accepted
+// candidate advances it, a rejected one is overwritten by the next); then whole chunks
+// of 8 go to the entry with 16-byte stores and the 0..7 coefficients left move to the
+// front of the row.  5 KB of LDS per wave leaves room for four waves per SIMD.
+constexpr int kStageRow = 40;
+constexpr int kPartWords = 7;
+static_assert(kRateShake128 % kPartWords == 0 && 7 + 4 * kPartWords <= kStageRow && kStageRow % 8 == 0, "stage row");
+
+struct SponLds {
+  alignas(16) int16_t stage[64][kStageRow];
+};
+
+// SHAKE128(rho || x || y) rejection-sampled (gen_matrix_n, indcpa.cu:339-403) into the
+// entry's chunks; as in the tiles the accepted candidates themselves (< 19 q) are kept.
+__device__ __forceinline__ bool sample_entry(uint8_t* entry, int16_t* row, const uint64_t (&rho)[4], int x, int y,
+                                             bool valid) {
+  uint64_t A[25];
+#pragma unroll
+  for (int t = 0; t < 25; ++t) A[t] = (t < 4) ? rho[t] : 0;
+  A[4] = (uint64_t)x | ((uint64_t)y << 8) | (0x1Full << 16);
+  A[kRateShake128 - 1] ^= 0x8000000000000000ull;
+  int left = 0;   // coefficients in the row
+  int chunk = 0;  // chunks written
+  for (int blk = 0; blk < kMaxBlocks; ++blk) {
+    if (blk >= 4 && !__any(valid && chunk < 32)) break;
+    keccakf1600_dense(A);
+#pragma unroll
+    for (int part = 0; part < kRateShake128 / kPartWords; ++part) {
+      int16_t* p = row + left;
+#pragma unroll
+      for (int w = kPartWords * part; w < kPartWords * (part + 1); ++w) {
+        const uint32_t half[2] = {(uint32_t)A[w], (uint32_t)(A[w] >> 32)};
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const uint32_t val = (h & 1) ? (half[h >> 1] >> 16) : (half[h >> 1] & 0xFFFFu);
+          *p = (int16_t)val;
+          p += val < 19u * Q ? 1 : 0;
+        }
+      }
+      const int have = (int)(p - row);
+      const int whole = have >> 3;
+#pragma unroll
+      for (int c = 0; c < (7 + 4 * kPartWords) / 8; ++c)
+        if (c < whole && chunk + c < 32 && valid)
+          *(global_t<u4v>*)(entry + (size_t)(chunk + c) * 256) = *reinterpret_cast<const u4v*>(row + 8 * c);
+      const u4v rest = *reinterpret_cast<const u4v*>(row + 8 * whole);
+      *reinterpret_cast<u4v*>(row) = rest;
+      left = have & 7;
+      chunk += whole;
+    }
+  }
+  return chunk >= 32;
+}
+
+// Matrix work of a bucket: wave w of matrix_waves, 4 (group, entry) pairs of 16 lanes.
+// TRANS: entry (i, j) = XOF(rho, i, j) of A^T (encryption); else XOF(rho, j, i).
+template <int K>
+__host__ __device__ __forceinline__ int matrix_waves(int n) {
+  return ((n + 15) / 16 * K * K + 3) / 4;
+}
+
+template <int K, bool TRANS, class RhoOf>
+__device__ __forceinline__ void matrix_wave(const Scratch& sc, const Bucket& b, int w, SponLds& sh, RhoOf&& rho_of) {
+  const int lane = threadIdx.x & 63;
+  const int pair = 4 * w + (lane >> 4);
+  const int grp = pair / (K * K), e = pair % (K * K);
+  const int r = 16 * grp + (lane & 15);
+  const bool valid = r < b.n;
+  const int i = e / K, j = e % K;
+  uint64_t rho[4];
+  load_words4(rho, rho_of(valid ? r : b.n - 1));
+  const bool ok = sample_entry(sc.at_chunk(b.grp0 + grp, lane & 15, e, 0), sh.stage[lane], rho, TRANS ? i : j,
+                               TRANS ? j : i, valid);
+  if (valid && !ok) atomicOr(sc.status, 1u);
+}
+
+// ---- decapsulation: sponge stage -------------------------------------------------------
+// H(ct) of 64 requests
+template <int K, class Src>
+__device__ __forceinline__ void dec_hash_wave(const Src& src, const Scratch& sc, const Bucket& b, int w) {
+  using P = Params<K>;
+  const int r = 64 * w + (threadIdx.x & 63);
+  const bool act = r < b.n;
+  const ReqP q = src.template req<K, true>(act ? r : b.n - 1);
+  uint64_t A[25];
+  sponge_absorb_dense<kRateSha3_256>(A, q.ct, P::ct_bytes / 8, 0x06);
+  if (act) store_words4(sc.row_of(b.grp0 + r / 16, r % 16) + kRowH, A);
+}
+
+// (Kbar, coins) = G(m || H(pk)), then the 2K + 1 noise streams, of 64 requests
+template <int K, class Src>
+__device__ __forceinline__ void dec_prf_wave(const Src& src, const Scratch& sc, const Bucket& b, int w) {
+  using P = Params<K>;
+  const int r = 64 * w + (threadIdx.x & 63);
+  const bool act = r < b.n;
+  const int rc = act ? r : b.n - 1;
+  const ReqP q = src.template req<K, true>(rc);
+  uint8_t* row = sc.row_of(b.grp0 + rc / 16, rc % 16);
+  uint64_t m[8], A[25], seed[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    m[i] = load_u64_global(row + kRowM + 8 * i);
+    m[4 + i] = load_u64_global(q.key + P::hpk_off + 8 * i);
+  }
+  absorb_fixed<kRateSha3_512, 8, true>(A, m, 0x06);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) seed[i] = A[4 + i];
+  if (act) {
+    store_words4(row + kRowKbar, A);
+    for (int nonce = 0; nonce < 2 * K + 1; ++nonce)
+      prf_store(sc, b.grp0 + r / 16, r % 16, seed, nonce);
+  }
+}
+
+// ---- product stages ----------------------------------------------------------------------
+constexpr int kProdThreads = 256;  // 4 waves, 64 requests
+
+// This lane's request of a 64-request tile: wave's group and slot (a slot past the
+// batch's end repeats its last request and stores nothing)
+struct Lane {
+  int grp;  // wave-uniform
+  int n, g, r;
+  bool act;
+  __device__ __forceinline__ uint32_t prf_off() const { return 64u * g + 4u * n; }   // in a column of 4 chunks
+  __device__ __forceinline__ uint32_t at_off() const { return 256u * g + 16u * n; }  // the same, matrix entries
+};
+__device__ __forceinline__ Lane lane_of(const Bucket& b, int tile) {
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // computed per tile: nothing derived from it is worth registers across tiles
+  const int l = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  Lane x;
+  x.n = l & 15;
+  x.g = l >> 4;
+  const int r = 64 * tile + 16 * w + x.n;
+  x.act = r < b.n;
+  x.r = x.act ? r : b.n - 1;
+  x.grp = b.grp0 + 4 * tile + w;
+  return x;
+}
+
+// a[8] of a chunk from 12-bit values (0..4095), reduced
+__device__ __forceinline__ void chunk_from12(float (&a)[8], const Words<12>& x) {
+  uint32_t v[8];
+  unpack_chunk<12>(v, x, 0);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) a[k] = f32::reduce_f((float)v[k]);
+}
+// and from sampled entries (16-bit, < 19 q)
+__device__ __forceinline__ void chunk_from16(float (&a)[8], const u4v& x) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    a[2 * i] = f32::reduce_f((float)(x[i] & 0xFFFFu));
+    a[2 * i + 1] = f32::reduce_f((float)(x[i] >> 16));
+  }
+}
+
+// sum_j row_j o x_j, chunk by chunk: load(t) fetches chunk t's words of all j into a
+// LOADED (issued PRE chunks ahead), conv(a, loaded, j, t) gives reduced coefficients,
+// out(t, even, odd) takes the reduced sums.
+template <int K, class LOADED, class Load, class Conv, class Out>
+__device__ __forceinline__ void row_product(const HPoly (&x)[K], const float* gamma, const float* gammaq, int g,
+                                            Load&& load, Conv&& conv, Out&& out) {
+  constexpr int PRE = 2;
+  LOADED q[PRE + 1];
+#pragma unroll
+  for (int t = 0; t < PRE; ++t) load(q[t], t);
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    if (t + PRE < 8) load(q[(t + PRE) % (PRE + 1)], t + PRE);
+    ChunkSum s;
+    chunk_zero(s);
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      if (j > 0 && j % f32::kBasemulTerms == 0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s.s01[i] = f32::reduce_f(s.s01[i]);
+      }
+      float a[8];
+      conv(a, q[t % (PRE + 1)], j, t);
+      chunk_mac(s, a, x[j], t);
+    }
+    f4v e, o;
+    chunk_finish(s, gamma, gammaq, t, g, e, o);
+    out(t, e, o);
+    tile_fence();
+  }
+}
+
+template <int K>
+struct Loaded12 {
+  Words<12> w[K];
+};
+template <int K>
+struct Loaded16 {
+  u4v w[K];
+};
+
+// r^ (or s^): noise polynomial p of the request, transformed and reduced
+__device__ __forceinline__ void noise_ntt(HPoly& out, const Scratch& sc, const Lane& x, int p, const u4v* fwd) {
+  HPoly c;
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    uint32_t e[2], o[2];
+    cbd_chunk(e, o, sc.prf_load(x.grp, p, t, x.prf_off()));
+    c.v[0][t][0] = e[0];
+    c.v[0][t][1] = e[1];
+    c.v[1][t][0] = o[0];
+    c.v[1][t][1] = o[1];
+  }
+  dft1(fwd, c, [&](int mt, f4v e, f4v o) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      e[i] = f32::reduce_f(e[i]);
+      o[i] = f32::reduce_f(o[i]);
+    }
+    set_chunk(out, mt, e, o);
+  });
+}
+
+// indcpa_dec of a tile (indcpa.cu:691-733): m' into the rows
+template <int K, class Src>
+__device__ __forceinline__ void open_tile(const Src& src, const Scratch& sc, const Bucket& b, int tile,
+                                          const DftLds<true, true>& sh) {
+  using P = Params<K>;
+  const Lane x = lane_of(b, tile);
+  const ReqP q = src.template req<K, true>(x.r);
+  const ChunkAt<P::du> au(x.g);
+  const ChunkAt<P::dv> av(x.g);
+  const ChunkAt<12> as(x.g);
+  HPoly u[K];
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    Words<P::du> w[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) load_chunk<P::du>(w[t], q.ct + 32 * P::du * j, au, t);
+    HPoly uh, ul;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      uint32_t v[8];
+      unpack_chunk<P::du>(v, w[t], au.sh);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = (uint32_t)decompress_d<P::du>(v[k]);  // [0, q)
+      // digits v >> 6, v & 63 of two values as the f16 pairs 1024 + digit
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          const uint32_t pr = v[4 * p + h] | (v[4 * p + 2 + h] << 16);
+          uh.v[h][t][p] = add_h2(((pr >> 6) & 0x003F003Fu) | 0x64006400u, -1024.f);
+          ul.v[h][t][p] = add_h2((pr & 0x003F003Fu) | 0x64006400u, -1024.f);
+        }
+    }
+    dft2(sh.fwd, uh, ul, [](int) {}, [&](int mt, const f4v& e, const f4v& o) { set_chunk(u[j], mt, e, o); });
+  }
+  HPoly ph, pl;
+  row_product<K, Loaded12<K>>(
+      u, sh.gamma, sh.gammaq, x.g,
+      [&](Loaded12<K>& l, int t) {
+#pragma unroll
+        for (int j = 0; j < K; ++j) load_chunk<12>(l.w[j], q.key + 384 * j, as, t);
+      },
+      [&](float (&a)[8], const Loaded12<K>& l, int j, int) { chunk_from12(a, l.w[j]); },
+      [&](int t, const f4v& e, const f4v& o) { set_digits(ph, pl, t, e, o); });
+  Words<P::dv> vw[3];
+  uint8_t* m = sc.row_of(x.grp, x.n) + kRowM;
+  auto pre = [&](int t) { load_chunk<P::dv>(vw[t % 3], q.ct + P::polyvec_cbytes, av, t); };
+  dft2(sh.inv, ph, pl, pre, [&](int mt, const f4v& e, const f4v& o) {
+    uint32_t v[8];
+    unpack_chunk<P::dv>(v, vw[mt % 3], av.sh);
+    uint32_t bits = 0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      bits |= f32::compress_f<1>((float)decompress_d<P::dv>(v[k]) - ((k & 1) ? o[k >> 1] : e[k >> 1])) << k;
+    if (x.act) m[4 * mt + x.g] = (uint8_t)bits;
+  });
+}
+
+// One output polynomial of indcpa_enc: inverse transform, + noise (+ message bits),
+// compressed to D bits; compared with the ciphertext (DEC) or stored.
+template <int D, bool DEC, bool MSG>
+__device__ __forceinline__ uint32_t finish_poly(const u4v* inv, const HPoly& ph, const HPoly& pl, const Scratch& sc,
+                                                int noise, const uint8_t* msg, uint8_t* ct, const Lane& x) {
+  int g = x.g;
+  asm volatile("" : "+v"(g));  // offsets per polynomial, not kept across the row products
+  const ChunkAt<D> ac(g);
+  Words<D> cw[DEC ? 3 : 1];
+  uint32_t pw[3], mw[3];
+  auto pre = [&](int t) {
+    pw[t % 3] = sc.prf_load(x.grp, noise, t, x.prf_off());
+    if constexpr (DEC) load_chunk<D>(cw[t % 3], ct, ac, t);
+    if constexpr (MSG) mw[t % 3] = (uint32_t)*(const global_t<uint8_t>*)(msg + 4 * t + x.g);
+  };
+  uint32_t bad = 0;
+  dft2(inv, ph, pl, pre, [&](int mt, const f4v& e, const f4v& o) {
+    uint32_t ne[2], no[2], v[8];
+    cbd_chunk(ne, no, pw[mt % 3]);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int i = k >> 1;
+      float c = ((k & 1) ? o[i] : e[i]) + h2_get((k & 1) ? no[i >> 1] : ne[i >> 1], i & 1);
+      if constexpr (MSG) c += ((mw[mt % 3] >> k) & 1) ? (float)((Q + 1) / 2) : 0.f;
+      v[k] = f32::compress_f<D>(c);
+    }
+    if constexpr (DEC) {
+      uint32_t t[8];
+      unpack_chunk<D>(t, cw[mt % 3], ac.sh);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) bad |= v[k] ^ t[k];
+      asm volatile("" : "+v"(bad));  // this tile's compare ends here (else the values wait for the last tile)
+    } else {
+      if (x.act) store_chunk<D>(ct, x.g, mt, v);
+    }
+  });
+  return bad;
+}
+
+// indcpa_enc of a tile (indcpa.cu:578-679).  DEC: compare, fail flags of the tile's 64
+// requests into LDS.  Otherwise write the ciphertexts.
+template <int K, bool DEC, class Src>
+__device__ __forceinline__ void reencrypt_tile(const Src& src, const Scratch& sc, const Bucket& b, int tile,
+                                               const DftLds<true, true>& sh) {
+  using P = Params<K>;
+  constexpr int PK_OFF = DEC ? P::sk_cpa_bytes : 0;  // public key inside the key buffer
+  const Lane x = lane_of(b, tile);
+  const ReqP q = src.template req<K, DEC>(x.r);
+  HPoly r[K];
+#pragma unroll
+  for (int j = 0; j < K; ++j) noise_ntt(r[j], sc, x, j, sh.fwd);
+  uint32_t bad = 0;
+#pragma unroll 1
+  for (int i = 0; i < K; ++i) {
+#pragma unroll
+    for (int j = 0; j < K; ++j) keep_packed(r[j]);
+    HPoly ph, pl;
+    const uint8_t* at = sc.at_chunk(x.grp, 0, i * K, 0);
+    row_product<K, Loaded16<K>>(
+        r, sh.gamma, sh.gammaq, x.g,
+        [&](Loaded16<K>& l, int t) {
+#pragma unroll
+          for (int j = 0; j < K; ++j) l.w[j] = *(const global_t<u4v>*)(at + (j * 32 + 4 * t) * 256 + x.at_off());
+        },
+        [&](float (&a)[8], const Loaded16<K>& l, int j, int) { chunk_from16(a, l.w[j]); },
+        [&](int t, const f4v& e, const f4v& o) { set_digits(ph, pl, t, e, o); });
+    bad |= finish_poly<P::du, DEC, false>(sh.inv, ph, pl, sc, K + i, nullptr, q.ct + 32 * P::du * i, x);
+  }
+  {
+    const ChunkAt<12> at12(x.g);
+    HPoly ph, pl;
+    row_product<K, Loaded12<K>>(
+        r, sh.gamma, sh.gammaq, x.g,
+        [&](Loaded12<K>& l, int t) {
+#pragma unroll
+          for (int j = 0; j < K; ++j) load_chunk<12>(l.w[j], q.key + PK_OFF + 384 * j, at12, t);
+        },
+        [&](float (&a)[8], const Loaded12<K>& l, int j, int) { chunk_from12(a, l.w[j]); },
+        [&](int t, const f4v& e, const f4v& o) { set_digits(ph, pl, t, e, o); });
+    bad |= finish_poly<P::dv, DEC, true>(sh.inv, ph, pl, sc, 2 * K, sc.row_of(x.grp, x.n) + kRowM,
+                                         q.ct + P::polyvec_cbytes, x);
+  }
+  if constexpr (DEC) {
+    bad |= (uint32_t)__shfl_xor((int)bad, 16);
+    bad |= (uint32_t)__shfl_xor((int)bad, 32);
+    if (x.g == 0 && x.act) *reinterpret_cast<uint32_t*>(sc.row_of(x.grp, x.n) + kRowFail) = bad;
+  }
+}
+
+// ss = KDF(Kbar or z, H(ct)) of 64 requests, one lane each
+template <int K, class Src>
+__device__ __forceinline__ void dec_kdf_wave(const Src& src, const Scratch& sc, const Bucket& b, int w) {
+  using P = Params<K>;
+  const int r = 64 * w + (threadIdx.x & 63);
+  if (r >= b.n) return;
+  const ReqP q = src.template req<K, true>(r);
+  const uint8_t* row = sc.row_of(b.grp0 + r / 16, r % 16);
+  const uint32_t f = *reinterpret_cast<const uint32_t*>(row + kRowFail);
+  const uint64_t mask = 0 - (uint64_t)((f | (0u - f)) >> 31);
+  uint64_t m[8], A[25];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint64_t kb = load_u64_global(row + kRowKbar + 8 * i), zz = load_u64_global(q.key + P::z_off + 8 * i);
+    m[i] = kb ^ (mask & (zz ^ kb));
+    m[4 + i] = load_u64_global(row + kRowH + 8 * i);
+  }
+  absorb_fixed<kRateShake256, 8, true>(A, m, 0x1F);
+  store_words4(q.ss, A);
+}
+
+// ---- dense kernels ---------------------------------------------------------------------------
+template <int K>
+__global__ __launch_bounds__(kProdThreads, 2) void k_open(int n, DenseSrc src, Scratch sc) {
+  __shared__ DftLds<true, true> sh;
+  load_tables<true, true, kProdThreads>(sh, &c_dft);
+  const Bucket b{n, 0};
+  for (int tile = blockIdx.x; tile < (n + 63) / 64; tile += gridDim.x) open_tile<K>(src, sc, b, tile, sh);
+}
+
+// waves: H(ct), then G and PRF (the longest chains first), then the matrix entries
+template <int K>
+__global__ __launch_bounds__(64, 4) void k_dec_sponge(int n, DenseSrc src, Scratch sc) {
+  using P = Params<K>;
+  __shared__ SponLds sh;
+  const Bucket b{n, 0};
+  const int wr = (n + 63) / 64, total = 2 * wr + matrix_waves<K>(n);
+  for (int w = blockIdx.x; w < total; w += gridDim.x) {
+    if (w < wr)
+      dec_hash_wave<K>(src, sc, b, w);
+    else if (w < 2 * wr)
+      dec_prf_wave<K>(src, sc, b, w - wr);
+    else
+      matrix_wave<K, true>(sc, b, w - 2 * wr, sh, [&](int r) {
+        return src.template req<K, true>(r).key + P::sk_cpa_bytes + P::polyvec_bytes;
+      });
+  }
+}
+
+template <int K>
+__global__ __launch_bounds__(kProdThreads, 2) void k_dec_reencrypt(int n, DenseSrc src, Scratch sc) {
+  __shared__ DftLds<true, true> sh;
+  load_tables<true, true, kProdThreads>(sh, &c_dft);
+  const Bucket b{n, 0};
+  for (int tile = blockIdx.x; tile < (n + 63) / 64; tile += gridDim.x) reencrypt_tile<K, true>(src, sc, b, tile, sh);
+}
+
+template <int K>
+__global__ __launch_bounds__(64) void k_dec_kdf(int n, DenseSrc src, Scratch sc) {
+  for (int w = blockIdx.x; w < (n + 63) / 64; w += gridDim.x) dec_kdf_wave<K>(src, sc, Bucket{n, 0}, w);
+}
+
+// ---- launchers ---------------------------------------------------------------------------------
+static Scratch scratch_of(const pqc_ctx* c, int k) {
+  return Scratch{c->kprf, (size_t)(2 * k + 1) * 2048, reinterpret_cast<uint8_t*>(c->kat), (size_t)k * k * 16 * 512, c->krow, c->status};
+}
+
+// Product stages: persistent, two workgroups per CU (66 KB of tables each) at the default
+// fused_waves_per_cu of 4.  Sponge stages: one workgroup per wave of work, handed out by
+// the hardware in the order of their number; below 4, as many as fit that many per SIMD.
+static int prod_grid(const pqc_ctx* c, int tiles) {
+  const int g = c->fused_grid_override > 0 ? c->fused_grid_override : c->cu_count * c->tune.fused_waves_per_cu / 2;
+  return std::max(1, std::min(g, tiles));
+}
+static int sponge_grid(const pqc_ctx* c, int waves) {
+  int g = waves;
+  if (c->fused_grid_override > 0)
+    g = c->fused_grid_override;
+  else if (c->tune.fused_waves_per_cu < 4)
+    g = c->cu_count * 4 * c->tune.fused_waves_per_cu;
+  return std::max(1, std::min(g, waves));
+}
+
+template <int K>
+static int dec(pqc_ctx* c, size_t n_all, uint8_t* ss, uint8_t* ct, const uint8_t* sk, hipStream_t s) {
+  using P = Params<K>;
+  const Scratch sc = scratch_of(c, K);
+  for (size_t at = 0; at < n_all; at += c->kstage_max) {
+    const int n = (int)std::min(n_all - at, c->kstage_max);
+    const int tiles = (n + 63) / 64, waves = 2 * tiles + matrix_waves<K>(n);
+    const DenseSrc src{ss + at * 32, ct + at * P::ct_bytes, sk + at * P::sk_bytes, nullptr, c->kprf};
+    hipLaunchKernelGGL((k_open<K>), dim3(prod_grid(c, tiles)), dim3(kProdThreads), 0, s, n, src, sc);
+    hipLaunchKernelGGL((k_dec_sponge<K>), dim3(sponge_grid(c, waves)), dim3(64), 0, s, n, src, sc);
+    hipLaunchKernelGGL((k_dec_reencrypt<K>), dim3(prod_grid(c, tiles)), dim3(kProdThreads), 0, s, n, src, sc);
+    hipLaunchKernelGGL((k_dec_kdf<K>), dim3(sponge_grid(c, tiles)), dim3(64), 0, s, n, src, sc);
+    const int rc = hip_err(hipGetLastError());
+    if (rc) return rc;
+  }
+  return PQC_OK;
+}
+
+}  // namespace staged
+}  // namespace kyber
+
+size_t kyber_stage_at_bytes(int k) { return (size_t)k * k * 512; }
+
+int kyber_staged_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct, const uint8_t* sk, hipStream_t s) {
+  uint8_t* ctm = const_cast<uint8_t*>(ct);
+  switch (k) {
+    case 2: return kyber::staged::dec<2>(c, n, ss, ctm, sk, s);
+    case 3: return kyber::staged::dec<3>(c, n, ss, ctm, sk, s);
+    case 4: return kyber::staged::dec<4>(c, n, ss, ctm, sk, s);
+    default: return PQC_ERR_UNSUPPORTED;
+  }
+}
+
+}  // namespace pqc

@@ -1,0 +1,54 @@
+"""Staged Kyber kernels (sponge stages, matrix-core product stages) at the edges of
+their groups of 16, tiles of 64 and persistent grids, bit-exact against the CPU oracle."""
+import sys
+
+import numpy as np
+import pytest
+
+from tests import oracle_lib as O
+
+pytestmark = pytest.mark.gpu
+
+ALG = {2: "kyber512", 3: "kyber768", 4: "kyber1024"}
+SIZES = [1, 15, 16, 17, 63, 64, 65, 193]
+
+
+@pytest.fixture(scope="module")
+def pqc():
+    import pqc_amd
+    return pqc_amd
+
+
+def staged_ctx(pqc, k, n, grid):
+    from pqc_amd import tuner as T
+    ctx = pqc.Context([ALG[k]], max_batch=n)
+    T.put_tuning(ctx, lowlat_max=-1)  # no batch is too small for the stages
+    ctx.set_tuning(grid=grid)
+    return ctx
+
+
+def inputs(k, n, seed):
+    """Valid key pairs and ciphertexts, a third of the ciphertexts damaged, and every
+    fourth secret key and ciphertext of arbitrary bytes (12-bit values up to 4095)."""
+    rng = np.random.default_rng(seed)
+    pk, sk = O.kyber_batch("keypair", k, [rng.integers(0, 256, (n, 64), dtype=np.uint8)])
+    ct, _ = O.kyber_batch("enc", k, [pk, rng.integers(0, 256, (n, 32), dtype=np.uint8)])
+    ct[::3, rng.integers(0, ct.shape[1])] ^= 1 << int(rng.integers(0, 8))
+    sk[3::4] = rng.integers(0, 256, sk[3::4].shape, dtype=np.uint8)
+    ct[3::8] = rng.integers(0, 256, ct[3::8].shape, dtype=np.uint8)
+    pk[3::4] = rng.integers(0, 256, pk[3::4].shape, dtype=np.uint8)
+    return pk, sk, ct
+
+
+@pytest.mark.parametrize("grid", [0, 1])
+@pytest.mark.parametrize("k", [2, 3, 4])
+def test_staged_decaps_vs_oracle(pqc, k, grid):
+    ctx = staged_ctx(pqc, k, max(SIZES), grid)
+    for n in SIZES:
+        print("staged decaps k", k, "n", n, "grid", grid, flush=True)
+        sys.stdout.flush()
+        _, sk, ct = inputs(k, n, 1000 * k + n)
+        want = O.kyber_batch("dec", k, [ct, sk])
+        got = ctx.dec_host(ALG[k], ct, sk)
+        assert (got == want).all(), np.nonzero((got != want).any(axis=1))[0][:8]
+    ctx.close()
