@@ -82,8 +82,8 @@ typedef struct pqc_tuning {
   int32_t frodo_stream_block; /* threads per workgroup of the Frodo noise-stream kernel: 64, 128 or 256 */
   int32_t lowlat_max;         /* Kyber batches of at most this many requests run one four-wave
                                  workgroup per request (latency) instead of the throughput forms
-                                 below: 0 = library defaults (1024 decapsulations of one parameter
-                                 set, 8192 mixed, 4096 encapsulations), -1 = never, else 1..65536
+                                 below: 0 = library defaults (1024 decapsulations and 256
+                                 encapsulations of one parameter set, 8192 and 4096 mixed), -1 = never, else 1..65536
                                  for all */
   int32_t frodo_chunk;        /* FrodoKEM-976 batches under one key above this many requests are cut
                                  into chunks of this many, run on four streams: 0 = library default

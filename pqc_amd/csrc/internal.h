@@ -116,6 +116,9 @@ int kyber_fused_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct,
 
 // the same in stages (kyber_staged.hip): throughput path of larger batches
 size_t kyber_stage_at_bytes(int k);  // sampled matrix entries of one request
+int kyber_staged_keypair(pqc_ctx* c, int k, size_t n, uint8_t* pk, uint8_t* sk, const uint8_t* coins, hipStream_t s);
+int kyber_staged_enc(pqc_ctx* c, int k, size_t n, uint8_t* ct, uint8_t* ss, const uint8_t* pk, const uint8_t* coins,
+                     hipStream_t s);
 int kyber_staged_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct, const uint8_t* sk, hipStream_t s);
 
 // mixed Kyber-512/768/1024 batch through the fused kernels (kyber_fused.hip)

@@ -902,16 +902,6 @@ __device__ __forceinline__ void enc_tile32(const Src& src, int base, int n, Lds3
   __syncthreads();
 }
 
-template <int K>
-__global__ __launch_bounds__(64, 2) void k_fused_enc32(int n, int ntiles, DenseSrc src, int16_t* at_scratch,
-                                                       uint32_t* __restrict__ status) {
-  __shared__ Lds32 sh;
-  LaneZF z;
-  load_lane_zf(z, &c_lane_twf);
-  global_t<int16_t>* at = (global_t<int16_t>*)(at_scratch + (size_t)blockIdx.x * Tile32<K>::ENTRIES * kAtStride);
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) enc_tile32<K>(src, tile * 32, n, sh, at, z, status);
-}
-
 // Mixed batches: the bucketed requests (k_mixed_classify) in 32-request tiles at
 // two waves per SIMD, K = 4 tiles first (the longest), then K = 3, then K = 2;
 // each wave's A^T scratch region holds `region` int16 (sized for the largest K
@@ -1114,112 +1104,6 @@ __device__ __forceinline__ void fused_keypair_tile(const KeySrc& src, int base, 
     }
   }
   __syncthreads();
-}
-
-// Key generation in the 32-request tiles of decapsulation and encapsulation
-// (two waves per SIMD, A through the per-wave global scratch): both lanes of a
-// pair compute G(d) and split the 2K PRF outputs (lane l the even nonces, lane
-// l + 32 the odd ones); the rounds of A entries, each followed by the key
-// computation of the requests it completes; H(pk) on lanes 0..31.  Same bytes
-// as fused_keypair_tile.
-template <int K>
-__device__ __forceinline__ void keypair_tile32(const KeySrc& src, int base, int n, Lds32& sh, global_t<int16_t>* at,
-                                               const LaneZF& z, uint32_t* __restrict__ status) {
-  using P = Params<K>;
-  using TL = Tile32<K>;
-  constexpr size_t PRFB = Tile<K>::PRFB;
-  const int lane = threadIdx.x;
-  const int rq = lane & 31;  // the request this lane serves in the sponge phases (lanes l and l + 32 alike)
-  const int nt = min(TL::T, n - base);
-  const bool act = rq < nt;
-  const bool hl = lane < 32;
-  const int rc = act ? base + rq : base;  // clamped request for address math
-  uint8_t* pk = src.pk + (size_t)rc * P::pk_bytes;
-  uint8_t* sk = src.sk + (size_t)rc * P::sk_bytes;
-  uint8_t* prf = src.prf + (size_t)rc * PRFB;
-  const uint8_t* coins = src.coins + (size_t)rc * 64;
-  // ---- (rho, sigma) = G(d) on both lanes of a pair; PRF(sigma, 2 i + (lane >= 32)),
-  // i = 0 .. K - 1 -> scratch; rho -> LDS and both pk copies
-  {
-    uint64_t d[4], A[25], sg[4];
-#pragma unroll
-    for (int w = 0; w < 4; ++w) d[w] = load_u64_global(coins + 8 * w);
-    absorb_fixed<kRateSha3_512, 4>(A, d, 0x06);
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      sg[w] = A[4 + w];
-      if (hl) store_u64(sh.msg[rq] + 8 * w, A[w]);
-      if (hl && act) {
-        store_u64(pk + P::polyvec_bytes + 8 * w, A[w]);
-        store_u64(sk + P::sk_cpa_bytes + P::polyvec_bytes + 8 * w, A[w]);
-      }
-    }
-    for (int i = 0; i < K; ++i) {
-      const int nonce = 2 * i + (hl ? 0 : 1);
-      absorb_fixed<kRateShake256, 4>(A, sg, (uint64_t)nonce | (0x1Full << 8));
-      if (act) {
-#pragma unroll
-        for (int w = 0; w < 16; ++w) store_u64(prf + 128 * nonce + 8 * w, A[w]);
-      }
-    }
-  }
-  __syncthreads();
-  // ---- rounds of 64 A entries into the scratch (entry E: request E / K^2, A[i][j]
-  // at position i K + j), then t and s of every request the round completes
-  const int ng = (nt * TL::KK + 63) / 64;
-  int t_done = 0;
-  for (int g = 0; g < ng; ++g) {
-    {
-      const int E = 64 * g + lane;
-      const int t = E / TL::KK;
-      const int ij = E % TL::KK;
-      const bool valid = t < nt;
-      uint64_t rho[4];
-#pragma unroll
-      for (int w = 0; w < 4; ++w) rho[w] = load_u64(sh.msg[valid ? t : 0] + 8 * w);
-      const int got = sample_entry_staged(at + (size_t)E * kAtStride, sh.stage[lane], rho, ij % K, ij / K, valid);
-      if (valid && got < N) atomicOr(status, 1u);
-    }
-    __syncthreads();  // the round's entries are in the scratch for every lane
-    const int t_end = min(nt, (64 * (g + 1)) / TL::KK);
-    if (t_done < t_end) {
-      KeyIn<K> cur, nxt;
-      key_load<K>(nxt, src.prf + (size_t)(base + t_done) * PRFB);
-      for (int t = t_done; t < t_end; ++t) {
-        cur = nxt;
-        if (t + 1 < t_end) key_load<K>(nxt, src.prf + (size_t)(base + t + 1) * PRFB);
-        AtRegs<K> a;
-        a.load(at, t);
-        coop_keypair<K>(a, cur, src.pk + (size_t)(base + t) * P::pk_bytes, src.sk + (size_t)(base + t) * P::sk_bytes,
-                        z);
-      }
-      t_done = t_end;
-    }
-  }
-  __syncthreads();
-  // ---- H(pk) over the packed key (written by the whole wave), z; lanes 0..31 store
-  {
-    uint64_t A[25];
-    sponge_absorb_words_prefetch<kRateSha3_256>(A, reinterpret_cast<const uint64_t*>(pk), P::pk_bytes / 8, 0x06);
-    if (hl && act) {
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        store_u64(sk + P::hpk_off + 8 * w, A[w]);
-        store_u64(sk + P::z_off + 8 * w, load_u64_global(coins + 32 + 8 * w));
-      }
-    }
-  }
-  __syncthreads();
-}
-
-template <int K>
-__global__ __launch_bounds__(64, 2) void k_fused_keypair32(int n, int ntiles, KeySrc src, int16_t* at_scratch,
-                                                           uint32_t* __restrict__ status) {
-  __shared__ Lds32 sh;
-  LaneZF z;
-  load_lane_zf(z, &c_lane_twf);
-  global_t<int16_t>* at = (global_t<int16_t>*)(at_scratch + (size_t)blockIdx.x * Tile32<K>::ENTRIES * kAtStride);
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) keypair_tile32<K>(src, tile * 32, n, sh, at, z, status);
 }
 
 template <int K>
@@ -1720,13 +1604,14 @@ static int launch_fused(pqc_ctx* c, size_t n, uint8_t* ss, uint8_t* ct, const ui
 }
 
 // Kyber batches of at most this many requests take the one-workgroup-per-request
-// kernels.  Dense decapsulation goes to the staged path above that (kyber_staged.hip):
-// measured on MI355X (Kyber-768), the per-request kernel takes 123 us at 761 requests,
-// 145 at 1024 and 219 at 2048, the stages 158 us at 761 and 163 at 2048.  For the other
-// operations a 32-request tile launch is the alternative, and the per-request kernels
-// win below ~10 K (mixed decapsulation) and ~5 K requests (encapsulation).
-// tuning.lowlat_max overrides them all (-1 = never).
-constexpr int kLowLatDenseDec = 1024, kLowLatDefaultDec = 8192, kLowLatDefaultEnc = 4096;
+// kernels.  Batches of one parameter set go to the staged path above that
+// (kyber_staged.hip): measured on MI355X (Kyber-768), the per-request kernels take 123 us
+// for 761 decapsulations, 145 for 1024, 219 for 2048 and 257 us for 300 encapsulations,
+// the stages 158 us at 761, 163 at 2048 and 239 us at 300.  For mixed batches a 32-request
+// tile launch is the alternative, and the per-request kernels win below ~10 K
+// decapsulations and ~5 K encapsulations.  tuning.lowlat_max overrides them all
+// (-1 = never).
+constexpr int kLowLatDenseDec = 1024, kLowLatDenseEnc = 256, kLowLatDefaultDec = 8192, kLowLatDefaultEnc = 4096;
 
 inline bool use_lowlat(const pqc_ctx* c, size_t n, int dflt) {
   const int lim = c->tune.lowlat_max != 0 ? c->tune.lowlat_max : dflt;
@@ -1741,32 +1626,8 @@ static int launch_lowlat(pqc_ctx* c, size_t n, uint8_t* ss, uint8_t* ct, const u
 }
 
 template <int K>
-static int launch_enc32(pqc_ctx* c, size_t n, uint8_t* ss, uint8_t* ct, const uint8_t* pk, const uint8_t* coins,
-                        hipStream_t s) {
-  const int ntiles = (int)((n + Tile32<K>::T - 1) / Tile32<K>::T);
-  int grid = c->fused_grid_override > 0 ? c->fused_grid_override : c->cu_count * 2 * c->tune.fused_waves_per_cu;
-  grid = std::min(grid, ntiles);
-  grid = std::min<long long>(grid, (long long)c->kat_waves);  // one scratch region per wave
-  if (grid < 1) return PQC_ERR_INVALID_ARG;
-  const DenseSrc src{ss, ct, pk, coins, c->kprf};
-  hipLaunchKernelGGL((k_fused_enc32<K>), dim3(grid), dim3(64), 0, s, (int)n, ntiles, src, c->kat, c->status);
-  return hip_err(hipGetLastError());
-}
-
-template <int K>
 static int launch_fused_keypair(pqc_ctx* c, size_t n, uint8_t* pk, uint8_t* sk, const uint8_t* coins, hipStream_t s) {
   if (n == 0) return PQC_OK;
-  if (c->tune.fused_key_tile != 64 && c->kat) {
-    // 32-request tiles, two waves per SIMD, one scratch region per wave
-    const int ntiles = (int)((n + Tile32<K>::T - 1) / Tile32<K>::T);
-    int grid = c->fused_grid_override > 0 ? c->fused_grid_override : c->cu_count * 2 * c->tune.fused_waves_per_cu;
-    grid = std::min(grid, ntiles);
-    grid = std::min<long long>(grid, (long long)c->kat_waves);
-    if (grid < 1) return PQC_ERR_INVALID_ARG;
-    const KeySrc src{pk, sk, coins, c->kprf};
-    hipLaunchKernelGGL((k_fused_keypair32<K>), dim3(grid), dim3(64), 0, s, (int)n, ntiles, src, c->kat, c->status);
-    return hip_err(hipGetLastError());
-  }
   const int ntiles = (int)((n + Tile<K>::T - 1) / Tile<K>::T);
   int grid = c->fused_grid_override > 0 ? c->fused_grid_override : c->cu_count * c->tune.fused_waves_per_cu;
   if (grid > ntiles) grid = ntiles;
@@ -1780,6 +1641,7 @@ static int launch_fused_keypair(pqc_ctx* c, size_t n, uint8_t* pk, uint8_t* sk, 
 }  // namespace kyber
 
 int kyber_fused_keypair(pqc_ctx* c, int k, size_t n, uint8_t* pk, uint8_t* sk, const uint8_t* coins, hipStream_t s) {
+  if (n > 0 && c->tune.fused_key_tile != 64 && c->kat) return kyber_staged_keypair(c, k, n, pk, sk, coins, s);
   switch (k) {
     case 2: return kyber::fused::launch_fused_keypair<2>(c, n, pk, sk, coins, s);
     case 3: return kyber::fused::launch_fused_keypair<3>(c, n, pk, sk, coins, s);
@@ -1816,15 +1678,9 @@ int kyber_fused_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct,
 
 int kyber_fused_enc(pqc_ctx* c, int k, size_t n, uint8_t* ct, uint8_t* ss, const uint8_t* pk, const uint8_t* coins,
                     hipStream_t s) {
-  if (n > 0 && !kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDefaultEnc) && c->tune.fused_enc_tile != 64 && c->kat) {
-    switch (k) {
-      case 2: return kyber::fused::launch_enc32<2>(c, n, ss, ct, pk, coins, s);
-      case 3: return kyber::fused::launch_enc32<3>(c, n, ss, ct, pk, coins, s);
-      case 4: return kyber::fused::launch_enc32<4>(c, n, ss, ct, pk, coins, s);
-      default: return PQC_ERR_UNSUPPORTED;
-    }
-  }
-  if (kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDefaultEnc)) {
+  if (n > 0 && !kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDenseEnc) && c->tune.fused_enc_tile != 64 && c->kat)
+    return kyber_staged_enc(c, k, n, ct, ss, pk, coins, s);
+  if (kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDenseEnc)) {
     switch (k) {
       case 2: return kyber::fused::launch_lowlat<2, false>(c, n, ss, ct, pk, coins, s);
       case 3: return kyber::fused::launch_lowlat<3, false>(c, n, ss, ct, pk, coins, s);

@@ -9,18 +9,18 @@
 // Between them: the noise bytes, the sampled entries and 96 bytes per request, in the
 // layouts the next stage reads (below).
 //
-//   decapsulation  k_open (indcpa_dec) -> k_sponge (H(ct); G, PRF; A^T)
-//                  -> k_reencrypt (indcpa_enc, verify, KDF)
-//   encapsulation  k_sponge (H(pk), m, G; A^T) -> k_prf -> k_reencrypt -> k_final
-//                  (H(ct), KDF)
-//   key generation k_key_seed (G) -> k_sponge (PRF; A) -> k_key_mul -> k_final (H(pk))
+//   decapsulation  k_open (indcpa_dec) -> k_dec_sponge (H(ct); G, PRF; A^T)
+//                  -> k_dec_reencrypt (indcpa_enc, verify) -> k_dec_kdf
+//   encapsulation  k_enc_sponge (H(pk), m, G; A^T) -> k_enc_prf -> k_enc_encrypt
+//                  (indcpa_enc) -> k_enc_final (H(ct), KDF)
+//   key generation k_key_seed (G) -> k_key_sponge (A; PRF) -> k_key_mul -> k_key_final (H(pk))
 //
 // Scratch, by group of 16 requests (request r of a bucket: group r / 16, slot r % 16;
 // dense batches have one bucket, mixed batches three whose groups follow each other):
 //   prf  [group][polynomial][chunk c][slot] 4 bytes: a wave's read of a chunk column is
 //        4 x 64 contiguous bytes, the writing lanes' stores too
 //   at   [group][entry][chunk c][slot] 16 bytes (8 coefficients)
-//   row  [group][slot] 128 bytes: m, Kbar, H(ct) or H(pk)
+//   row  [group][slot] 128 bytes: m, Kbar, H(ct) or the noise seed, mismatch
 //
 // The data flow and the reference functions are those of the 64-request tiles
 // (kyber_fused.hip); every path gives the same bytes.
@@ -215,6 +215,98 @@ __device__ __forceinline__ void dec_prf_wave(const Src& src, const Scratch& sc, 
     for (int nonce = 0; nonce < 2 * K + 1; ++nonce)
       prf_store(sc, b.grp0 + r / 16, r % 16, seed, nonce);
   }
+}
+
+// ---- encapsulation: sponge stages ---------------------------------------------------------
+// H(pk), m = H(coins) ("don't release system RNG output"), (Kbar, coins') = G(m || H(pk))
+// of 64 requests; coins' takes the row's hash place until the noise streams are drawn
+template <int K, class Src>
+__device__ __forceinline__ void enc_open_wave(const Src& src, const Scratch& sc, const Bucket& b, int w) {
+  using P = Params<K>;
+  const int r = 64 * w + (threadIdx.x & 63);
+  const bool act = r < b.n;
+  const int rc = act ? r : b.n - 1;
+  const ReqP q = src.template req<K, false>(rc);
+  uint64_t A[25], m[8], c4[4];
+  sponge_absorb_dense<kRateSha3_256>(A, q.key, P::pk_bytes / 8, 0x06);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) m[4 + i] = A[i];
+  load_words4(c4, q.coins);
+  absorb_fixed<kRateSha3_256, 4, true>(A, c4, 0x06);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) m[i] = A[i];
+  absorb_fixed<kRateSha3_512, 8, true>(A, m, 0x06);
+  if (act) {
+    uint8_t* row = sc.row_of(b.grp0 + r / 16, r % 16);
+    store_words4(row + kRowM, m);
+    store_words4(row + kRowKbar, A);
+    store_words4(row + kRowH, A + 4);
+  }
+}
+
+// noise stream `nonce` of 64 requests, from the seeds in the rows
+__device__ __forceinline__ void prf_wave(const Scratch& sc, const Bucket& b, int w, int nonce) {
+  const int r = 64 * w + (threadIdx.x & 63);
+  if (r >= b.n) return;
+  uint64_t seed[4];
+  load_words4(seed, sc.row_of(b.grp0 + r / 16, r % 16) + kRowH);
+  prf_store(sc, b.grp0 + r / 16, r % 16, seed, nonce);
+}
+
+// ss = KDF(Kbar, H(ct)) of 64 requests
+template <int K, class Src>
+__device__ __forceinline__ void enc_final_wave(const Src& src, const Scratch& sc, const Bucket& b, int w) {
+  using P = Params<K>;
+  const int r = 64 * w + (threadIdx.x & 63);
+  const bool act = r < b.n;
+  const int rc = act ? r : b.n - 1;
+  const ReqP q = src.template req<K, false>(rc);
+  uint64_t A[25], m[8];
+  sponge_absorb_dense<kRateSha3_256>(A, q.ct, P::ct_bytes / 8, 0x06);
+  const uint8_t* row = sc.row_of(b.grp0 + rc / 16, rc % 16);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    m[i] = load_u64_global(row + kRowKbar + 8 * i);
+    m[4 + i] = A[i];
+  }
+  absorb_fixed<kRateShake256, 8, true>(A, m, 0x1F);
+  if (act) store_words4(q.ss, A);
+}
+
+// ---- key generation: sponge stages -----------------------------------------------------------
+struct KeySrc {
+  uint8_t* pk;
+  uint8_t* sk;
+  const uint8_t* coins;  // 64 bytes per request: d || z
+};
+
+// (rho, sigma) = G(d) of 64 requests: rho into both copies of the public key, sigma into
+// the row, z into the secret key
+template <int K>
+__device__ __forceinline__ void key_seed_wave(const KeySrc& src, const Scratch& sc, int n, int w) {
+  using P = Params<K>;
+  const int r = 64 * w + (threadIdx.x & 63);
+  if (r >= n) return;
+  uint64_t d[4], z[4], A[25];
+  load_words4(d, src.coins + (size_t)r * 64);
+  load_words4(z, src.coins + (size_t)r * 64 + 32);
+  absorb_fixed<kRateSha3_512, 4, true>(A, d, 0x06);
+  uint8_t* sk = src.sk + (size_t)r * P::sk_bytes;
+  store_words4(src.pk + (size_t)r * P::pk_bytes + P::polyvec_bytes, A);
+  store_words4(sk + P::sk_cpa_bytes + P::polyvec_bytes, A);
+  store_words4(sk + P::z_off, z);
+  store_words4(sc.row_of(r / 16, r % 16) + kRowH, A + 4);
+}
+
+// H(pk) of 64 requests into the secret key
+template <int K>
+__device__ __forceinline__ void key_final_wave(const KeySrc& src, int n, int w) {
+  using P = Params<K>;
+  const int r = 64 * w + (threadIdx.x & 63);
+  const int rc = r < n ? r : n - 1;
+  uint64_t A[25];
+  sponge_absorb_dense<kRateSha3_256>(A, src.pk + (size_t)rc * P::pk_bytes, P::pk_bytes / 8, 0x06);
+  if (r < n) store_words4(src.sk + (size_t)r * P::sk_bytes + P::hpk_off, A);
 }
 
 // ---- product stages ----------------------------------------------------------------------
@@ -469,6 +561,56 @@ __device__ __forceinline__ void reencrypt_tile(const Src& src, const Scratch& sc
   }
 }
 
+// Key generation of a tile (indcpa_keypair, indcpa.cu:474-533): s^ = NTT(s) into the
+// secret key, t^ = A o s^ + NTT(e) into both copies of the public key, as canonical
+// residues (the reference's frommont(A o s^) + e^, csubq'd; A o s^ carries no Montgomery
+// factor here)
+template <int K>
+__device__ __forceinline__ void key_tile(const KeySrc& src, const Scratch& sc, const Bucket& b, int tile,
+                                         const DftLds<true, false>& sh) {
+  using P = Params<K>;
+  const Lane x = lane_of(b, tile);
+  uint8_t* sk = src.sk + (size_t)x.r * P::sk_bytes;
+  uint8_t* pk = src.pk + (size_t)x.r * P::pk_bytes;
+  HPoly sv[K];
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    noise_ntt(sv[j], sc, x, j, sh.fwd);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      uint32_t v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = f32::canon_f(h2_get(sv[j].v[k & 1][t][k >> 2], (k >> 1) & 1));
+      if (x.act) store_chunk<12>(sk + 384 * j, x.g, t, v);
+    }
+  }
+#pragma unroll 1
+  for (int i = 0; i < K; ++i) {
+#pragma unroll
+    for (int j = 0; j < K; ++j) keep_packed(sv[j]);
+    HPoly eh;
+    noise_ntt(eh, sc, x, K + i, sh.fwd);
+    const uint8_t* at = sc.at_chunk(x.grp, 0, i * K, 0);
+    row_product<K, Loaded16<K>>(
+        sv, sh.gamma, sh.gammaq, x.g,
+        [&](Loaded16<K>& l, int t) {
+#pragma unroll
+          for (int j = 0; j < K; ++j) l.w[j] = *(const global_t<u4v>*)(at + (j * 32 + 4 * t) * 256 + x.at_off());
+        },
+        [&](float (&a)[8], const Loaded16<K>& l, int j, int) { chunk_from16(a, l.w[j]); },
+        [&](int t, const f4v& e, const f4v& o) {
+          uint32_t v[8];
+#pragma unroll
+          for (int k = 0; k < 8; ++k)
+            v[k] = f32::canon_f(((k & 1) ? o[k >> 1] : e[k >> 1]) + h2_get(eh.v[k & 1][t][k >> 2], (k >> 1) & 1));
+          if (x.act) {
+            store_chunk<12>(pk + 384 * i, x.g, t, v);
+            store_chunk<12>(sk + P::sk_cpa_bytes + 384 * i, x.g, t, v);
+          }
+        });
+  }
+}
+
 // ss = KDF(Kbar or z, H(ct)) of 64 requests, one lane each
 template <int K, class Src>
 __device__ __forceinline__ void dec_kdf_wave(const Src& src, const Scratch& sc, const Bucket& b, int w) {
@@ -531,6 +673,73 @@ __global__ __launch_bounds__(64) void k_dec_kdf(int n, DenseSrc src, Scratch sc)
   for (int w = blockIdx.x; w < (n + 63) / 64; w += gridDim.x) dec_kdf_wave<K>(src, sc, Bucket{n, 0}, w);
 }
 
+// encapsulation: H(pk), m, G (the longest chains first), then the matrix entries
+template <int K>
+__global__ __launch_bounds__(64, 4) void k_enc_sponge(int n, DenseSrc src, Scratch sc) {
+  using P = Params<K>;
+  __shared__ SponLds sh;
+  const Bucket b{n, 0};
+  const int wr = (n + 63) / 64, total = wr + matrix_waves<K>(n);
+  for (int w = blockIdx.x; w < total; w += gridDim.x) {
+    if (w < wr)
+      enc_open_wave<K>(src, sc, b, w);
+    else
+      matrix_wave<K, true>(sc, b, w - wr, sh,
+                           [&](int r) { return src.template req<K, false>(r).key + P::polyvec_bytes; });
+  }
+}
+
+template <int K>
+__global__ __launch_bounds__(64, 4) void k_enc_prf(int n, Scratch sc) {
+  const int wr = (n + 63) / 64;
+  for (int w = blockIdx.x; w < wr * (2 * K + 1); w += gridDim.x) prf_wave(sc, Bucket{n, 0}, w % wr, w / wr);
+}
+
+template <int K>
+__global__ __launch_bounds__(kProdThreads, 2) void k_enc_encrypt(int n, DenseSrc src, Scratch sc) {
+  __shared__ DftLds<true, true> sh;
+  load_tables<true, true, kProdThreads>(sh, &c_dft);
+  const Bucket b{n, 0};
+  for (int tile = blockIdx.x; tile < (n + 63) / 64; tile += gridDim.x) reencrypt_tile<K, false>(src, sc, b, tile, sh);
+}
+
+template <int K>
+__global__ __launch_bounds__(64, 4) void k_enc_final(int n, DenseSrc src, Scratch sc) {
+  for (int w = blockIdx.x; w < (n + 63) / 64; w += gridDim.x) enc_final_wave<K>(src, sc, Bucket{n, 0}, w);
+}
+
+// key generation
+template <int K>
+__global__ __launch_bounds__(64, 4) void k_key_seed(int n, KeySrc src, Scratch sc) {
+  for (int w = blockIdx.x; w < (n + 63) / 64; w += gridDim.x) key_seed_wave<K>(src, sc, n, w);
+}
+
+template <int K>
+__global__ __launch_bounds__(64, 4) void k_key_sponge(int n, KeySrc src, Scratch sc) {
+  using P = Params<K>;
+  __shared__ SponLds sh;
+  const Bucket b{n, 0};
+  const int mw = matrix_waves<K>(n), wr = (n + 63) / 64;
+  for (int w = blockIdx.x; w < mw + 2 * K * wr; w += gridDim.x) {
+    if (w < mw)
+      matrix_wave<K, false>(sc, b, w, sh, [&](int r) { return src.pk + (size_t)r * P::pk_bytes + P::polyvec_bytes; });
+    else
+      prf_wave(sc, b, (w - mw) % wr, (w - mw) / wr);
+  }
+}
+
+template <int K>
+__global__ __launch_bounds__(kProdThreads, 2) void k_key_mul(int n, KeySrc src, Scratch sc) {
+  __shared__ DftLds<true, false> sh;
+  load_tables<true, false, kProdThreads>(sh, &c_dft);
+  for (int tile = blockIdx.x; tile < (n + 63) / 64; tile += gridDim.x) key_tile<K>(src, sc, Bucket{n, 0}, tile, sh);
+}
+
+template <int K>
+__global__ __launch_bounds__(64, 4) void k_key_final(int n, KeySrc src) {
+  for (int w = blockIdx.x; w < (n + 63) / 64; w += gridDim.x) key_final_wave<K>(src, n, w);
+}
+
 // ---- launchers ---------------------------------------------------------------------------------
 static Scratch scratch_of(const pqc_ctx* c, int k) {
   return Scratch{c->kprf, (size_t)(2 * k + 1) * 2048, reinterpret_cast<uint8_t*>(c->kat), (size_t)k * k * 16 * 512, c->krow, c->status};
@@ -570,6 +779,44 @@ static int dec(pqc_ctx* c, size_t n_all, uint8_t* ss, uint8_t* ct, const uint8_t
   return PQC_OK;
 }
 
+template <int K>
+static int enc(pqc_ctx* c, size_t n_all, uint8_t* ss, uint8_t* ct, const uint8_t* pk, const uint8_t* coins,
+               hipStream_t s) {
+  using P = Params<K>;
+  const Scratch sc = scratch_of(c, K);
+  for (size_t at = 0; at < n_all; at += c->kstage_max) {
+    const int n = (int)std::min(n_all - at, c->kstage_max);
+    const int tiles = (n + 63) / 64;
+    const DenseSrc src{ss + at * 32, ct + at * P::ct_bytes, pk + at * P::pk_bytes, coins + at * 32, c->kprf};
+    hipLaunchKernelGGL((k_enc_sponge<K>), dim3(sponge_grid(c, tiles + matrix_waves<K>(n))), dim3(64), 0, s, n, src, sc);
+    hipLaunchKernelGGL((k_enc_prf<K>), dim3(sponge_grid(c, tiles * (2 * K + 1))), dim3(64), 0, s, n, sc);
+    hipLaunchKernelGGL((k_enc_encrypt<K>), dim3(prod_grid(c, tiles)), dim3(kProdThreads), 0, s, n, src, sc);
+    hipLaunchKernelGGL((k_enc_final<K>), dim3(sponge_grid(c, tiles)), dim3(64), 0, s, n, src, sc);
+    const int rc = hip_err(hipGetLastError());
+    if (rc) return rc;
+  }
+  return PQC_OK;
+}
+
+template <int K>
+static int keypair(pqc_ctx* c, size_t n_all, uint8_t* pk, uint8_t* sk, const uint8_t* coins, hipStream_t s) {
+  using P = Params<K>;
+  const Scratch sc = scratch_of(c, K);
+  for (size_t at = 0; at < n_all; at += c->kstage_max) {
+    const int n = (int)std::min(n_all - at, c->kstage_max);
+    const int tiles = (n + 63) / 64;
+    const KeySrc src{pk + at * P::pk_bytes, sk + at * P::sk_bytes, coins + at * 64};
+    hipLaunchKernelGGL((k_key_seed<K>), dim3(sponge_grid(c, tiles)), dim3(64), 0, s, n, src, sc);
+    hipLaunchKernelGGL((k_key_sponge<K>), dim3(sponge_grid(c, matrix_waves<K>(n) + 2 * K * tiles)), dim3(64), 0, s, n,
+                       src, sc);
+    hipLaunchKernelGGL((k_key_mul<K>), dim3(prod_grid(c, tiles)), dim3(kProdThreads), 0, s, n, src, sc);
+    hipLaunchKernelGGL((k_key_final<K>), dim3(sponge_grid(c, tiles)), dim3(64), 0, s, n, src);
+    const int rc = hip_err(hipGetLastError());
+    if (rc) return rc;
+  }
+  return PQC_OK;
+}
+
 }  // namespace staged
 }  // namespace kyber
 
@@ -581,6 +828,25 @@ int kyber_staged_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct
     case 2: return kyber::staged::dec<2>(c, n, ss, ctm, sk, s);
     case 3: return kyber::staged::dec<3>(c, n, ss, ctm, sk, s);
     case 4: return kyber::staged::dec<4>(c, n, ss, ctm, sk, s);
+    default: return PQC_ERR_UNSUPPORTED;
+  }
+}
+
+int kyber_staged_enc(pqc_ctx* c, int k, size_t n, uint8_t* ct, uint8_t* ss, const uint8_t* pk, const uint8_t* coins,
+                     hipStream_t s) {
+  switch (k) {
+    case 2: return kyber::staged::enc<2>(c, n, ss, ct, pk, coins, s);
+    case 3: return kyber::staged::enc<3>(c, n, ss, ct, pk, coins, s);
+    case 4: return kyber::staged::enc<4>(c, n, ss, ct, pk, coins, s);
+    default: return PQC_ERR_UNSUPPORTED;
+  }
+}
+
+int kyber_staged_keypair(pqc_ctx* c, int k, size_t n, uint8_t* pk, uint8_t* sk, const uint8_t* coins, hipStream_t s) {
+  switch (k) {
+    case 2: return kyber::staged::keypair<2>(c, n, pk, sk, coins, s);
+    case 3: return kyber::staged::keypair<3>(c, n, pk, sk, coins, s);
+    case 4: return kyber::staged::keypair<4>(c, n, pk, sk, coins, s);
     default: return PQC_ERR_UNSUPPORTED;
   }
 }

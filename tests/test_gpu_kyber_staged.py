@@ -52,3 +52,22 @@ def test_staged_decaps_vs_oracle(pqc, k, grid):
         got = ctx.dec_host(ALG[k], ct, sk)
         assert (got == want).all(), np.nonzero((got != want).any(axis=1))[0][:8]
     ctx.close()
+
+
+@pytest.mark.parametrize("grid", [0, 1])
+@pytest.mark.parametrize("k", [2, 3, 4])
+def test_staged_keypair_and_encaps_vs_oracle(pqc, k, grid):
+    ctx = staged_ctx(pqc, k, max(SIZES), grid)
+    for n in SIZES:
+        print("staged keypair and encaps k", k, "n", n, "grid", grid, flush=True)
+        rng = np.random.default_rng(2000 * k + n)
+        coins = rng.integers(0, 256, (n, 64), dtype=np.uint8)
+        pk, sk = ctx.keypair_host(ALG[k], coins)
+        opk, osk = O.kyber_batch("keypair", k, [coins])
+        assert (pk == opk).all() and (sk == osk).all()
+        pk, _, _ = inputs(k, n, 3000 * k + n)  # every fourth public key of arbitrary bytes
+        coins = rng.integers(0, 256, (n, 32), dtype=np.uint8)
+        ct, ss = ctx.enc_host(ALG[k], pk, coins)
+        oct_, oss = O.kyber_batch("enc", k, [pk, coins])
+        assert (ct == oct_).all() and (ss == oss).all()
+    ctx.close()
