@@ -82,17 +82,16 @@ typedef struct pqc_tuning {
   int32_t frodo_stream_block; /* threads per workgroup of the Frodo noise-stream kernel: 64, 128 or 256 */
   int32_t lowlat_max;         /* Kyber batches of at most this many requests run one four-wave
                                  workgroup per request (latency) instead of the throughput forms
-                                 below: 0 = library defaults (1024 decapsulations and 256
-                                 encapsulations of one parameter set, 8192 and 4096 mixed), -1 = never, else 1..65536
+                                 below: 0 = library defaults (1024 decapsulations, 256
+                                 encapsulations, 512 in a mixed batch), -1 = never, else 1..65536
                                  for all */
   int32_t frodo_chunk;        /* FrodoKEM-976 batches under one key above this many requests are cut
                                  into chunks of this many, run on four streams: 0 = library default
                                  (no split up to 65536), else a multiple of 32 in 32..65536 */
   int32_t fused_dec_tile;     /* fused Kyber decapsulation: 64 = one persistent kernel over 64-request tiles
-                                 (one wave per SIMD, A^T in an LDS ring); 32 = the throughput form, whose
-                                 entries A^T go through a global scratch: sponge and matrix-core stages
-                                 (one parameter set) or 32-request tiles at two waves per SIMD (mixed
-                                 batches); 0 = library default (32) */
+                                 (one wave per SIMD, A^T in an LDS ring); 32 = the throughput form, sponge
+                                 and matrix-core stages with A^T in a global scratch; 0 = library
+                                 default (32) */
   int32_t fused_enc_tile;     /* the same for the fused Kyber encapsulation */
   int32_t fused_key_tile;     /* the same for the fused Kyber key generation */
   int32_t frodo_lane_min;     /* Keccak lane layout of the FrodoKEM-976 noise stream and F prefix in
@@ -149,7 +148,7 @@ int crypto_kem_enc_batch(pqc_ctx *ctx, int alg, size_t n, uint8_t *ct, uint8_t *
  * installed in the context and returned.                                       */
 #define PQC_TUNE_PLAIN_KYBER 0 /* plain_block */
 #define PQC_TUNE_FUSED_KYBER 1 /* fused_waves_per_cu */
-#define PQC_TUNE_MIXED_KYBER 2 /* fused_waves_per_cu x tile layout: 32-request tiles both ways, or
+#define PQC_TUNE_MIXED_KYBER 2 /* fused_waves_per_cu x tile layout: the stages both ways, or
                                   64-request tiles (fused_enc_tile = fused_dec_tile = 64) in mixed_order 0, 1, 3 */
 #define PQC_TUNE_FRODO 3       /* frodo_stream_block x Keccak lane layout (frodo_lane_min) */
 #define PQC_TUNE_NEWHOPE 4     /* newhope_block */

@@ -491,456 +491,6 @@ __device__ __forceinline__ void fused_tile(const Src& src, int base, int n, Lds<
   __syncthreads();
 }
 
-// ---- decapsulation in 32-request tiles, two waves per SIMD --------------------------
-// fused_tile runs one wave per SIMD: a batch of 65536 is 1024 tiles, one per SIMD,
-// and its A^T ring takes 40 KB of LDS, so four waves fill a CU's 160 KB.  A lone
-// wave issues a VALU instruction every ~4.8 cycles; two waves per SIMD issue the
-// same Keccak mix at ~3.9 cycles per instruction per SIMD (measured on MI355X).
-// This tile serves 32 requests, so 65536 requests are 2048 waves, two per SIMD,
-// and its A^T entries go to a per-wave global scratch (written and read back by
-// the same wave while the lines are in L2) instead of LDS: ~1.2 KB of LDS per
-// wave.  So that the per-request sponge chains still keep all 64 lanes busy with
-// 32 requests, lanes 0..31 absorb H(ct) of request `lane` while lanes 32..63
-// compute G and the 2K + 1 PRF outputs of request `lane - 32` in the same
-// permutations (H(ct) is the longer chain for every K).  Same bytes as fused_tile.
-template <int K>
-struct Tile32 {
-  static constexpr int T = 32;
-  static constexpr int KK = K * K;
-  static constexpr int NR = (T * KK + 63) / 64;                              // sampling rounds: 2, 5, 8
-  static constexpr int HB = Params<K>::ct_bytes / 8 / kRateSha3_256 + 1;     // H(ct) blocks: 6, 9, 12
-  static constexpr int ENTRIES = 64 * NR;                                    // scratch entries per wave
-  static_assert(HB >= 2 * K + 2, "the H(ct) lanes run the longest chain of the sponge phase");
-};
-constexpr int kAtStride = 264;  // int16 per A^T entry in the scratch: 256 + guard slots, 16-byte multiple
-static_assert(kAtStride >= N + 4 && (kAtStride * 2) % 16 == 0, "entry stride");
-
-// Sampling stage: one row per lane.  A block's candidates go to the row at their
-// entry position minus base8 (the entry's last 8-aligned position before the
-// block), so that whole 16-byte chunks can be copied to the global entry; the
-// row holds the 0..7 earlier coefficients of that chunk and the block's <= 84
-// candidates written at the running position (the last write at most at index
-// 7 + 83), and the chunk copies read up to the next multiple of 8.  A 208-byte
-// row (13 x 16 B) spreads the lanes' rows over 16 bank offsets.
-constexpr int kStageRow = 104;  // int16 per lane row
-static_assert(7 + 84 + 7 <= kStageRow && kStageRow % 8 == 0 && (kStageRow / 8) % 2 == 1, "stage row");
-
-struct Lds32 {
-  alignas(16) int16_t stage[64][kStageRow];
-  uint8_t msg[32][32];
-  uint32_t fail[32];
-};
-
-// SHAKE128(rho || x || y) rejection-sampled into the global entry `dst` (as
-// sample_entry: the accepted candidates themselves), through this lane's LDS
-// stage row: after each block the chunks
-// [base8, round_up_8(ctr)) are copied to dst with 16-byte stores, and the last,
-// partial chunk moves to the front of the row for the next block.  So every
-// global store is a whole 16 bytes of one entry (a 2-byte store per candidate
-// would be one L2 request each).  Returns the accept count, clamped at 256.
-__device__ __forceinline__ int sample_entry_staged(global_t<int16_t>* dst, int16_t* row, const uint64_t (&rho)[4],
-                                                   int x, int y, bool valid) {
-  uint64_t A[25];
-#pragma unroll
-  for (int t = 0; t < 25; ++t) A[t] = (t < 4) ? rho[t] : 0;
-  A[4] = (uint64_t)x | ((uint64_t)y << 8) | (0x1Full << 16);
-  A[kRateShake128 - 1] ^= 0x8000000000000000ull;
-  int ctr = 0, base8 = 0;
-  for (int blk = 0; blk < kMaxBlocks; ++blk) {
-    if (blk >= 4 && !__any(valid && ctr < N)) break;
-    keccakf1600(A);
-    int16_t* p = row + (ctr - base8);
-    int16_t* const pend = row + (N - base8);  // position N: the clamp
-#pragma unroll
-    for (int w = 0; w < kRateShake128; ++w) {
-      const uint32_t half[2] = {(uint32_t)A[w], (uint32_t)(A[w] >> 32)};
-#pragma unroll
-      for (int h = 0; h < 4; ++h) {
-        const uint32_t val = (h & 1) ? (half[h >> 1] >> 16) : (half[h >> 1] & 0xFFFFu);
-        *p = (int16_t)val;  // overwritten by the next candidate unless accepted
-        p += val < 19u * Q ? 1 : 0;
-      }
-      p = p < pend ? p : pend;
-    }
-    ctr = base8 + (int)(p - row);
-    // whole 16-byte chunks of [base8, ctr): at most (7 + 84 + 7) / 8 = 12
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    const int nchunks = (ctr - base8 + 7) >> 3;
-#pragma unroll
-    for (int c = 0; c < (7 + 84 + 7) / 8; ++c) {
-      if (c < nchunks) {
-        const u32x4 v = *reinterpret_cast<const u32x4*>(row + 8 * c);
-        *(global_t<u32x4>*)(dst + base8 + 8 * c) = v;
-      }
-    }
-    // the partial chunk that holds position ctr starts the row for the next block
-    const int keep = (ctr & ~7) - base8;
-    const u32x4 t = *reinterpret_cast<const u32x4*>(row + keep);
-    *reinterpret_cast<u32x4*>(row) = t;
-    base8 = ctr & ~7;
-  }
-  return ctr;
-}
-
-// This lane's group of the A^T entries of one request, loaded from the scratch
-// ahead of their use (the entries of request t start at entry t K^2).
-template <int K>
-struct AtRegs {
-  uint32_t w[K * K][2];
-  __device__ __forceinline__ void load(const global_t<int16_t>* at, int t) {
-    const global_t<uint32_t>* p =
-        (const global_t<uint32_t>*)(at + (size_t)t * K * K * kAtStride + 4 * ntt_group(lane_id()));
-#pragma unroll
-    for (int e = 0; e < K * K; ++e) {
-      w[e][0] = p[e * (kAtStride / 2)];
-      w[e][1] = p[e * (kAtStride / 2) + 1];
-    }
-  }
-  __device__ __forceinline__ void get(int i, int j, uint32_t& w0, uint32_t& w1) const {
-    w0 = w[i * K + j][0];
-    w1 = w[i * K + j][1];
-  }
-};
-
-// The A^T rounds of a 32-request tile: round g samples entries 64 g .. 64 g + 63
-// (entry E = request E / K^2, position E % K^2) into the scratch, then re-encrypts
-// every request whose entries are all sampled (request t's words load during
-// request t - 1).  Decapsulation compares with the ciphertext and sets sh.fail[t];
-// encapsulation writes the ciphertext.
-template <int K, bool DEC>
-__device__ __forceinline__ void at_reencrypt32(const ReqP& me, int nt, Lds32& sh, global_t<int16_t>* at,
-                                               const LaneZF& z, uint32_t* __restrict__ status) {
-  using P = Params<K>;
-  using TL = Tile32<K>;
-  constexpr int PK_OFF = DEC ? P::sk_cpa_bytes : 0;  // public key inside the key buffer
-  const int lane = threadIdx.x;
-  const int ng = (nt * TL::KK + 63) / 64;
-  int t_done = 0;
-  auto load_rho = [&](uint64_t (&rho)[4], int g) {
-    const int t = (64 * g + lane) / TL::KK;
-    const uint8_t* key = reinterpret_cast<const uint8_t*>(__shfl((long long)me.key, t < nt ? t : 0));
-#pragma unroll
-    for (int w = 0; w < 4; ++w) rho[w] = load_u64_global(key + PK_OFF + P::polyvec_bytes + 8 * w);
-  };
-  uint64_t rho_next[4];
-  load_rho(rho_next, 0);
-  for (int g = 0; g < ng; ++g) {
-    {
-      const int E = 64 * g + lane;
-      const int t = E / TL::KK;
-      const int ij = E % TL::KK;
-      const bool valid = t < nt;
-      uint64_t rho[4];
-#pragma unroll
-      for (int w = 0; w < 4; ++w) rho[w] = rho_next[w];
-      const int got = sample_entry_staged(at + (size_t)E * kAtStride, sh.stage[lane], rho, ij / K, ij % K, valid);
-      if (valid && got < N) atomicOr(status, 1u);
-    }
-    __syncthreads();  // the round's entries are in the scratch for every lane
-    if (g + 1 < ng) load_rho(rho_next, g + 1);
-    const int t_end = min(nt, (64 * (g + 1)) / TL::KK);
-    if (t_done < t_end) {
-      EncIn<K, DEC> cur, nxt;
-      {
-        const ReqP q = lane_req(me, t_done);
-        enc_load<K, DEC>(nxt, q.prf, q.key + PK_OFF, q.ct);
-      }
-      for (int t = t_done; t < t_end; ++t) {
-        cur = nxt;
-        if (t + 1 < t_end) {
-          const ReqP q = lane_req(me, t + 1);
-          enc_load<K, DEC>(nxt, q.prf, q.key + PK_OFF, q.ct);
-        }
-        AtRegs<K> a;
-        a.load(at, t);
-        if constexpr (DEC) {
-          const uint32_t mm = coop_reencrypt_f<K, true>(a, cur, sh.msg[t], nullptr, z);
-          const uint32_t f = __any(mm != 0) ? 1u : 0u;
-          if (lane == 0) sh.fail[t] = f;
-        } else {
-          coop_reencrypt_f<K, false>(a, cur, sh.msg[t], lane_req(me, t).ct, z);
-        }
-      }
-      t_done = t_end;
-    }
-  }
-}
-
-template <int K, class Src>
-__device__ __forceinline__ void dec_tile32(const Src& src, int base, int n, Lds32& sh, global_t<int16_t>* at,
-                                           const LaneZF& z, uint32_t* __restrict__ status) {
-  using P = Params<K>;
-  using TL = Tile32<K>;
-  const int lane = threadIdx.x;
-  const int rq = lane & 31;  // the request this lane serves in the sponge phases (lanes l and l + 32 alike)
-  const int nt = min(TL::T, n - base);
-  const bool act = rq < nt;
-  const ReqP me = src.template req<K, true>(act ? base + rq : base);
-  const bool hl = lane < 32;  // H(ct) lane; the others compute G and the PRF outputs
-
-  // ---- indcpa_dec, wave-cooperative, one request at a time; request t's words are
-  // loaded during request t - 1
-  {
-    DecIn<K> cur, nxt;
-    {
-      const ReqP q = lane_req(me, 0);
-      dec_load<K>(nxt, q.ct, q.key);
-    }
-    for (int t = 0; t < nt; ++t) {
-      cur = nxt;
-      if (t + 1 < nt) {
-        const ReqP q = lane_req(me, t + 1);
-        dec_load<K>(nxt, q.ct, q.key);
-      }
-      coop_indcpa_dec_f<K>(cur, z, sh.msg[t]);
-    }
-  }
-  __syncthreads();
-
-  // ---- one sponge phase: lanes 0..31 H(ct) (SHA3-256, HB blocks); lanes 32..63
-  // step 0: (Kbar, coins) = G(m || H(pk)), steps 1 .. 2K+1: PRF(coins, step - 1)
-  uint64_t hct[4], kbar[4] = {0, 0, 0, 0};
-  {
-    constexpr int W = P::ct_bytes / 8;
-    constexpr int R = kRateSha3_256;
-    static_assert(W >= R, "the first H(ct) block is whole");
-    const global_t<uint64_t>* cw = gptr(reinterpret_cast<const uint64_t*>(me.ct));
-    uint64_t A[25], cur[R], coins[4];
-#pragma unroll
-    for (int i = 0; i < 25; ++i) A[i] = 0;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) coins[w] = 0;
-    if (hl) {
-#pragma unroll
-      for (int w = 0; w < R; ++w) cur[w] = cw[w];
-    } else {
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        A[w] = load_u64(sh.msg[rq] + 8 * w);
-        A[4 + w] = load_u64_global(me.key + P::hpk_off + 8 * w);
-      }
-      A[8] ^= 0x06;
-      A[kRateSha3_512 - 1] ^= 0x8000000000000000ull;
-    }
-    for (int st = 0; st < TL::HB; ++st) {
-      if (hl) {
-        const int rem = W - st * R;  // message words left (uniform), >= 0
-#pragma unroll
-        for (int w = 0; w < R; ++w) {
-          if (w < rem) A[w] ^= cur[w];
-          if (w == rem) A[w] ^= 0x06;
-        }
-        if (st == TL::HB - 1) A[R - 1] ^= 0x8000000000000000ull;
-        // the next block's words load during this permutation
-#pragma unroll
-        for (int w = 0; w < R; ++w)
-          if (w < rem - R) cur[w] = cw[(st + 1) * R + w];
-      } else if (st >= 1 && st <= 2 * K + 1) {
-#pragma unroll
-        for (int i = 0; i < 25; ++i) A[i] = i < 4 ? coins[i] : 0;
-        A[4] = (uint64_t)(st - 1) | (0x1Full << 8);
-        A[kRateShake256 - 1] ^= 0x8000000000000000ull;
-      }
-      keccakf1600(A);
-      if (!hl) {
-        if (st == 0) {
-#pragma unroll
-          for (int w = 0; w < 4; ++w) {
-            kbar[w] = A[w];
-            coins[w] = A[4 + w];
-          }
-        } else if (st <= 2 * K + 1 && act) {
-#pragma unroll
-          for (int w = 0; w < 16; ++w) store_u64(me.prf + 128 * (st - 1) + 8 * w, A[w]);
-        }
-      }
-    }
-#pragma unroll
-    for (int w = 0; w < 4; ++w) hct[w] = A[w];  // lanes 0..31
-  }
-  __syncthreads();
-
-  // ---- A^T rounds of 64 entries into the scratch, then the re-encryption of every
-  // request whose entries are complete
-  at_reencrypt32<K, true>(me, nt, sh, at, z, status);
-  __syncthreads();
-
-  // ---- KDF(Kbar or z, H(ct)) on lanes 0..31; Kbar comes from lane + 32
-  {
-    uint64_t m[8], A[25];
-    const uint64_t mask = 0 - (uint64_t)(sh.fail[rq] & 1u);
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const uint64_t kb = (uint64_t)__shfl_xor((long long)kbar[w], 32);
-      const uint64_t zz = load_u64_global(me.key + P::z_off + 8 * w);
-      m[w] = kb ^ (mask & (zz ^ kb));
-      m[4 + w] = hct[w];
-    }
-    absorb_fixed<kRateShake256, 8>(A, m, 0x1F);
-    if (hl && act) {
-#pragma unroll
-      for (int w = 0; w < 4; ++w) store_u64(me.ss + 8 * w, A[w]);
-    }
-  }
-  __syncthreads();
-}
-
-// Encapsulation in the same 32-request tiles.  The first sponge phase runs
-// H(pk) (the longest chain) on lanes 0..31 while lanes 32..63 compute
-// m = H(coins) ("don't release system RNG output") in its first permutation;
-// then both lanes of a pair compute G(m || H(pk)) and split the 2K + 1 PRF
-// outputs (lane l the even nonces, lane l + 32 the odd ones); the A^T rounds
-// and re-encryptions write the ciphertexts; H(ct) and the KDF end it.  Same
-// bytes as fused_tile<K, false>.
-template <int K>
-struct EncTile32 {
-  static constexpr int HB = Params<K>::pk_bytes / 8 / kRateSha3_256 + 1;  // H(pk) blocks: 6, 9, 12
-  static_assert(Params<K>::pk_bytes / 8 >= kRateSha3_256, "the first H(pk) block is whole");
-};
-
-template <int K, class Src>
-__device__ __forceinline__ void enc_tile32(const Src& src, int base, int n, Lds32& sh, global_t<int16_t>* at,
-                                           const LaneZF& z, uint32_t* __restrict__ status) {
-  using P = Params<K>;
-  using TL = Tile32<K>;
-  const int lane = threadIdx.x;
-  const int rq = lane & 31;  // the request this lane serves in the sponge phases (lanes l and l + 32 alike)
-  const int nt = min(TL::T, n - base);
-  const bool act = rq < nt;
-  const ReqP me = src.template req<K, false>(act ? base + rq : base);
-  const bool hl = lane < 32;  // H(pk) lane; the others compute m = H(coins)
-
-  // ---- lanes 0..31: H(pk) (SHA3-256, HB blocks); lanes 32..63: m = H(coins)
-  uint64_t hpk[4];
-  {
-    constexpr int W = P::pk_bytes / 8;
-    constexpr int R = kRateSha3_256;
-    const global_t<uint64_t>* pw = gptr(reinterpret_cast<const uint64_t*>(me.key));
-    uint64_t A[25], cur[R];
-#pragma unroll
-    for (int i = 0; i < 25; ++i) A[i] = 0;
-    if (hl) {
-#pragma unroll
-      for (int w = 0; w < R; ++w) cur[w] = pw[w];
-    } else {
-#pragma unroll
-      for (int w = 0; w < 4; ++w) A[w] = load_u64_global(me.coins + 8 * w);
-      A[4] ^= 0x06;
-      A[R - 1] ^= 0x8000000000000000ull;
-    }
-    for (int st = 0; st < EncTile32<K>::HB; ++st) {
-      if (hl) {
-        const int rem = W - st * R;  // message words left (uniform), >= 0
-#pragma unroll
-        for (int w = 0; w < R; ++w) {
-          if (w < rem) A[w] ^= cur[w];
-          if (w == rem) A[w] ^= 0x06;
-        }
-        if (st == EncTile32<K>::HB - 1) A[R - 1] ^= 0x8000000000000000ull;
-        // the next block's words load during this permutation
-#pragma unroll
-        for (int w = 0; w < R; ++w)
-          if (w < rem - R) cur[w] = pw[(st + 1) * R + w];
-      }
-      keccakf1600(A);
-      if (!hl && st == 0 && act) {
-#pragma unroll
-        for (int w = 0; w < 4; ++w) store_u64(sh.msg[rq] + 8 * w, A[w]);
-      }
-    }
-#pragma unroll
-    for (int w = 0; w < 4; ++w) hpk[w] = A[w];  // lanes 0..31
-  }
-  __syncthreads();
-
-  // ---- (Kbar, coins) = G(m || H(pk)) on both lanes of a pair, then PRF(coins,
-  // 2 i + (lane >= 32)) for i = 0 .. K (lane l + 32's last one, nonce 2K + 1, unused)
-  uint64_t kbar[4];
-  {
-    uint64_t m[8], A[25], coins[4];
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      m[w] = load_u64(sh.msg[rq] + 8 * w);
-      m[4 + w] = (uint64_t)__shfl((long long)hpk[w], rq);
-    }
-    absorb_fixed<kRateSha3_512, 8>(A, m, 0x06);
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      kbar[w] = A[w];
-      coins[w] = A[4 + w];
-    }
-    for (int i = 0; i <= K; ++i) {
-      const int nonce = 2 * i + (hl ? 0 : 1);
-      absorb_fixed<kRateShake256, 4>(A, coins, (uint64_t)nonce | (0x1Full << 8));
-      if (act && nonce <= 2 * K) {
-#pragma unroll
-        for (int w = 0; w < 16; ++w) store_u64(me.prf + 128 * nonce + 8 * w, A[w]);
-      }
-    }
-  }
-  __syncthreads();
-
-  // ---- A^T rounds and the re-encryptions, which write the ciphertexts
-  at_reencrypt32<K, false>(me, nt, sh, at, z, status);
-  __syncthreads();
-
-  // ---- KDF(Kbar, H(ct)); both lanes of a pair compute it, lanes 0..31 store
-  {
-    uint64_t m[8], A[25];
-    sponge_absorb_words_prefetch<kRateSha3_256>(A, reinterpret_cast<const uint64_t*>(me.ct), P::ct_bytes / 8, 0x06);
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      m[w] = kbar[w];
-      m[4 + w] = A[w];
-    }
-    absorb_fixed<kRateShake256, 8>(A, m, 0x1F);
-    if (hl && act) {
-#pragma unroll
-      for (int w = 0; w < 4; ++w) store_u64(me.ss + 8 * w, A[w]);
-    }
-  }
-  __syncthreads();
-}
-
-// Mixed batches: the bucketed requests (k_mixed_classify) in 32-request tiles at
-// two waves per SIMD, K = 4 tiles first (the longest), then K = 3, then K = 2;
-// each wave's A^T scratch region holds `region` int16 (sized for the largest K
-// the context holds).
-template <bool DEC>
-__device__ __forceinline__ void mixed32_body(const MixedSrc& src, const uint32_t* __restrict__ counts,
-                                             int16_t* at_scratch, size_t region, uint32_t* __restrict__ status) {
-  __shared__ Lds32 sh;
-  LaneZF z;
-  load_lane_zf(z, &c_lane_twf);
-  global_t<int16_t>* at = (global_t<int16_t>*)(at_scratch + (size_t)blockIdx.x * region);
-  const int n2 = (int)counts[0], n3 = (int)counts[1], n4 = (int)counts[2];
-  const int t4 = (n4 + 31) / 32, t3 = (n3 + 31) / 32, t2 = (n2 + 31) / 32;
-  for (int tile = blockIdx.x; tile < t4 + t3 + t2; tile += gridDim.x) {
-    if (tile < t4) {
-      if constexpr (DEC) dec_tile32<4>(src, tile * 32, n4, sh, at, z, status);
-      else enc_tile32<4>(src, tile * 32, n4, sh, at, z, status);
-    } else if (tile < t4 + t3) {
-      if constexpr (DEC) dec_tile32<3>(src, (tile - t4) * 32, n3, sh, at, z, status);
-      else enc_tile32<3>(src, (tile - t4) * 32, n3, sh, at, z, status);
-    } else {
-      if constexpr (DEC) dec_tile32<2>(src, (tile - t4 - t3) * 32, n2, sh, at, z, status);
-      else enc_tile32<2>(src, (tile - t4 - t3) * 32, n2, sh, at, z, status);
-    }
-  }
-}
-
-__global__ __launch_bounds__(64, 2) void k_fused_mixed_dec32(MixedSrc src, const uint32_t* __restrict__ counts,
-                                                            int16_t* at_scratch, size_t region,
-                                                            uint32_t* __restrict__ status) {
-  mixed32_body<true>(src, counts, at_scratch, region, status);
-}
-
-__global__ __launch_bounds__(64, 2) void k_fused_mixed_enc32(MixedSrc src, const uint32_t* __restrict__ counts,
-                                                            int16_t* at_scratch, size_t region,
-                                                            uint32_t* __restrict__ status) {
-  mixed32_body<false>(src, counts, at_scratch, region, status);
-}
-
 // ---- key generation -----------------------------------------------------------------
 // indcpa_keypair (Kyber_GPU_Batched/indcpa.cu:474-564) + the KEM tail: (rho, sigma)
 // = G(d); s_j = CBD(PRF(sigma, j)), e_i = CBD(PRF(sigma, K + i)), both through
@@ -1604,14 +1154,12 @@ static int launch_fused(pqc_ctx* c, size_t n, uint8_t* ss, uint8_t* ct, const ui
 }
 
 // Kyber batches of at most this many requests take the one-workgroup-per-request
-// kernels.  Batches of one parameter set go to the staged path above that
-// (kyber_staged.hip): measured on MI355X (Kyber-768), the per-request kernels take 123 us
-// for 761 decapsulations, 145 for 1024, 219 for 2048 and 257 us for 300 encapsulations,
-// the stages 158 us at 761, 163 at 2048 and 239 us at 300.  For mixed batches a 32-request
-// tile launch is the alternative, and the per-request kernels win below ~10 K
-// decapsulations and ~5 K encapsulations.  tuning.lowlat_max overrides them all
-// (-1 = never).
-constexpr int kLowLatDenseDec = 1024, kLowLatDenseEnc = 256, kLowLatDefaultDec = 8192, kLowLatDefaultEnc = 4096;
+// kernels, larger ones the stages (kyber_staged.hip).  Measured on MI355X (Kyber-768),
+// per-request against staged: 123 / 158 us for 761 decapsulations, 145 / 160 for 1024,
+// 219 / 163 for 2048; 233 / 238 us for 64 encapsulations, 257 / 239 for 300.  Mixed
+// 1:2:1, encapsulation + decapsulation: 441 / 542 us at 300, 529 / 541 at 1000, 1123 /
+// 574 at 3000.  tuning.lowlat_max overrides them all (-1 = never).
+constexpr int kLowLatDec = 1024, kLowLatEnc = 256, kLowLatMixedEnc = 512;
 
 inline bool use_lowlat(const pqc_ctx* c, size_t n, int dflt) {
   const int lim = c->tune.lowlat_max != 0 ? c->tune.lowlat_max : dflt;
@@ -1650,17 +1198,11 @@ int kyber_fused_keypair(pqc_ctx* c, int k, size_t n, uint8_t* pk, uint8_t* sk, c
   }
 }
 
-size_t tile32_scratch_bytes(int k) {
-  using namespace kyber::fused;
-  const int entries = k == 2 ? Tile32<2>::ENTRIES : k == 3 ? Tile32<3>::ENTRIES : Tile32<4>::ENTRIES;
-  return (size_t)entries * kAtStride * sizeof(int16_t);
-}
-
 int kyber_fused_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct, const uint8_t* sk, hipStream_t s) {
   uint8_t* ctm = const_cast<uint8_t*>(ct);  // read-only in the decaps instantiation
-  if (n > 0 && !kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDenseDec) && c->tune.fused_dec_tile != 64 && c->kat)
+  if (n > 0 && !kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDec) && c->tune.fused_dec_tile != 64 && c->kat)
     return kyber_staged_dec(c, k, n, ss, ct, sk, s);
-  if (kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDenseDec)) {
+  if (kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDec)) {
     switch (k) {
       case 2: return kyber::fused::launch_lowlat<2, true>(c, n, ss, ctm, sk, nullptr, s);
       case 3: return kyber::fused::launch_lowlat<3, true>(c, n, ss, ctm, sk, nullptr, s);
@@ -1678,9 +1220,9 @@ int kyber_fused_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct,
 
 int kyber_fused_enc(pqc_ctx* c, int k, size_t n, uint8_t* ct, uint8_t* ss, const uint8_t* pk, const uint8_t* coins,
                     hipStream_t s) {
-  if (n > 0 && !kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDenseEnc) && c->tune.fused_enc_tile != 64 && c->kat)
+  if (n > 0 && !kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatEnc) && c->tune.fused_enc_tile != 64 && c->kat)
     return kyber_staged_enc(c, k, n, ct, ss, pk, coins, s);
-  if (kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDenseEnc)) {
+  if (kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatEnc)) {
     switch (k) {
       case 2: return kyber::fused::launch_lowlat<2, false>(c, n, ss, ct, pk, coins, s);
       case 3: return kyber::fused::launch_lowlat<3, false>(c, n, ss, ct, pk, coins, s);
@@ -1705,7 +1247,7 @@ int kyber_fused_mixed(pqc_ctx* c, int dec, size_t n, const pqc_kem_req* reqs, ui
   using namespace kyber::fused;
   if (n == 0) return PQC_OK;
   if (!c->kmix_order || !c->kprf) return PQC_ERR_UNSUPPORTED;
-  if (use_lowlat(c, n, dec ? kLowLatDefaultDec : kLowLatDefaultEnc)) {  // one workgroup per descriptor, no bucketing
+  if (use_lowlat(c, n, dec ? kLowLatDec : kLowLatMixedEnc)) {  // one workgroup per descriptor, no bucketing
     if (dec)
       hipLaunchKernelGGL(k_lowlat_mixed<true>, dim3((unsigned)n), dim3(256), 0, s, (int)n, c->alg_mask, reqs, ct,
                          (uint64_t)ct_bytes, key, (uint64_t)key_bytes, ss, (uint64_t)ss_bytes, coins,
@@ -1717,28 +1259,27 @@ int kyber_fused_mixed(pqc_ctx* c, int dec, size_t n, const pqc_kem_req* reqs, ui
     return hip_err(hipGetLastError());
   }
   const int cap = (int)c->max_batch;
-  hipLaunchKernelGGL(k_mixed_zero, dim3(1), dim3(64), 0, s, c->kmix_counts);
-  hipLaunchKernelGGL(k_mixed_classify, dim3((unsigned)((n + kClassifyBlock - 1) / kClassifyBlock)),
-                     dim3(kClassifyBlock), 0, s, (int)n, cap, dec,
-                     c->alg_mask, reqs,
-                     (uint64_t)ct_bytes, (uint64_t)key_bytes, (uint64_t)ss_bytes, (uint64_t)coins_bytes,
-                     c->kmix_order, c->kmix_counts, c->status);
-  const kyber::MixedSrc src{reqs, c->kmix_order, cap, ss, ct, key, coins, c->kprf, c->kprf_per_elem};
-  const int max_tiles = (int)((n + 31) / 32) + 2;  // half tiles at most; buckets round up separately
-  if (c->kat && (dec ? c->tune.fused_dec_tile : c->tune.fused_enc_tile) != 64) {
-    // 32-request tiles, two waves per SIMD, one A^T scratch region per wave
-    int grid = c->fused_grid_override > 0 ? c->fused_grid_override : c->cu_count * 2 * c->tune.fused_waves_per_cu;
-    grid = std::min(grid, max_tiles);
-    grid = std::min<long long>(grid, (long long)c->kat_waves);
-    if (grid < 1) return PQC_ERR_INVALID_ARG;
-    if (dec)
-      hipLaunchKernelGGL(k_fused_mixed_dec32, dim3(grid), dim3(64), 0, s, src, (const uint32_t*)c->kmix_counts,
-                         c->kat, c->kat_region, c->status);
-    else
-      hipLaunchKernelGGL(k_fused_mixed_enc32, dim3(grid), dim3(64), 0, s, src, (const uint32_t*)c->kmix_counts,
-                         c->kat, c->kat_region, c->status);
-    return hip_err(hipGetLastError());
+  auto classify = [&](const pqc_kem_req* r, size_t m) {
+    hipLaunchKernelGGL(k_mixed_zero, dim3(1), dim3(64), 0, s, c->kmix_counts);
+    hipLaunchKernelGGL(k_mixed_classify, dim3((unsigned)((m + kClassifyBlock - 1) / kClassifyBlock)),
+                       dim3(kClassifyBlock), 0, s, (int)m, cap, dec, c->alg_mask, r, (uint64_t)ct_bytes,
+                       (uint64_t)key_bytes, (uint64_t)ss_bytes, (uint64_t)coins_bytes, c->kmix_order, c->kmix_counts,
+                       c->status);
+  };
+  kyber::MixedSrc src{reqs, c->kmix_order, cap, ss, ct, key, coins, c->kprf, c->kprf_per_elem};
+  if ((dec ? c->tune.fused_dec_tile : c->tune.fused_enc_tile) != 64) {
+    // in stages, kstage_max requests at a time (their scratch)
+    for (size_t at = 0; at < n; at += c->kstage_max) {
+      const size_t m = std::min(n - at, c->kstage_max);
+      classify(reqs + at, m);
+      src.reqs = reqs + at;
+      const int rc = kyber_staged_mixed(c, dec, m, src, s);
+      if (rc) return rc;
+    }
+    return PQC_OK;
   }
+  classify(reqs, n);
+  const int max_tiles = (int)((n + 31) / 32) + 2;  // half tiles at most; buckets round up separately
   int grid = c->fused_grid_override > 0 ? c->fused_grid_override : c->cu_count * c->tune.fused_waves_per_cu;
   if (grid > max_tiles) grid = max_tiles;
   if (grid < 1) grid = 1;
@@ -1801,7 +1342,9 @@ template <int K>
 int noalloc_dec(const NoAllocDev& d, size_t n, uint8_t* ss, uint8_t* ct, const uint8_t* sk, uint32_t* status,
                 hipStream_t s) {
   using namespace kyber::fused;
-  if (n <= (size_t)kLowLatDefaultDec) {
+  // a workgroup per request up to where a 64-request tile launch (~1 ms for any batch)
+  // is faster: ~10.6 M decapsulations/s
+  if (n <= 8192) {
     hipLaunchKernelGGL((k_lowlat<K, true>), dim3((unsigned)n), dim3(256), 0, s, (int)n, ss, ct, sk,
                        (const uint8_t*)nullptr, status);
   } else {

@@ -53,4 +53,8 @@ struct MixedSrc {
 };
 
 }  // namespace kyber
+
+// a classified mixed batch in stages (kyber_staged.hip); n <= ctx->kstage_max
+int kyber_staged_mixed(pqc_ctx* c, int dec, size_t n, const kyber::MixedSrc& src, hipStream_t s);
+
 }  // namespace pqc

@@ -32,6 +32,7 @@
 // At 65536 the sponge stage takes ~370 us (53 permutations per request at 9.4 G/s, the
 // rate of the VALU on this mix), the product stages ~65 and ~140, the KDF ~15.
 #include <algorithm>
+#include <type_traits>
 
 #include "internal.h"
 #include "kyber_mfma.cuh"
@@ -740,9 +741,143 @@ __global__ __launch_bounds__(64, 4) void k_key_final(int n, KeySrc src) {
   for (int w = blockIdx.x; w < (n + 63) / 64; w += gridDim.x) key_final_wave<K>(src, n, w);
 }
 
+// ---- mixed kernels ------------------------------------------------------------------------------
+// The three buckets of k_mixed_classify, longest requests first.  Their sizes are known
+// on the device only, so a launch has workgroups for the worst case and those without
+// work leave.
+struct Buckets {
+  Bucket b2, b3, b4;
+};
+__device__ __forceinline__ Buckets buckets_of(const uint32_t* __restrict__ counts) {
+  const int n2 = (int)counts[0], n3 = (int)counts[1], n4 = (int)counts[2];
+  const int g4 = (n4 + 15) / 16, g3 = (n3 + 15) / 16;
+  return Buckets{Bucket{n2, g4 + g3}, Bucket{n3, g4}, Bucket{n4, 0}};
+}
+
+// item w of the sequence [c4 items of K = 4][c3 of K = 3][c2 of K = 2]: f(K, bucket, item)
+// for it; false when w is past them (then w is what is left)
+template <class F>
+__device__ __forceinline__ bool bucket_item(const Buckets& bs, int& w, int c4, int c3, int c2, F&& f) {
+  if (w < c4) {
+    f(std::integral_constant<int, 4>{}, bs.b4, w);
+    return true;
+  }
+  w -= c4;
+  if (w < c3) {
+    f(std::integral_constant<int, 3>{}, bs.b3, w);
+    return true;
+  }
+  w -= c3;
+  if (w < c2) {
+    f(std::integral_constant<int, 2>{}, bs.b2, w);
+    return true;
+  }
+  w -= c2;
+  return false;
+}
+
+template <class F>
+__device__ __forceinline__ bool bucket_tile(const Buckets& bs, int& w, F&& f) {
+  return bucket_item(bs, w, (bs.b4.n + 63) / 64, (bs.b3.n + 63) / 64, (bs.b2.n + 63) / 64, f);
+}
+
+template <bool DEC, class F>
+__device__ __forceinline__ void mixed_matrix(const Buckets& bs, const MixedSrc& src, const Scratch& sc, int w, F& sh) {
+  bucket_item(bs, w, matrix_waves<4>(bs.b4.n), matrix_waves<3>(bs.b3.n), matrix_waves<2>(bs.b2.n),
+              [&](auto k, const Bucket& b, int i) {
+                constexpr int K = decltype(k)::value;
+                using P = Params<K>;
+                matrix_wave<K, true>(sc, b, i, sh, [&](int r) {
+                  return src.template req<K, DEC>(r).key + (DEC ? P::sk_cpa_bytes : 0) + P::polyvec_bytes;
+                });
+              });
+}
+
+__global__ __launch_bounds__(kProdThreads, 2) void k_mixed_open(const uint32_t* counts, MixedSrc src, Scratch sc) {
+  __shared__ DftLds<true, true> sh;
+  load_tables<true, true, kProdThreads>(sh, &c_dft);
+  const Buckets bs = buckets_of(counts);
+  for (int t = blockIdx.x;; t += gridDim.x) {
+    int w = t;
+    if (!bucket_tile(bs, w, [&](auto k, const Bucket& b, int i) { open_tile<decltype(k)::value>(src, sc, b, i, sh); }))
+      break;
+  }
+}
+
+__global__ __launch_bounds__(64, 4) void k_mixed_dec_sponge(const uint32_t* counts, MixedSrc src, Scratch sc) {
+  __shared__ SponLds sh;
+  const Buckets bs = buckets_of(counts);
+  const int end = (bs.b4.n + 63) / 64 + (bs.b3.n + 63) / 64 + (bs.b2.n + 63) / 64;
+  const int total = 2 * end + matrix_waves<4>(bs.b4.n) + matrix_waves<3>(bs.b3.n) + matrix_waves<2>(bs.b2.n);
+  for (int t = blockIdx.x; t < total; t += gridDim.x) {
+    int w = t;
+    if (bucket_tile(bs, w, [&](auto k, const Bucket& b, int i) { dec_hash_wave<decltype(k)::value>(src, sc, b, i); }))
+      continue;
+    if (bucket_tile(bs, w, [&](auto k, const Bucket& b, int i) { dec_prf_wave<decltype(k)::value>(src, sc, b, i); }))
+      continue;
+    mixed_matrix<true>(bs, src, sc, w, sh);
+  }
+}
+
+template <bool DEC>
+__global__ __launch_bounds__(kProdThreads, 2) void k_mixed_encrypt(const uint32_t* counts, MixedSrc src, Scratch sc) {
+  __shared__ DftLds<true, true> sh;
+  load_tables<true, true, kProdThreads>(sh, &c_dft);
+  const Buckets bs = buckets_of(counts);
+  for (int t = blockIdx.x;; t += gridDim.x) {
+    int w = t;
+    if (!bucket_tile(bs, w, [&](auto k, const Bucket& b, int i) {
+          reencrypt_tile<decltype(k)::value, DEC>(src, sc, b, i, sh);
+        }))
+      break;
+  }
+}
+
+// KDF (DEC), or H(ct) and KDF
+template <bool DEC>
+__global__ __launch_bounds__(64, 4) void k_mixed_final(const uint32_t* counts, MixedSrc src, Scratch sc) {
+  const Buckets bs = buckets_of(counts);
+  for (int t = blockIdx.x;; t += gridDim.x) {
+    int w = t;
+    if (!bucket_tile(bs, w, [&](auto k, const Bucket& b, int i) {
+          if constexpr (DEC)
+            dec_kdf_wave<decltype(k)::value>(src, sc, b, i);
+          else
+            enc_final_wave<decltype(k)::value>(src, sc, b, i);
+        }))
+      break;
+  }
+}
+
+__global__ __launch_bounds__(64, 4) void k_mixed_enc_sponge(const uint32_t* counts, MixedSrc src, Scratch sc) {
+  __shared__ SponLds sh;
+  const Buckets bs = buckets_of(counts);
+  const int end = (bs.b4.n + 63) / 64 + (bs.b3.n + 63) / 64 + (bs.b2.n + 63) / 64;
+  const int total = end + matrix_waves<4>(bs.b4.n) + matrix_waves<3>(bs.b3.n) + matrix_waves<2>(bs.b2.n);
+  for (int t = blockIdx.x; t < total; t += gridDim.x) {
+    int w = t;
+    if (bucket_tile(bs, w, [&](auto k, const Bucket& b, int i) { enc_open_wave<decltype(k)::value>(src, sc, b, i); }))
+      continue;
+    mixed_matrix<false>(bs, src, sc, w, sh);
+  }
+}
+
+__global__ __launch_bounds__(64, 4) void k_mixed_prf(const uint32_t* counts, Scratch sc) {
+  const Buckets bs = buckets_of(counts);
+  for (int t = blockIdx.x;; t += gridDim.x) {
+    int w = t;
+    if (!bucket_item(bs, w, 9 * ((bs.b4.n + 63) / 64), 7 * ((bs.b3.n + 63) / 64), 5 * ((bs.b2.n + 63) / 64),
+                     [&](auto, const Bucket& b, int i) {
+                       const int wr = (b.n + 63) / 64;
+                       prf_wave(sc, b, i % wr, i / wr);
+                     }))
+      break;
+  }
+}
+
 // ---- launchers ---------------------------------------------------------------------------------
 static Scratch scratch_of(const pqc_ctx* c, int k) {
-  return Scratch{c->kprf, (size_t)(2 * k + 1) * 2048, reinterpret_cast<uint8_t*>(c->kat), (size_t)k * k * 16 * 512, c->krow, c->status};
+  return Scratch{c->kprf, (size_t)(2 * k + 1) * 2048, c->kat, (size_t)k * k * 16 * 512, c->krow, c->status};
 }
 
 // Product stages: persistent, two workgroups per CU (66 KB of tables each) at the default
@@ -817,6 +952,28 @@ static int keypair(pqc_ctx* c, size_t n_all, uint8_t* pk, uint8_t* sk, const uin
   return PQC_OK;
 }
 
+// A mixed batch of at most kstage_max requests, already classified
+static int mixed(pqc_ctx* c, int dec, size_t n, const MixedSrc& src, hipStream_t s) {
+  const int kmax = (int)(c->kprf_per_elem / 128 - 1) / 2;  // largest K the context holds
+  const Scratch sc = scratch_of(c, kmax);
+  const uint32_t* counts = c->kmix_counts;
+  const int tiles = (int)(n / 64) + 3;  // each bucket rounds up by itself
+  const int mat = ((int)((n + 15) / 16) + 3) * kmax * kmax / 4 + 3;
+  const dim3 prod(prod_grid(c, tiles)), prod_wg(kProdThreads), wg(64);
+  if (dec) {
+    hipLaunchKernelGGL(k_mixed_open, prod, prod_wg, 0, s, counts, src, sc);
+    hipLaunchKernelGGL(k_mixed_dec_sponge, dim3(sponge_grid(c, 2 * tiles + mat)), wg, 0, s, counts, src, sc);
+    hipLaunchKernelGGL(k_mixed_encrypt<true>, prod, prod_wg, 0, s, counts, src, sc);
+    hipLaunchKernelGGL(k_mixed_final<true>, dim3(sponge_grid(c, tiles)), wg, 0, s, counts, src, sc);
+  } else {
+    hipLaunchKernelGGL(k_mixed_enc_sponge, dim3(sponge_grid(c, tiles + mat)), wg, 0, s, counts, src, sc);
+    hipLaunchKernelGGL(k_mixed_prf, dim3(sponge_grid(c, tiles * (2 * kmax + 1))), wg, 0, s, counts, sc);
+    hipLaunchKernelGGL(k_mixed_encrypt<false>, prod, prod_wg, 0, s, counts, src, sc);
+    hipLaunchKernelGGL(k_mixed_final<false>, dim3(sponge_grid(c, tiles)), wg, 0, s, counts, src, sc);
+  }
+  return hip_err(hipGetLastError());
+}
+
 }  // namespace staged
 }  // namespace kyber
 
@@ -849,6 +1006,10 @@ int kyber_staged_keypair(pqc_ctx* c, int k, size_t n, uint8_t* pk, uint8_t* sk, 
     case 4: return kyber::staged::keypair<4>(c, n, pk, sk, coins, s);
     default: return PQC_ERR_UNSUPPORTED;
   }
+}
+
+int kyber_staged_mixed(pqc_ctx* c, int dec, size_t n, const kyber::MixedSrc& src, hipStream_t s) {
+  return kyber::staged::mixed(c, dec, n, src, s);
 }
 
 }  // namespace pqc

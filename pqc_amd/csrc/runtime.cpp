@@ -392,21 +392,17 @@ int pqc_ctx_create(pqc_ctx** out, unsigned alg_mask, size_t max_batch, size_t hb
     if (rc) goto fail;
     c->kbytes = (uint8_t*)p;
     c->kprf_per_elem = (size_t)(2 * kmax + 1) * 128;
-    rc = ctx_alloc(c, &p, c->kprf_per_elem * (c->ld + 64));
+    rc = ctx_alloc(c, &p, c->kprf_per_elem * (c->ld + 128));
     if (rc) goto fail;
     c->kprf = (uint8_t*)p;
-    // A^T scratch of the 32-request decapsulation tiles: one region per wave of the
-    // largest grid (two waves per SIMD) the batch size can use
-    c->kat_waves = std::min<size_t>((size_t)c->cu_count * 8, (max_batch + 31) / 32);
-    c->kat_region = pqc::tile32_scratch_bytes(kmax) / sizeof(int16_t);
-    // the staged path keeps whole batches of up to kstage_max requests there (groups of
-    // 16 of each parameter set: up to 64 rows of padding); larger ones run in passes
+    // scratch of the staged path for up to kstage_max requests (groups of 16 of each
+    // parameter set, read in tiles of 64: under 128 rows of padding); larger batches run
+    // in passes
     c->kstage_max = std::min<size_t>(c->ld, 65536);
-    rc = ctx_alloc(c, &p, std::max(pqc::tile32_scratch_bytes(kmax) * c->kat_waves,
-                                   pqc::kyber_stage_at_bytes(kmax) * (c->kstage_max + 64)));
+    rc = ctx_alloc(c, &p, pqc::kyber_stage_at_bytes(kmax) * (c->kstage_max + 128));
     if (rc) goto fail;
-    c->kat = (int16_t*)p;
-    rc = ctx_alloc(c, &p, (size_t)128 * (c->kstage_max + 64));
+    c->kat = (uint8_t*)p;
+    rc = ctx_alloc(c, &p, (size_t)128 * (c->kstage_max + 128));
     if (rc) goto fail;
     c->krow = (uint8_t*)p;
     rc = ctx_alloc(c, &p, (size_t)3 * c->ld * sizeof(uint32_t) + 256);

@@ -30,7 +30,7 @@ struct Samples {
 
 static float log2f_safe(double v) { return (float)std::log2(v > 1.0 ? v : 1.0); }
 
-// The mixed family's tile layouts: 32-request tiles for both operations (the
+// The mixed family's tile layouts: the stages for both operations (the
 // tile order does not apply), or 64-request tiles in tile order 0, 1 or 3.
 constexpr int kMixedOrders[3] = {0, 1, 3};
 static int mixed_layout(const pqc_tuning& t) {
@@ -114,7 +114,7 @@ static std::vector<pqc_tuning> candidates(const pqc_tune_request& r, const pqc_t
   return out;
 }
 
-// 0 and 32 both mean 32-request tiles
+// 0 and 32 both mean the staged throughput form
 static int tile_of(int v) { return v == 64 ? 64 : 32; }
 // 0 means the library's threshold
 static int lane_min_of(int v) { return v == 0 ? kFrodoLaneMinDefault : v; }
