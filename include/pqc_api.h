@@ -80,11 +80,10 @@ typedef struct pqc_tuning {
   int32_t mixed_order;        /* mixed-batch tile order: 0 = K 4,3,2; 1 = K 2,3,4; 2 = round-robin over K;
                                  3 = K 4,3,2 with 32-request tiles for K = 4 and K = 2 */
   int32_t frodo_stream_block; /* threads per workgroup of the Frodo noise-stream kernel: 64, 128 or 256 */
-  int32_t lowlat_max;         /* Kyber batches of at most this many requests run one four-wave
+  int32_t lowlat_max;         /* Kyber batches of at most this many requests run one
                                  workgroup per request (latency) instead of the throughput forms
-                                 below: 0 = library defaults (1024 decapsulations, 256
-                                 encapsulations, 512 in a mixed batch), -1 = never, else 1..65536
-                                 for all */
+                                 below: 0 = library default (1280), -1 = never, else 1..65536;
+                                 key generation with fused_key_tile = 64 never does */
   int32_t frodo_chunk;        /* FrodoKEM-976 batches under one key above this many requests are cut
                                  into chunks of this many, run on four streams: 0 = library default
                                  (no split up to 65536), else a multiple of 32 in 32..65536 */

@@ -112,6 +112,17 @@ int kyber_fused_enc(pqc_ctx* c, int k, size_t n, uint8_t* ct, uint8_t* ss, const
 int kyber_fused_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct, const uint8_t* sk,
                     hipStream_t s);
 
+// one workgroup per request (kyber_lowlat.hip): small batches
+int kyber_lowlat_keypair(int k, size_t n, uint8_t* pk, uint8_t* sk, const uint8_t* coins, uint32_t* status,
+                         hipStream_t s);
+int kyber_lowlat_enc(int k, size_t n, uint8_t* ct, uint8_t* ss, const uint8_t* pk, const uint8_t* coins,
+                     uint32_t* status, hipStream_t s);
+int kyber_lowlat_dec(int k, size_t n, uint8_t* ss, const uint8_t* ct, const uint8_t* sk, uint32_t* status,
+                     hipStream_t s);
+int kyber_lowlat_mixed(const pqc_ctx* c, int dec, size_t n, const pqc_kem_req* reqs, uint8_t* ct, size_t ct_bytes,
+                       const uint8_t* key, size_t key_bytes, uint8_t* ss, size_t ss_bytes, const uint8_t* coins,
+                       size_t coins_bytes, hipStream_t s);
+
 // the same in stages (kyber_staged.hip): throughput path of larger batches
 size_t kyber_stage_at_bytes(int k);  // sampled matrix entries of one request
 int kyber_staged_keypair(pqc_ctx* c, int k, size_t n, uint8_t* pk, uint8_t* sk, const uint8_t* coins, hipStream_t s);

@@ -25,6 +25,7 @@
 
 #include "internal.h"
 #include "req_check.h"
+#include "kyber_coop.cuh"
 #include "kyber_src.cuh"
 #include "kyber_wave.cuh"
 #include "kyber_wavef.cuh"
@@ -62,79 +63,6 @@ struct Lds {
   uint32_t fail[64];
 };
 
-// ---- wave-cooperative pieces -------------------------------------------------
-
-// indcpa_dec inputs of one request, as this lane's words: the ciphertext's u and v
-// groups and the secret key's 12-bit groups.
-template <int K>
-struct DecIn {
-  uint32_t u[K][3], s[K][2], v[3];
-};
-
-template <int K>
-__device__ __forceinline__ void dec_load(DecIn<K>& in, const uint8_t* ct, const uint8_t* sk) {
-  using P = Params<K>;
-  const int l = lane_id();
-#pragma unroll
-  for (int i = 0; i < K; ++i) {
-    load_group<P::du>(in.u[i], ct + 32 * P::du * i, nat_group(l));
-    load_h12(in.s[i], sk + 384 * i, ntt_group(l));
-  }
-  load_group<P::dv>(in.v, ct + P::polyvec_cbytes, nat_group(l));
-}
-
-// Pack the lane's 4 D-bit values with its odd neighbour's: even lanes write D bytes.
-template <int D>
-__device__ __forceinline__ void pack_pair(uint8_t* dst, const uint32_t (&t)[4]) {
-  const int l = lane_id();
-  uint64_t mine = 0;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) mine |= (uint64_t)t[r] << (D * r);
-  const uint64_t nb = (uint64_t)__shfl_xor((long long)mine, 1);
-  if ((l & 1) == 0) {
-    // 8 values, 8*D bits: low 4*D bits mine, next 4*D bits the neighbour's
-    const uint64_t lo = mine | (nb << (4 * D));
-    const uint64_t hi = (4 * D + 4 * D > 64) ? (nb >> (64 - 4 * D)) : 0;
-    uint8_t* o = dst + D * (l >> 1);
-#pragma unroll
-    for (int b = 0; b < D; ++b) o[b] = (uint8_t)(b < 8 ? (lo >> (8 * b)) : (hi >> (8 * (b - 8))));
-  }
-}
-
-// Re-encryption inputs of one request, as this lane's words: its 16-bit PRF
-// groups (2K+1 noise polynomials), the public key's 12-bit groups and, for
-// decapsulation, the ciphertext's u and v groups to compare with.
-template <int K, bool DEC>
-struct EncIn {
-  uint32_t prf[2 * K + 1];
-  uint32_t t[K][2];
-  uint32_t cu[DEC ? K : 1][3], cv[3];
-};
-
-// PRF_LDS: the PRF rows are in LDS (the per-request kernels); otherwise in the
-// global scratch, read through a global-address-space pointer.
-template <int K, bool DEC, bool PRF_LDS = false>
-__device__ __forceinline__ void enc_load(EncIn<K, DEC>& in, const uint8_t* prf, const uint8_t* pk, const uint8_t* ct) {
-  using P = Params<K>;
-  const int l = lane_id();
-  if constexpr (PRF_LDS) {
-    const uint16_t* prf16 = reinterpret_cast<const uint16_t*>(prf);
-#pragma unroll
-    for (int j = 0; j < 2 * K + 1; ++j) in.prf[j] = prf16[64 * j + l];
-  } else {
-    const global_t<uint16_t>* prf16 = gptr(reinterpret_cast<const uint16_t*>(prf));
-#pragma unroll
-    for (int j = 0; j < 2 * K + 1; ++j) in.prf[j] = prf16[64 * j + l];
-  }
-#pragma unroll
-  for (int j = 0; j < K; ++j) load_h12(in.t[j], pk + 384 * j, ntt_group(l));
-  if constexpr (DEC) {
-#pragma unroll
-    for (int i = 0; i < K; ++i) load_group<P::du>(in.cu[i], ct + 32 * P::du * i, nat_group(l));
-    load_group<P::dv>(in.cv, ct + P::polyvec_cbytes, nat_group(l));
-  }
-}
-
 // Sources of the A^T entries for the re-encryption: at.get(i, j, w0, w1) gives
 // this lane's group of entry (i, j) as two words of two coefficients.
 template <int K>
@@ -148,128 +76,6 @@ struct AtRing {  // the LDS ring of the 64-request tiles: entry e0 + i K + j in 
     w1 = e32[1];
   }
 };
-
-// ---- indcpa_dec and the re-encryption on exact FP32 values (kyber_wavef.cuh) -----
-// Every polynomial value equals the reference's int16 value mod q (the
-// reference's arithmetic never leaves the int16 range, so its values are exact
-// residues too), and the outputs leave through compress_f, which reads only the
-// residue: the message bits, the ciphertext and the mismatch bits are the
-// reference's.
-
-// indcpa_dec (indcpa.cu:691-733, poly_tomsg) for one request; the message is written to
-// msg (LDS, 32 bytes).
-template <int K>
-__device__ __forceinline__ void coop_indcpa_dec_f(const DecIn<K>& in, const LaneZF& z, uint8_t* msg) {
-  using P = Params<K>;
-  const int l = lane_id();
-  F4 u[K];
-  Bz uz[K];
-#pragma unroll
-  for (int i = 0; i < K; ++i) {
-    uint32_t t[4];
-    unpack_loaded<P::du>(t, in.u[i], nat_group(l));
-#pragma unroll
-    for (int r = 0; r < 4; ++r) u[i].v[r] = (float)decompress_d<P::du>(t[r]);  // [0, q)
-    ntt_f<Q>(u[i], z);
-    reduce_f4(u[i]);
-    uz[i] = basemul_twist(u[i], z);
-  }
-  F4 mp = basemul_sum_f<K>(
-      [&](int i) {
-        P4 s;
-        poly12_loaded(s, in.s[i], ntt_group(l));  // 12-bit, unreduced
-        F4 sf = to_f4(s);
-        reduce_f4(sf);
-        return sf;
-      },
-      u, uz);
-  invntt_f(mp, z);
-  uint32_t tv[4];
-  unpack_loaded<P::dv>(tv, in.v, nat_group(l));
-  uint32_t nib = 0;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) nib |= f32::compress_f<1>((float)decompress_d<P::dv>(tv[r]) - mp.v[r]) << r;
-  const uint32_t other = (uint32_t)__shfl_xor((int)nib, 1);
-  if ((l & 1) == 0) msg[l >> 1] = (uint8_t)(nib | (other << 4));
-}
-
-// Re-encryption of one request (indcpa_enc from sp-sampling on).  DEC: compare
-// with ct and return the lane's mismatch bits.  ENC: write ct.
-template <int K, bool DEC, class AT>
-__device__ __forceinline__ uint32_t coop_reencrypt_f(const AT& at, const EncIn<K, DEC>& in, const uint8_t* msg,
-                                                     uint8_t* ct, const LaneZF& z) {
-  using P = Params<K>;
-  const int l = lane_id();
-  const int gn = ntt_group(l);
-  F4 sp[K];
-  Bz spz[K];
-#pragma unroll
-  for (int j = 0; j < K; ++j) {
-    P4 c;
-    cbd_group(c, in.prf[j]);  // [-2, 2]
-    sp[j] = to_f4(c);
-    ntt_f<2>(sp[j], z);
-    reduce_f4(sp[j]);
-    spz[j] = basemul_twist(sp[j], z);
-  }
-  uint32_t mismatch = 0;
-#pragma unroll
-  for (int i = 0; i < K; ++i) {
-    F4 acc = basemul_sum_f<K>(
-        [&](int j) {
-          uint32_t w0, w1;
-          at.get(i, j, w0, w1);  // accepted candidates, [0, 19q)
-          F4 a = {{(float)(w0 & 0xFFFF), (float)(w0 >> 16), (float)(w1 & 0xFFFF), (float)(w1 >> 16)}};
-          reduce_f4(a);
-          return a;
-        },
-        sp, spz);
-    invntt_f(acc, z);
-    P4 e;
-    cbd_group(e, in.prf[K + i]);
-    uint32_t c[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) c[r] = f32::compress_f<P::du>(acc.v[r] + (float)e.v[r]);
-    if constexpr (DEC) {
-      uint32_t t[4];
-      unpack_loaded<P::du>(t, in.cu[i], nat_group(l));
-#pragma unroll
-      for (int r = 0; r < 4; ++r) mismatch |= c[r] ^ t[r];
-    } else {
-      pack_pair<P::du>(ct + 32 * P::du * i, c);
-    }
-  }
-  {
-    F4 acc = basemul_sum_f<K>(
-        [&](int j) {
-          P4 t;
-          poly12_loaded(t, in.t[j], gn);
-          F4 tf = to_f4(t);
-          reduce_f4(tf);
-          return tf;
-        },
-        sp, spz);
-    invntt_f(acc, z);
-    P4 e;
-    cbd_group(e, in.prf[2 * K]);
-    const uint32_t nib = (msg[l >> 1] >> (4 * (l & 1))) & 0xF;
-    uint32_t c[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float kq = ((nib >> r) & 1) ? (float)((Q + 1) / 2) : 0.f;
-      c[r] = f32::compress_f<P::dv>(acc.v[r] + (float)e.v[r] + kq);
-    }
-    if constexpr (DEC) {
-      uint32_t t[4];
-      unpack_loaded<P::dv>(t, in.cv, nat_group(l));
-#pragma unroll
-      for (int r = 0; r < 4; ++r) mismatch |= c[r] ^ t[r];
-    } else {
-      pack_pair<P::dv>(ct + P::polyvec_cbytes, c);
-    }
-  }
-  return mismatch;
-}
 
 // ---- per-lane sponge pieces ---------------------------------------------------
 
@@ -499,15 +305,6 @@ __device__ __forceinline__ void fused_tile(const Src& src, int base, int n, Lds<
 // coefficient after csubq (polyvec_tobytes).  A is not transposed:
 // A[i][j] = SHAKE128(rho || j || i) (gen_matrix_n with transposed = 0).
 
-// 12-bit pack of a group in its NTT-order slot (the inverse of load_poly12)
-__device__ __forceinline__ void store_poly12(uint8_t* base, int g, const P4& p) {
-  uint16_t* h = reinterpret_cast<uint16_t*>(base + 6 * g);
-  const uint32_t c0 = (uint32_t)p.v[0], c1 = (uint32_t)p.v[1], c2 = (uint32_t)p.v[2], c3 = (uint32_t)p.v[3];
-  h[0] = (uint16_t)(c0 | (c1 << 12));
-  h[1] = (uint16_t)((c1 >> 4) | (c2 << 8));
-  h[2] = (uint16_t)((c2 >> 8) | (c3 << 4));
-}
-
 template <int K>
 struct KeyIn {
   uint32_t prf[2 * K];
@@ -670,278 +467,6 @@ __global__ __launch_bounds__(64) void k_fused(int n, int ntiles, DenseSrc src, u
   LaneZF z;
   load_lane_zf(z, &c_lane_twf);
   for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) fused_tile<K, DEC>(src, tile * 64, n, sh, z, status);
-}
-
-// ---- low latency: one workgroup of four waves per request -------------------------
-// A tile's latency is one lane's serial sponge chain (H(ct), G, the 2K + 1 PRF
-// outputs, the A^T entries, KDF) plus the wave's cooperative work for all its
-// requests in turn, about 1 ms for a full tile whatever the batch size.  For
-// small batches (the single-instance drop-ins, a serving loop's batches) these
-// kernels spread one request over four waves and many lanes.  Decapsulation:
-//   phase 1  wave 0: indcpa_dec (wave-cooperative), then G and the 2K + 1 PRF
-//                    outputs on 2K + 1 lanes at once;
-//            wave 1: the K^2 A^T entries on K^2 lanes at once;
-//            wave 2: the first blocks of H(ct) on a lane pair (keccakf1600_pair,
-//                    about 2/3 of the single-lane latency per block);
-//   phase 2  wave 0: re-encryption and compare; wave 2: the rest of H(ct), its
-//                    sponge state kept in registers across the barrier;
-//   phase 3  one lane: KDF.
-// Encapsulation: see lowlat_enc_body.  Results are byte-identical to the tile
-// kernel's.
-
-template <int K>
-struct alignas(16) LowLds {
-  uint8_t prf[(2 * K + 1) * 128];                 // PRF(coins, nonce) at 128 nonce
-  alignas(16) uint8_t msg[32];
-  uint32_t kbar[8], hct[8], hpk[8];               // 32-byte values as words
-  uint32_t fail;
-  alignas(16) uint8_t ct[Params<K>::ct_bytes];    // encapsulation: the ciphertext before it is stored
-  alignas(16) int16_t a[K * K * kAStride];        // A^T entry i K + j in slot i K + j
-};
-
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
-// K^2 A^T entries of one request on lanes 0 .. K^2 - 1 of the calling wave
-template <int K>
-__device__ __forceinline__ void lowlat_sample(LowLds<K>& sh, const uint8_t* pk, int l, uint32_t* status) {
-  using P = Params<K>;
-  if (l < K * K) {
-    // entry ij = i K + j on lane ij: A^T[i][j] = SHAKE128(rho || i || j)
-    uint64_t rho[4];
-#pragma unroll
-    for (int w = 0; w < 4; ++w) rho[w] = load_u64(pk + P::polyvec_bytes + 8 * w);
-    const int got = sample_entry(sh.a + l * kAStride, rho, l / K, l % K, true);
-    if (got < N) atomicOr(status, 1u);
-  }
-}
-
-// (Kbar, coins) = G(msg || h) on lanes 0 .. 2K; lane j then writes PRF(coins, j)
-// to sh.prf and lane 0 Kbar to sh.kbar.  Every lane recomputes G (same inputs)
-// instead of waiting for a broadcast.
-template <int K>
-__device__ __forceinline__ void lowlat_g_prf(LowLds<K>& sh, const uint64_t (&h)[4], int l) {
-  if (l < 2 * K + 1) {
-    uint64_t m[8], A[25], rc4[4];
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      m[w] = load_u64(sh.msg + 8 * w);
-      m[4 + w] = h[w];
-    }
-    absorb_fixed<kRateSha3_512, 8>(A, m, 0x06);
-#pragma unroll
-    for (int w = 0; w < 4; ++w) rc4[w] = A[4 + w];
-    if (l == 0) {
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        sh.kbar[2 * w] = (uint32_t)A[w];
-        sh.kbar[2 * w + 1] = (uint32_t)(A[w] >> 32);
-      }
-    }
-    absorb_fixed<kRateShake256, 4>(A, rc4, (uint64_t)l | (0x1Full << 8));
-#pragma unroll
-    for (int w = 0; w < 16; ++w) store_u64(sh.prf + 128 * l + 8 * w, A[w]);
-  }
-}
-
-// KDF(key || H(c)) -> ss on the calling lane
-__device__ __forceinline__ void lowlat_kdf(uint8_t* ss, const uint32_t (&kb)[8], const uint32_t (&hc)[8]) {
-  uint64_t m[8], A[25];
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    m[w] = (uint64_t)kb[2 * w] | ((uint64_t)kb[2 * w + 1] << 32);
-    m[4 + w] = (uint64_t)hc[2 * w] | ((uint64_t)hc[2 * w + 1] << 32);
-  }
-  absorb_fixed<kRateShake256, 8>(A, m, 0x1F);
-#pragma unroll
-  for (int w = 0; w < 4; ++w) store_u64(ss + 8 * w, A[w]);
-}
-
-// One decapsulation by the four waves of the workgroup (wave = threadIdx.x / 64)
-template <int K>
-__device__ __forceinline__ void lowlat_dec_body(uint8_t* ss, const uint8_t* c, const uint8_t* key, LowLds<K>& sh,
-                                                const LaneZF& z, int wave, int l, uint32_t* status) {
-  using P = Params<K>;
-  constexpr int HW = P::ct_bytes / 8;         // H(ct) message words
-  constexpr int HB = HW / kRateSha3_256 + 1;  // H(ct) blocks, padding included
-  constexpr int HB1 = (2 * HB + 2) / 3;       // of them absorbed during phase 1
-  const uint8_t* pk = key + P::sk_cpa_bytes;
-  uint32_t S[25];  // wave 2's H(ct) state, held across the first barrier
-  // ---- phase 1
-  if (wave == 0) {
-    {
-      DecIn<K> in;
-      dec_load<K>(in, c, key);
-      coop_indcpa_dec_f<K>(in, z, sh.msg);
-    }
-    wave_sync();
-    uint64_t h[4];
-#pragma unroll
-    for (int w = 0; w < 4; ++w) h[w] = load_u64(key + P::hpk_off + 8 * w);
-    lowlat_g_prf<K>(sh, h, l);
-  } else if (wave == 1) {
-    lowlat_sample<K>(sh, pk, l, status);
-  } else if (wave == 2 && l < 2) {
-    absorb_range_pair(S, c, HW, 0, HB1, 0x06, (uint32_t)l);
-  }
-  __syncthreads();
-  // ---- phase 2
-  if (wave == 0) {
-    EncIn<K, true> in;
-    enc_load<K, true, true>(in, sh.prf, pk, c);
-    const uint32_t mm = coop_reencrypt_f<K, true>(AtRing<K>{sh.a, 0}, in, sh.msg, nullptr, z);
-    const uint32_t f = __any(mm != 0) ? 1u : 0u;
-    if (l == 0) sh.fail = f;
-  } else if (wave == 2 && l < 2) {
-    absorb_range_pair(S, c, HW, HB1, HB, 0x06, (uint32_t)l);
-#pragma unroll
-    for (int w = 0; w < 4; ++w) sh.hct[2 * w + l] = S[w];
-  }
-  __syncthreads();
-  // ---- phase 3: KDF(Kbar or z, H(ct)), z chosen by mask
-  if (wave == 0 && l == 0) {
-    const uint32_t mask = 0u - (sh.fail & 1u);
-    uint32_t kb[8], hc[8];
-#pragma unroll
-    for (int w = 0; w < 8; ++w) {
-      const uint32_t zz = reinterpret_cast<const uint32_t*>(key + P::z_off)[w];
-      kb[w] = sh.kbar[w] ^ (mask & (zz ^ sh.kbar[w]));
-      hc[w] = sh.hct[w];
-    }
-    lowlat_kdf(ss, kb, hc);
-  }
-}
-
-// One encapsulation by the four waves of the workgroup
-//   phase 1  wave 0: m = H(coins); wave 1: A^T; wave 2: H(pk) on a lane pair
-//   phase 2  wave 0: G and the PRF outputs, then the encryption into LDS
-//   phase 3  wave 0: ct to memory; wave 2: H(ct) on a lane pair
-//   phase 4  one lane: KDF(Kbar || H(ct))
-template <int K>
-__device__ __forceinline__ void lowlat_enc_body(uint8_t* ss, uint8_t* c, const uint8_t* pk, const uint8_t* coins,
-                                                LowLds<K>& sh, const LaneZF& z, int wave, int l, uint32_t* status) {
-  using P = Params<K>;
-  // ---- phase 1
-  if (wave == 0 && l == 0) {
-    uint64_t A[25], c4[4];
-#pragma unroll
-    for (int w = 0; w < 4; ++w) c4[w] = load_u64(coins + 8 * w);
-    absorb_fixed<kRateSha3_256, 4>(A, c4, 0x06);  // "don't release system RNG output"
-#pragma unroll
-    for (int w = 0; w < 4; ++w) store_u64(sh.msg + 8 * w, A[w]);
-  } else if (wave == 1) {
-    lowlat_sample<K>(sh, pk, l, status);
-  } else if (wave == 2 && l < 2) {
-    uint32_t S[25];
-    constexpr int W = P::pk_bytes / 8;
-    absorb_range_pair(S, pk, W, 0, W / kRateSha3_256 + 1, 0x06, (uint32_t)l);
-#pragma unroll
-    for (int w = 0; w < 4; ++w) sh.hpk[2 * w + l] = S[w];
-  }
-  __syncthreads();
-  // ---- phase 2
-  if (wave == 0) {
-    uint64_t h[4];
-#pragma unroll
-    for (int w = 0; w < 4; ++w) h[w] = (uint64_t)sh.hpk[2 * w] | ((uint64_t)sh.hpk[2 * w + 1] << 32);
-    lowlat_g_prf<K>(sh, h, l);
-    wave_sync();
-    EncIn<K, false> in;
-    enc_load<K, false, true>(in, sh.prf, pk, nullptr);
-    (void)coop_reencrypt_f<K, false>(AtRing<K>{sh.a, 0}, in, sh.msg, sh.ct, z);
-  }
-  __syncthreads();
-  // ---- phase 3
-  if (wave == 0) {
-    for (int w = l; w < P::ct_bytes / 8; w += 64) store_u64(c + 8 * w, load_u64(sh.ct + 8 * w));
-  } else if (wave == 2 && l < 2) {
-    uint32_t S[25];
-    constexpr int W = P::ct_bytes / 8;
-    absorb_range_pair(S, sh.ct, W, 0, W / kRateSha3_256 + 1, 0x06, (uint32_t)l);
-#pragma unroll
-    for (int w = 0; w < 4; ++w) sh.hct[2 * w + l] = S[w];
-  }
-  __syncthreads();
-  // ---- phase 4
-  if (wave == 0 && l == 0) {
-    uint32_t kb[8], hc[8];
-#pragma unroll
-    for (int w = 0; w < 8; ++w) {
-      kb[w] = sh.kbar[w];
-      hc[w] = sh.hct[w];
-    }
-    lowlat_kdf(ss, kb, hc);
-  }
-}
-
-// Dense batches: request x at x * size in each buffer
-template <int K, bool DEC>
-__global__ __launch_bounds__(256) void k_lowlat(int n, uint8_t* __restrict__ ss, uint8_t* __restrict__ ct,
-                                                const uint8_t* __restrict__ key, const uint8_t* __restrict__ coins,
-                                                uint32_t* __restrict__ status) {
-  using P = Params<K>;
-  __shared__ LowLds<K> sh;
-  const int x = blockIdx.x;
-  if (x >= n) return;  // whole workgroup
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int l = threadIdx.x & 63;
-  LaneZF z;
-  load_lane_zf(z, &c_lane_twf);
-  if constexpr (DEC)
-    lowlat_dec_body<K>(ss + (size_t)x * 32, ct + (size_t)x * P::ct_bytes, key + (size_t)x * P::sk_bytes, sh, z, wave,
-                       l, status);
-  else
-    lowlat_enc_body<K>(ss + (size_t)x * 32, ct + (size_t)x * P::ct_bytes, key + (size_t)x * P::pk_bytes,
-                       coins + (size_t)x * 32, sh, z, wave, l, status);
-}
-
-// Mixed batches: one descriptor per workgroup, checked as k_mixed_classify
-// checks it (a rejected one sets status bit 1 and is skipped)
-union LowLdsMixed {
-  LowLds<2> k2;
-  LowLds<3> k3;
-  LowLds<4> k4;
-};
-
-template <bool DEC>
-__global__ __launch_bounds__(256) void k_lowlat_mixed(int n, unsigned alg_mask, const pqc_kem_req* __restrict__ reqs,
-                                                      uint8_t* ct, uint64_t ct_bytes, const uint8_t* key,
-                                                      uint64_t key_bytes, uint8_t* ss, uint64_t ss_bytes,
-                                                      const uint8_t* coins, uint64_t coins_bytes,
-                                                      uint32_t* __restrict__ status) {
-  __shared__ LowLdsMixed sh;
-  const int x = blockIdx.x;
-  if (x >= n) return;
-  const pqc_kem_req d = reqs[x];
-  const int k = pqc_req_k(d, DEC, alg_mask, ct_bytes, key_bytes, ss_bytes, coins_bytes);
-  if (!k) {  // uniform: every lane read the same descriptor
-    if (threadIdx.x == 0) atomicOr(status, 2u);
-    return;
-  }
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int l = threadIdx.x & 63;
-  LaneZF z;
-  load_lane_zf(z, &c_lane_twf);
-  uint8_t* s_ = ss + d.ss_off;
-  uint8_t* c_ = ct + d.ct_off;
-  const uint8_t* k_ = key + d.key_off;
-  const uint8_t* r_ = DEC ? nullptr : coins + d.coins_off;
-  switch (k) {
-    case 2:
-      if constexpr (DEC) lowlat_dec_body<2>(s_, c_, k_, sh.k2, z, wave, l, status);
-      else lowlat_enc_body<2>(s_, c_, k_, r_, sh.k2, z, wave, l, status);
-      break;
-    case 3:
-      if constexpr (DEC) lowlat_dec_body<3>(s_, c_, k_, sh.k3, z, wave, l, status);
-      else lowlat_enc_body<3>(s_, c_, k_, r_, sh.k3, z, wave, l, status);
-      break;
-    default:
-      if constexpr (DEC) lowlat_dec_body<4>(s_, c_, k_, sh.k4, z, wave, l, status);
-      else lowlat_enc_body<4>(s_, c_, k_, r_, sh.k4, z, wave, l, status);
-      break;
-  }
 }
 
 // ---- mixed parameter sets ------------------------------------------------------
@@ -1153,24 +678,17 @@ static int launch_fused(pqc_ctx* c, size_t n, uint8_t* ss, uint8_t* ct, const ui
   return hip_err(hipGetLastError());
 }
 
-// Kyber batches of at most this many requests take the one-workgroup-per-request
-// kernels, larger ones the stages (kyber_staged.hip).  Measured on MI355X (Kyber-768),
-// per-request against staged: 123 / 158 us for 761 decapsulations, 145 / 160 for 1024,
-// 219 / 163 for 2048; 233 / 238 us for 64 encapsulations, 257 / 239 for 300.  Mixed
-// 1:2:1, encapsulation + decapsulation: 441 / 542 us at 300, 529 / 541 at 1000, 1123 /
-// 574 at 3000.  tuning.lowlat_max overrides them all (-1 = never).
-constexpr int kLowLatDec = 1024, kLowLatEnc = 256, kLowLatMixedEnc = 512;
+// Kyber batches of at most this many requests take the one-workgroup-per-request kernels
+// (kyber_lowlat.hip), larger ones the stages (kyber_staged.hip).  Measured on MI355X,
+// per-request against staged, us: Kyber-768 decapsulation 92 / 155 at 1000, 149 / 159 at
+// 1500, 186 / 160 at 2000; encapsulation 124 / 238 at 1000, 264 / 245 at 2000; key
+// generation 89 / 164 at 1000, 181 / 169 at 2000; Kyber-1024 decapsulation 124 / 193 at
+// 1000, 196 / 200 at 1500.  tuning.lowlat_max overrides them all (-1 = never).
+constexpr int kLowLatDec = 1280, kLowLatEnc = 1280, kLowLatKey = 1280;
 
 inline bool use_lowlat(const pqc_ctx* c, size_t n, int dflt) {
   const int lim = c->tune.lowlat_max != 0 ? c->tune.lowlat_max : dflt;
   return n > 0 && (long long)n <= (long long)lim;
-}
-
-template <int K, bool DEC>
-static int launch_lowlat(pqc_ctx* c, size_t n, uint8_t* ss, uint8_t* ct, const uint8_t* key, const uint8_t* coins,
-                         hipStream_t s) {
-  hipLaunchKernelGGL((k_lowlat<K, DEC>), dim3((unsigned)n), dim3(256), 0, s, (int)n, ss, ct, key, coins, c->status);
-  return hip_err(hipGetLastError());
 }
 
 template <int K>
@@ -1189,7 +707,9 @@ static int launch_fused_keypair(pqc_ctx* c, size_t n, uint8_t* pk, uint8_t* sk, 
 }  // namespace kyber
 
 int kyber_fused_keypair(pqc_ctx* c, int k, size_t n, uint8_t* pk, uint8_t* sk, const uint8_t* coins, hipStream_t s) {
-  if (n > 0 && c->tune.fused_key_tile != 64 && c->kat) return kyber_staged_keypair(c, k, n, pk, sk, coins, s);
+  if (c->tune.fused_key_tile != 64 && kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatKey))
+    return kyber_lowlat_keypair(k, n, pk, sk, coins, c->status, s);
+  if (n > 0 && c->tune.fused_key_tile != 64) return kyber_staged_keypair(c, k, n, pk, sk, coins, s);
   switch (k) {
     case 2: return kyber::fused::launch_fused_keypair<2>(c, n, pk, sk, coins, s);
     case 3: return kyber::fused::launch_fused_keypair<3>(c, n, pk, sk, coins, s);
@@ -1200,16 +720,8 @@ int kyber_fused_keypair(pqc_ctx* c, int k, size_t n, uint8_t* pk, uint8_t* sk, c
 
 int kyber_fused_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct, const uint8_t* sk, hipStream_t s) {
   uint8_t* ctm = const_cast<uint8_t*>(ct);  // read-only in the decaps instantiation
-  if (n > 0 && !kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDec) && c->tune.fused_dec_tile != 64 && c->kat)
-    return kyber_staged_dec(c, k, n, ss, ct, sk, s);
-  if (kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDec)) {
-    switch (k) {
-      case 2: return kyber::fused::launch_lowlat<2, true>(c, n, ss, ctm, sk, nullptr, s);
-      case 3: return kyber::fused::launch_lowlat<3, true>(c, n, ss, ctm, sk, nullptr, s);
-      case 4: return kyber::fused::launch_lowlat<4, true>(c, n, ss, ctm, sk, nullptr, s);
-      default: return PQC_ERR_UNSUPPORTED;
-    }
-  }
+  if (kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDec)) return kyber_lowlat_dec(k, n, ss, ct, sk, c->status, s);
+  if (n > 0 && c->tune.fused_dec_tile != 64) return kyber_staged_dec(c, k, n, ss, ct, sk, s);
   switch (k) {
     case 2: return kyber::fused::launch_fused<2, true>(c, n, ss, ctm, sk, nullptr, s);
     case 3: return kyber::fused::launch_fused<3, true>(c, n, ss, ctm, sk, nullptr, s);
@@ -1220,16 +732,9 @@ int kyber_fused_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct,
 
 int kyber_fused_enc(pqc_ctx* c, int k, size_t n, uint8_t* ct, uint8_t* ss, const uint8_t* pk, const uint8_t* coins,
                     hipStream_t s) {
-  if (n > 0 && !kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatEnc) && c->tune.fused_enc_tile != 64 && c->kat)
-    return kyber_staged_enc(c, k, n, ct, ss, pk, coins, s);
-  if (kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatEnc)) {
-    switch (k) {
-      case 2: return kyber::fused::launch_lowlat<2, false>(c, n, ss, ct, pk, coins, s);
-      case 3: return kyber::fused::launch_lowlat<3, false>(c, n, ss, ct, pk, coins, s);
-      case 4: return kyber::fused::launch_lowlat<4, false>(c, n, ss, ct, pk, coins, s);
-      default: return PQC_ERR_UNSUPPORTED;
-    }
-  }
+  if (kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatEnc))
+    return kyber_lowlat_enc(k, n, ct, ss, pk, coins, c->status, s);
+  if (n > 0 && c->tune.fused_enc_tile != 64) return kyber_staged_enc(c, k, n, ct, ss, pk, coins, s);
   switch (k) {
     case 2: return kyber::fused::launch_fused<2, false>(c, n, ss, ct, pk, coins, s);
     case 3: return kyber::fused::launch_fused<3, false>(c, n, ss, ct, pk, coins, s);
@@ -1247,17 +752,8 @@ int kyber_fused_mixed(pqc_ctx* c, int dec, size_t n, const pqc_kem_req* reqs, ui
   using namespace kyber::fused;
   if (n == 0) return PQC_OK;
   if (!c->kmix_order || !c->kprf) return PQC_ERR_UNSUPPORTED;
-  if (use_lowlat(c, n, dec ? kLowLatDec : kLowLatMixedEnc)) {  // one workgroup per descriptor, no bucketing
-    if (dec)
-      hipLaunchKernelGGL(k_lowlat_mixed<true>, dim3((unsigned)n), dim3(256), 0, s, (int)n, c->alg_mask, reqs, ct,
-                         (uint64_t)ct_bytes, key, (uint64_t)key_bytes, ss, (uint64_t)ss_bytes, coins,
-                         (uint64_t)coins_bytes, c->status);
-    else
-      hipLaunchKernelGGL(k_lowlat_mixed<false>, dim3((unsigned)n), dim3(256), 0, s, (int)n, c->alg_mask, reqs, ct,
-                         (uint64_t)ct_bytes, key, (uint64_t)key_bytes, ss, (uint64_t)ss_bytes, coins,
-                         (uint64_t)coins_bytes, c->status);
-    return hip_err(hipGetLastError());
-  }
+  if (use_lowlat(c, n, dec ? kLowLatDec : kLowLatEnc))  // one workgroup per descriptor, no bucketing
+    return kyber_lowlat_mixed(c, dec, n, reqs, ct, ct_bytes, key, key_bytes, ss, ss_bytes, coins, coins_bytes, s);
   const int cap = (int)c->max_batch;
   auto classify = [&](const pqc_kem_req* r, size_t m) {
     hipLaunchKernelGGL(k_mixed_zero, dim3(1), dim3(64), 0, s, c->kmix_counts);
@@ -1345,8 +841,7 @@ int noalloc_dec(const NoAllocDev& d, size_t n, uint8_t* ss, uint8_t* ct, const u
   // a workgroup per request up to where a 64-request tile launch (~1 ms for any batch)
   // is faster: ~10.6 M decapsulations/s
   if (n <= 8192) {
-    hipLaunchKernelGGL((k_lowlat<K, true>), dim3((unsigned)n), dim3(256), 0, s, (int)n, ss, ct, sk,
-                       (const uint8_t*)nullptr, status);
+    return kyber_lowlat_dec(K, n, ss, ct, sk, status, s);
   } else {
     const int ntiles = (int)((n + Tile<K>::T - 1) / Tile<K>::T);
     const int grid = std::max(1, std::min(ntiles, d.cus * 4));  // the default fused_waves_per_cu

@@ -1,5 +1,6 @@
 """Staged Kyber kernels (sponge stages, matrix-core product stages) at the edges of
-their groups of 16, tiles of 64 and persistent grids, bit-exact against the CPU oracle."""
+their groups of 16, tiles of 64 and persistent grids, and the one-workgroup-per-request
+kernels, bit-exact against the CPU oracle."""
 import sys
 
 import numpy as np
@@ -70,4 +71,20 @@ def test_staged_keypair_and_encaps_vs_oracle(pqc, k, grid):
         ct, ss = ctx.enc_host(ALG[k], pk, coins)
         oct_, oss = O.kyber_batch("enc", k, [pk, coins])
         assert (ct == oct_).all() and (ss == oss).all()
+    ctx.close()
+
+
+@pytest.mark.parametrize("k", [2, 3, 4])
+def test_per_request_kernels_vs_oracle(pqc, k):
+    sizes = [1, 5, 200]
+    ctx = pqc.Context([ALG[k]], max_batch=max(sizes))
+    for n in sizes:
+        print("per-request kernels k", k, "n", n, flush=True)
+        pk, sk, ct = inputs(k, n, 4000 * k + n)
+        rng = np.random.default_rng(5000 * k + n)
+        coins = rng.integers(0, 256, (n, 64), dtype=np.uint8)
+        assert all((a == b).all() for a, b in zip(ctx.keypair_host(ALG[k], coins), O.kyber_batch("keypair", k, [coins])))
+        c32 = np.ascontiguousarray(coins[:, :32])
+        assert all((a == b).all() for a, b in zip(ctx.enc_host(ALG[k], pk, c32), O.kyber_batch("enc", k, [pk, c32])))
+        assert (ctx.dec_host(ALG[k], ct, sk) == O.kyber_batch("dec", k, [ct, sk])).all()
     ctx.close()
