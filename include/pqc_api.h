@@ -79,7 +79,8 @@ typedef struct pqc_tuning {
                                  many sponge waves per SIMD and half as many product workgroups per CU */
   int32_t mixed_order;        /* mixed-batch tile order: 0 = K 4,3,2; 1 = K 2,3,4; 2 = round-robin over K;
                                  3 = K 4,3,2 with 32-request tiles for K = 4 and K = 2 */
-  int32_t frodo_stream_block; /* threads per workgroup of the Frodo noise-stream kernel: 64, 128 or 256 */
+  int32_t frodo_stream_block; /* threads per workgroup of the Frodo noise-stream kernel on lane pairs
+                                 or lanes (calls above 4096 requests): 64, 128 or 256 */
   int32_t lowlat_max;         /* Kyber batches of at most this many requests run one
                                  workgroup per request (latency) instead of the throughput forms
                                  below: 0 = library default (1280), -1 = never, else 1..65536;
@@ -95,7 +96,8 @@ typedef struct pqc_tuning {
   int32_t fused_key_tile;     /* the same for the fused Kyber key generation */
   int32_t frodo_lane_min;     /* Keccak lane layout of the FrodoKEM-976 noise stream and F prefix in
                                  shared-key decapsulation: calls of at least this many requests run one state
-                                 per lane (throughput), smaller ones one state per lane pair (latency);
+                                 per lane (throughput), smaller ones one state per lane pair, or up to 4096
+                                 requests on 16 lanes (latency);
                                  0 = library default (49152), -1 = lane pairs always, else >= 1 */
 } pqc_tuning;
 int pqc_ctx_get_tuning(const pqc_ctx *ctx, pqc_tuning *t);

@@ -16,6 +16,7 @@
 #include <algorithm>
 
 #include "internal.h"
+#include "keccak_wide.cuh"
 #include "sponge.cuh"
 
 namespace pqc {
@@ -365,6 +366,77 @@ __global__ __launch_bounds__(256) void k_shake(int n, int npad, int with_f, FrKe
     absorb_ct_pair(S, ct + (size_t)r * CT, half);
 #pragma unroll
     for (int w = 0; w < 25; ++w) fstate[(size_t)r * 50 + 2 * w + half] = S[w];
+  }
+}
+
+// The same on 16 lanes per request (keccak_wide.cuh), four requests per wave: calls of
+// up to kWideMax requests, which leave SIMDs idle on lane pairs and are bound by the
+// serial chain.  Waves [0, ceil(n / 4)) are streams, written as k_shake writes them; waves
+// from there on (decapsulation) absorb the F prefixes.
+template <int W>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_shake_wide(int n, FrKeys keys, const uint8_t* mu, int mu_stride,
+                                                   uint8_t* raw, uint8_t* kout, const uint8_t* ct, uint32_t* fstate) {
+  __shared__ wide::Consts consts;
+  __shared__ wide::States states;
+  __shared__ uint32_t seed[4][8];
+  const int waves = (n + 3) / 4;
+  const int w0 = blockIdx.x;
+  wide::init_consts(consts);
+  __syncthreads();
+  wide::Sponge s;
+  s.init(states, consts);
+  const int rq = 4 * (w0 < waves ? w0 : w0 - waves) + s.st;
+  const bool act = rq < n;
+  const int r = act ? rq : n - 1;
+  if (w0 >= waves) {
+    s.absorb17<24>(reinterpret_cast<const uint32_t*>(ct + (size_t)r * CT), CT / 8, 0x1F, 0, (CT + SS) / 136);
+    s.squeeze<5>([&](int x, uint32_t v) {
+      const int w = s.word(x);
+      if (act && w < 25) fstate[(size_t)r * 50 + 2 * w + s.h] = v;
+    });
+    return;
+  }
+  uint32_t m[5];
+  {  // (seedSE || k) = SHAKE256(pkh || mu, 48)
+    const uint32_t* ph = reinterpret_cast<const uint32_t*>(keys.pkh_of(r));
+    const uint32_t* pm = reinterpret_cast<const uint32_t*>(mu + (size_t)r * mu_stride);
+#pragma unroll
+    for (int x = 0; x < 5; ++x) {
+      const int w = s.word(x);
+      m[x] = 0;
+      if (w < 3) m[x] = ph[2 * w + s.h];
+      if (w >= 3 && w < 6) m[x] = pm[2 * (w - 3) + s.h];
+      if (w == 6 && s.h == 0) m[x] = 0x1Fu;
+      if (w == kRateShake256 - 1 && s.h == 1) m[x] = 0x80000000u;
+    }
+    s.absorb(m);
+    s.permute();
+    uint32_t* ko = reinterpret_cast<uint32_t*>(kout + (size_t)r * 32);
+    s.squeeze<5>([&](int x, uint32_t v) {
+      const int w = s.word(x);
+      if (w < 3) seed[s.st][2 * w + s.h] = v;
+      if (act && w >= 3 && w < 6) ko[2 * (w - 3) + s.h] = v;
+    });
+    wide::sync();
+  }
+  // 0x96 || seedSE, padded: dword i of it
+#pragma unroll
+  for (int x = 0; x < 5; ++x) {
+    const int w = s.word(x), i = 2 * w + s.h;
+    const uint32_t lo = i == 0 ? 0x96000000u : seed[s.st][i < 7 ? i - 1 : 0], hi = i < 6 ? seed[s.st][i & 7] : 0x1Fu;
+    m[x] = i < 7 ? (lo >> 24) | (hi << 8) : 0;
+    if (w == kRateShake256 - 1 && s.h == 1) m[x] = 0x80000000u;
+  }
+  s.clear();
+  s.absorb(m);
+  // word x + 5 y of block b: its even-bit, then its odd-bit half
+  uint32_t* out = reinterpret_cast<uint32_t*>(raw + (size_t)r * RAWB) + 2 * (5 * s.y) + s.h;
+  for (int blk = 0; blk < 231; ++blk) {
+    s.permute<24>();
+#pragma unroll
+    for (int x = 0; x < 5; ++x)
+      if (act && s.word(x) < kRateShake256) out[2 * x] = s.a[x];
+    out += 2 * kRateShake256;
   }
 }
 
@@ -839,6 +911,40 @@ __global__ __launch_bounds__(64) void k_f_full(int n, uint8_t* ss, const uint8_t
   for (int w = 0; w < 3; ++w) o[2 * w] = S[w];
 }
 
+// The same on 16 lanes per request
+template <int W>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_f_full_wide(int n, uint8_t* ss, const uint8_t* ct, const uint8_t* kp) {
+  __shared__ wide::Consts consts;
+  __shared__ wide::States states;
+  wide::init_consts(consts);
+  __syncthreads();
+  wide::Sponge s;
+  s.init(states, consts);
+  const int rq = 4 * blockIdx.x + s.st;
+  const int r = rq < n ? rq : n - 1;
+  const uint32_t* c = reinterpret_cast<const uint32_t*>(ct + (size_t)r * CT);
+  const uint32_t* k = reinterpret_cast<const uint32_t*>(kp + (size_t)r * 32);
+  constexpr int FB = (CT + SS) / 136, CW = CT / 8 - 17 * FB;  // whole ciphertext blocks, ciphertext words after them
+  static_assert(CW + SS / 8 == 16, "the key's words and one padding word fill the last block");
+  s.absorb17<24>(c, CT / 8, 0x1F, 0, FB);
+  uint32_t m[5];
+#pragma unroll
+  for (int x = 0; x < 5; ++x) {
+    const int w = s.word(x);
+    m[x] = 0;
+    if (w < CW) m[x] = c[2 * (17 * FB + w) + s.h];
+    if (w >= CW && w < 16) m[x] = k[2 * (w - CW) + s.h];
+    if (w == 16) m[x] = s.h ? 0x80000000u : 0x1Fu;
+  }
+  s.absorb(m);
+  s.permute();
+  uint32_t* o = reinterpret_cast<uint32_t*>(ss + (size_t)r * SS);
+  s.squeeze<5>([&](int x, uint32_t v) {
+    const int w = s.word(x);
+    if (rq < n && w < SS / 8) o[2 * w + s.h] = v;
+  });
+}
+
 // ---- many keys: products on packed 16-bit VALU ---------------------------------------
 // [B'' | V] = S'.[A | B] + [E' | E''] (mod 2^16) for one request per workgroup
 // pair: workgroup (r, y) computes columns 512 y + 2 t, +1 for thread t with
@@ -957,12 +1063,24 @@ __global__ __launch_bounds__(64) void k_pkh_many(int n, uint8_t* pkh, size_t out
   for (int w = 0; w < 3; ++w) o[2 * w] = S[w];
 }
 
-// pkh = SHAKE256(pk, 24) for a loaded public key (lane 0)
-__global__ void k_pkh(uint8_t* pkh, const uint8_t* pk) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  uint64_t S[25];
-  sponge_absorb_words<kRateShake256>(S, reinterpret_cast<const uint64_t*>(pk), PK / 8, 0x1F);
-  for (int w = 0; w < 3; ++w) store_u64(pkh + 8 * w, S[w]);
+// The same on 16 lanes per key (a loaded public key; small batches)
+template <int W>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_pkh_wide(int n, uint8_t* pkh, size_t out_stride, const uint8_t* pk,
+                                                 size_t pk_stride) {
+  __shared__ wide::Consts consts;
+  __shared__ wide::States states;
+  wide::init_consts(consts);
+  __syncthreads();
+  wide::Sponge s;
+  s.init(states, consts);
+  const int rq = 4 * blockIdx.x + s.st;
+  const int r = rq < n ? rq : n - 1;
+  s.absorb17<24>(reinterpret_cast<const uint32_t*>(pk + (size_t)r * pk_stride), PK / 8, 0x1F, 0, PK / 8 / 17 + 1);
+  uint32_t* o = reinterpret_cast<uint32_t*>(pkh + (size_t)r * out_stride);
+  s.squeeze<5>([&](int x, uint32_t v) {
+    const int w = s.word(x);
+    if (rq < n && w < SS / 8) o[2 * w + s.h] = v;
+  });
 }
 
 // ---- key generation (kem.c:13-61), one key at a time ----------------------------------
@@ -1050,7 +1168,8 @@ int frodo_load_key(pqc_ctx* c, const uint8_t* key, int is_sk, hipStream_t s) {
     if (hipMemcpyAsync(c->fr_pkh, key + SK_PKH, SS, hipMemcpyDeviceToDevice, s) != hipSuccess) return PQC_ERR_DEVICE;
   } else {
     if (hipMemcpyAsync(c->fr_pk, key, PK, hipMemcpyDeviceToDevice, s) != hipSuccess) return PQC_ERR_DEVICE;
-    hipLaunchKernelGGL(k_pkh, dim3(1), dim3(64), 0, s, c->fr_pkh, (const uint8_t*)c->fr_pk);
+    hipLaunchKernelGGL(k_pkh_wide<1>, dim3(1), dim3(64), 0, s, 1, c->fr_pkh, (size_t)SS, (const uint8_t*)c->fr_pk,
+                       (size_t)PK);
   }
   c->fr_has_sk = is_sk;
   hipLaunchKernelGGL(k_gen_a, dim3((N + 63) / 64), dim3(64), 0, s, c->fr_a16, (const uint8_t*)c->fr_pk);
@@ -1127,6 +1246,35 @@ static FrKeys loaded_key(pqc_ctx* c) {
   return FrKeys{c->fr_sk, 0, c->fr_pkh, 0, c->fr_pk, 0, c->fr_a16, 0, nullptr};
 }
 
+// Calls of up to this many requests run their sponges on 16 lanes per request: one stream
+// wave per SIMD at 4096 (two with the F prefixes).  Measured on MI355X, us per call, lane
+// pairs and 16 lanes: decapsulation of 1 / 501 / 2048 / 4096 requests 1394 / 1182 / 1225 /
+// 1284 -> 769 / 790 / 871 / 950; encapsulation 2086 / 1912 / 1960 / 2019 -> 1122 / 1147 /
+// 1232 / 1286.  At 6000, pairs (one wave per SIMD or less) take 1361, about what 16 lanes
+// would at three waves per SIMD.
+constexpr int kWideMax = 4096;
+
+static void launch_f_full(const pqc_ctx* c, int ni, uint8_t* ss, const uint8_t* ct, const uint8_t* kp, hipStream_t s) {
+  const int waves = (ni + 3) / 4;
+  if (ni <= kWideMax)
+    with_simd_waves(c->cu_count, waves, [&](auto w) {
+      hipLaunchKernelGGL(k_f_full_wide<decltype(w)::value>, dim3(waves), dim3(64), 0, s, ni, ss, ct, kp);
+    });
+  else
+    hipLaunchKernelGGL(k_f_full, dim3((2 * ni + 63) / 64), dim3(64), 0, s, ni, ss, ct, kp);
+}
+
+static void launch_pkh(const pqc_ctx* c, int m, uint8_t* pkh, size_t out_stride, const uint8_t* pk, size_t pk_stride, hipStream_t s) {
+  const int waves = (m + 3) / 4;
+  if (m <= kWideMax)
+    with_simd_waves(c->cu_count, waves, [&](auto w) {
+      hipLaunchKernelGGL(k_pkh_wide<decltype(w)::value>, dim3(waves), dim3(64), 0, s, m, pkh, out_stride, pk,
+                         pk_stride);
+    });
+  else
+    hipLaunchKernelGGL(k_pkh_many, dim3((2 * m + 63) / 64), dim3(64), 0, s, m, pkh, out_stride, pk, pk_stride);
+}
+
 // G2 and the S'/E'/E'' stream of n requests (lane pairs; with_f adds the F prefix
 // of each ciphertext), then its sampling into the ROWS or fragment layouts.
 template <bool ROWS>
@@ -1141,6 +1289,16 @@ static void launch_stream(pqc_ctx* c, const FrScratch& f, int ni, int with_f, co
     hipLaunchKernelGGL(k_shake_lane, dim3((lanes + sb - 1) / sb), dim3(sb), 0, s, ni, nlane, with_f, keys, mu,
                        mu_stride, f.raw, f.kp, ct, with_f ? reinterpret_cast<uint64_t*>(f.fstate) : nullptr);
     hipLaunchKernelGGL((k_sample<false, false>), dim3((nt + 255) / 256), dim3(256), 0, s, ni, (const uint8_t*)f.raw,
+                       f.sfrag, f.efrag);
+    return;
+  }
+  if (ni <= kWideMax) {
+    const int waves = (with_f ? 2 : 1) * ((ni + 3) / 4);
+    with_simd_waves(c->cu_count, waves, [&](auto w) {
+      hipLaunchKernelGGL(k_shake_wide<decltype(w)::value>, dim3(waves), dim3(64), 0, s, ni, keys, mu, mu_stride, f.raw,
+                         f.kp, ct, with_f ? f.fstate : (uint32_t*)nullptr);
+    });
+    hipLaunchKernelGGL((k_sample<ROWS, true>), dim3((nt + 255) / 256), dim3(256), 0, s, ni, (const uint8_t*)f.raw,
                        f.sfrag, f.efrag);
     return;
   }
@@ -1239,8 +1397,7 @@ int frodo_enc_keyed(pqc_ctx* c, size_t n, uint8_t* ct, uint8_t* ss, const uint8_
   launch_stream<true>(c, f, ni, 0, keys, mu, MU, nullptr, s);
   hipLaunchKernelGGL(k_mk_product<kEncaps>, dim3(ni, 2), dim3(256), 0, s, ni, (const int8_t*)f.sfrag,
                      (const int8_t*)f.efrag, keys, ct, mu, MU, (uint8_t*)nullptr);
-  hipLaunchKernelGGL(k_f_full, dim3((2 * ni + 63) / 64), dim3(64), 0, s, ni, ss, (const uint8_t*)ct,
-                     (const uint8_t*)f.kp);
+  launch_f_full(c, ni, ss, ct, f.kp, s);
   return hip_err(hipGetLastError());
 }
 
@@ -1274,7 +1431,7 @@ int frodo_enc_batch_strided(pqc_ctx* c, size_t n, uint8_t* ct, uint8_t* ss, cons
     const int m = (int)(n - off < (size_t)kFrChunk ? n - off : (size_t)kFrChunk);
     const uint8_t* pkc = pk + off * pk_stride;
     hipLaunchKernelGGL(k_gen_a_many, dim3((m * N + 255) / 256), dim3(256), 0, s, m, c->fr_abuf, pkc, pk_stride);
-    hipLaunchKernelGGL(k_pkh_many, dim3((2 * m + 63) / 64), dim3(64), 0, s, m, pkh, (size_t)24, pkc, pk_stride);
+    launch_pkh(c, m, pkh, 24, pkc, pk_stride, s);
     const FrKeys keys{nullptr, 0, pkh, 24, pkc, pk_stride, c->fr_abuf, (size_t)N * N, nullptr};
     int rc = frodo_enc_keyed(c, m, ct + off * CT, ss + off * SS, mu + off * MU, keys, s);
     if (rc) return rc;
@@ -1296,8 +1453,7 @@ int frodo_enc(pqc_ctx* c, size_t n, uint8_t* ct, uint8_t* ss, const uint8_t* mu,
     launch_stream<false>(c, f, ni, 0, keys, muc, MU, nullptr, t);
     int r = launch_gemm<kEncaps>(c, m, f, ctc, muc, MU, t);
     if (r) return r;
-    hipLaunchKernelGGL(k_f_full, dim3((2 * ni + 63) / 64), dim3(64), 0, t, ni, ss + e0 * SS, (const uint8_t*)ctc,
-                       (const uint8_t*)f.kp);
+    launch_f_full(c, ni, ss + e0 * SS, ctc, f.kp, t);
     return hip_err(hipGetLastError());
   });
 }
@@ -1316,8 +1472,7 @@ int frodo_keypair(pqc_ctx* c, size_t n, uint8_t* pk, uint8_t* sk, const uint8_t*
                        (const uint16_t*)f.se, (const uint8_t*)seedA, rnd);
   }
   // sk tail: H(pk) of every key in one launch
-  hipLaunchKernelGGL(k_pkh_many, dim3((2 * ni + 63) / 64), dim3(64), 0, s, ni, sk + SK_PKH, (size_t)SK,
-                     (const uint8_t*)pk, (size_t)PK);
+  launch_pkh(c, ni, sk + SK_PKH, SK, pk, PK, s);
   c->fr_loaded = 0;  // the A buffer now holds the last generated key's A
   return hip_err(hipGetLastError());
 }

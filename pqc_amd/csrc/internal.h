@@ -4,6 +4,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/pqc_api.h"
 
 constexpr int kFrSideStreams = 3;
@@ -86,6 +88,25 @@ struct pqc_ctx {
 };
 
 namespace pqc {
+
+// Waves per SIMD that a launch of `wgs` one-wave workgroups needs: 1, 2 or 4 (4: as many
+// as fit).  The hardware spreads workgroups evenly over CUs but not over a CU's SIMDs:
+// of 1024 workgroups ~100 SIMDs get two and as many none, and two serial Keccak chains on
+// one SIMD take 40% longer (1024 waves of 116 permutations on 16 lanes per state: 551 us,
+// one wave on every SIMD 388 us).  A kernel compiled for at most W waves per SIMD
+// (PQC_SIMD_WAVES: the compiler rounds its registers up to that) is spread evenly.
+inline int simd_waves(int cus, int wgs) { return wgs <= 4 * cus ? 1 : wgs <= 8 * cus ? 2 : 4; }
+#define PQC_SIMD_WAVES(W) __attribute__((amdgpu_waves_per_eu(W, (W) < 4 ? (W) : 8)))
+
+// f(std::integral_constant<int, W>) for W = simd_waves(cus, wgs)
+template <class F>
+inline void with_simd_waves(int cus, int wgs, F&& f) {
+  switch (simd_waves(cus, wgs)) {
+    case 1: f(std::integral_constant<int, 1>{}); break;
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    default: f(std::integral_constant<int, 4>{}); break;
+  }
+}
 
 inline int hip_err(hipError_t e) { return e == hipSuccess ? PQC_OK : PQC_ERR_DEVICE; }
 

@@ -136,11 +136,11 @@ __device__ __forceinline__ void keccakf1600(uint64_t (&A64)[25]) {
   for (int i = 0; i < 25; ++i) A64[i] = (uint64_t)A[i].lo | ((uint64_t)A[i].hi << 32);
 }
 
-// The same permutation for kernels that keep several waves on a SIMD: two rounds per
-// trip, the next round constant loaded a round ahead.  Measured on MI355X, G state
-// permutations/s of the whole GPU at 1 / 2 / 4 waves per SIMD: 7.1 / 9.4 / 10.1, against
-// 6.7 / 9.0 / 9.8 for the loop above (a taken branch costs a lone wave ~200 cycles).
-__device__ __forceinline__ void keccakf1600_dense(uint64_t (&A64)[25]) {
+// The same permutation, two rounds per trip and the next round constant loaded a round
+// ahead.  Measured on MI355X, us per permutation of a lone wave: 7.65, against 8.35 for
+// the loop above and 8.2 to 8.6 for three to twelve rounds per trip (24: 7.2, at 34 KB of
+// code); at four waves per SIMD 10.1 G state permutations/s against 9.8.
+__device__ __forceinline__ void keccakf1600_two(uint64_t (&A64)[25]) {
   Lane2 A[25];
 #pragma unroll
   for (int i = 0; i < 25; ++i) A[i] = Lane2{(uint32_t)A64[i], (uint32_t)(A64[i] >> 32)};

@@ -17,12 +17,19 @@
 // unrolled interleaved lane pair, 6.3 for the rolled pair, 7.9 for one state per lane; at
 // two waves per SIMD 4.8.  Its throughput is a fifth of the one-state-per-lane form's.
 #pragma once
+#include <stddef.h>
+
 #include "keccak.cuh"
 
 namespace pqc {
 namespace wide {
 
-constexpr int kRowWords = 8, kHalfWords = 5 * kRowWords, kStateWords = 2 * kHalfWords;
+// LDS image of a state: rows (half, plane) of words x = 0..3 at 4 row, word x = 4 at
+// kCol4 + row.  With these strides and the zero lanes' places after the four states, a
+// round's five writes and two reads meet ~40 bank cycles per wave; rows of 8 words took
+// 50, and four waves on a CU ran 40% slower for it (116 permutations each: 551 against
+// 388 us).
+constexpr int kCol4 = 45, kStateWords = 80;
 
 struct Maps {
   uint8_t amt[2][8][5];   // alignbit amount of the word about to move
@@ -38,7 +45,8 @@ constexpr Maps make_maps() {
         const int o = kKeccakMaps.rho[x + 5 * y];
         const int rot = o / 2 + ((o & 1) && h ? 1 : 0);
         m.amt[h][y][x] = (uint8_t)((32 - rot) & 31);
-        m.dst[h][y][x] = (uint16_t)((h ^ (o & 1)) * kHalfWords + (2 * x + 3 * y) % 5 * kRowWords + y);
+        const int row = (h ^ (o & 1)) * 5 + (2 * x + 3 * y) % 5;
+        m.dst[h][y][x] = (uint16_t)(y < 4 ? 4 * row + y : kCol4 + row);
       }
   return m;
 }
@@ -47,18 +55,18 @@ static __device__ const IlRc c_rc = il_round_constants();
 
 // Constants of a workgroup's waves, and one wave's states
 struct Consts {
-  alignas(16) uint32_t zero[8];
-  uint32_t trash[8];
   uint32_t rc[2][24], none[24];
 };
 struct States {
   alignas(16) uint32_t w[4 * kStateWords];
+  uint32_t trash[72];  // where the zero lanes write: a word each
+  uint32_t zero[8];    // and read
 };
+static_assert(offsetof(States, zero) % 16 == 0, "16-byte read");
 
 // every thread of the workgroup; a barrier must follow
 __device__ __forceinline__ void init_consts(Consts& c) {
   const int t = threadIdx.x;
-  if (t < 8) c.zero[t] = 0;
   if (t < 24) {
     c.rc[0][t] = c_rc.e[t];
     c.rc[1][t] = c_rc.o[t];
@@ -82,7 +90,7 @@ struct Sponge {
   uint32_t a[5];
   uint32_t amt[5];
   uint32_t* dst[5];
-  const uint32_t* src;
+  const uint32_t *src, *src4;
   const uint32_t* rc;
   uint32_t rot1, sel_in, sel_out;
   int h, y, st;
@@ -96,9 +104,11 @@ struct Sponge {
 #pragma unroll
     for (int x = 0; x < 5; ++x) {
       amt[x] = c_maps.amt[h][y][x];
-      dst[x] = y < 5 ? base + c_maps.dst[h][y][x] : c.trash;
+      dst[x] = y < 5 ? base + c_maps.dst[h][y][x] : s.trash + l;
     }
-    src = y < 5 ? base + h * kHalfWords + y * kRowWords : c.zero;
+    src = y < 5 ? base + 4 * (5 * h + y) : s.zero;
+    src4 = y < 5 ? base + kCol4 + 5 * h + y : s.zero + 4;
+    if (l < 8) s.zero[l] = 0;
     rc = y == 0 ? c.rc[h] : c.none;
     rot1 = h ? 31u : 0u;
     sel_in = h ? 0x03010705u : 0x06040200u;
@@ -110,8 +120,11 @@ struct Sponge {
     for (int x = 0; x < 5; ++x) a[x] = 0;
   }
 
+  // UNROLL rounds per loop trip: 24 (9 KB of code) for a kernel that is one long chain,
+  // 3% faster than 4
+  template <int UNROLL = 4>
   __device__ __forceinline__ void permute() {
-#pragma unroll 4
+#pragma unroll UNROLL
     for (int r = 0; r < 24; ++r) {
       const uint32_t k = rc[r];
       uint32_t C[5], S[5];
@@ -131,7 +144,7 @@ struct Sponge {
       sync();
       typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
       const u32x4 q = *reinterpret_cast<const u32x4*>(src);
-      const uint32_t B[5] = {q[0], q[1], q[2], q[3], src[4]};
+      const uint32_t B[5] = {q[0], q[1], q[2], q[3], *src4};
       sync();
 #pragma unroll
       for (int x = 0; x < 5; ++x) a[x] = chi_32(B[x], B[(x + 1) % 5], B[(x + 2) % 5]);
@@ -174,30 +187,35 @@ struct Sponge {
   }
   __device__ __forceinline__ int word(int x) const { return x + 5 * y; }  // >= 25 on the zero lanes
 
-  // this lane's halves of block b (17 words) of a message of nwords 64-bit words at the
-  // 4-byte aligned p (the same one, or one per state), SHA3-256 / SHAKE256 padding included
-  template <class P>
-  __device__ __forceinline__ void load_block17(uint32_t (&m)[5], P p, int nwords, int b, uint32_t domain) const {
-    const int rem = nwords - 17 * b;  // words left
-#pragma unroll
-    for (int x = 0; x < 5; ++x) {
-      const int w = word(x);
-      uint32_t v = 0;
-      if (w < 17 && w < rem) v = p[2 * (17 * b + w) + h];
-      if (w < 17 && w == rem && h == 0) v = domain;
-      if (w == 16 && rem < 17 && h == 1) v ^= 0x80000000u;
-      m[x] = v;
-    }
-  }
-  // absorb blocks [b0, b1) of it, the next block's words loaded during a permutation
-  template <class P>
+  // Absorb blocks [b0, b1) (17 words each) of a message of nwords 64-bit words at the
+  // 4-byte aligned p (the same for all states or one per state), SHA3-256 / SHAKE256 padding
+  // included in the last one; the next block's words load during a permutation.  The words
+  // stay as loaded until they are absorbed (a select on a loaded value waits for it where it
+  // stands), and no branch goes around a load: lanes without a word read the message's
+  // first one and drop it.
+  template <int UNROLL = 4, class P>
   __device__ __forceinline__ void absorb17(P p, int nwords, uint32_t domain, int b0, int b1) {
-    uint32_t m[5];
-    load_block17(m, p, nwords, b0, domain);
+    uint32_t raw[5];
+    auto load = [&](int b) {
+      const int rem = nwords - 17 * b, own = rem < 17 ? rem : 17;
+#pragma unroll
+      for (int x = 0; x < 5; ++x) raw[x] = p[word(x) < own ? 2 * (17 * b + word(x)) + h : h];
+    };
+    load(b0);
     for (int b = b0; b < b1; ++b) {
+      const int rem = nwords - 17 * b, own = rem < 17 ? rem : 17;  // words left
+      uint32_t m[5];
+#pragma unroll
+      for (int x = 0; x < 5; ++x) {
+        const int w = word(x);
+        uint32_t v = w < own ? raw[x] : 0u;
+        v = (w < 17 && w == rem && h == 0) ? domain : v;
+        v ^= (w == 16 && rem < 17 && h == 1) ? 0x80000000u : 0u;
+        m[x] = v;
+      }
       absorb(m);
-      if (b + 1 < b1) load_block17(m, p, nwords, b + 1, domain);
-      permute();
+      load(b + 1 < b1 ? b + 1 : b);
+      permute<UNROLL>();
     }
   }
 };

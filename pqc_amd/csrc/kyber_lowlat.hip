@@ -36,10 +36,11 @@ struct Shape {
 constexpr int kMaxWaves = Shape<4>::waves;
 // Waves per SIMD the registers are cut for.  K = 4's six waves fit a CU four times at 6
 // (80 VGPRs, a few spills): 1000 decapsulations 124 us against 154 at 5 and 181 at 4, one
-// 53 against 51.  K = 2, 3 need no more than 96 VGPRs: 5, four workgroups per CU.
-template <int K>
+// 53 against 51.  K = 2, 3 decapsulation needs no more than 96
+// VGPRs: 5, four workgroups per CU.
+template <int K, bool DEC>
 constexpr int simd_waves() {
-  return K == 4 ? 6 : 5;
+  return K == 4 || !DEC ? 6 : 5;
 }
 
 template <int K>
@@ -426,7 +427,7 @@ __device__ __forceinline__ void key_body(uint8_t* pk, uint8_t* sk, const uint8_t
 //   encapsulation 1 / 257 / 1000:                188 / 235 / 297 -> 82 / 92 / 124
 //   key generation 1 / 300 / 1000 (was staged):  163 / 164 / 165 -> 57 / 66 / 89
 template <int K, bool DEC>
-__global__ __launch_bounds__(64 * Shape<K>::waves, simd_waves<K>()) void k_lowlat(int n, uint8_t* __restrict__ ss,
+__global__ __launch_bounds__(64 * Shape<K>::waves, (simd_waves<K, DEC>())) void k_lowlat(int n, uint8_t* __restrict__ ss,
                                                                     uint8_t* __restrict__ ct,
                                                                     const uint8_t* __restrict__ key,
                                                                     const uint8_t* __restrict__ coins,
@@ -445,7 +446,7 @@ __global__ __launch_bounds__(64 * Shape<K>::waves, simd_waves<K>()) void k_lowla
 }
 
 template <int K>
-__global__ __launch_bounds__(64 * Shape<K>::waves, simd_waves<K>()) void k_lowlat_key(int n, uint8_t* __restrict__ pk,
+__global__ __launch_bounds__(64 * Shape<K>::waves, 6) void k_lowlat_key(int n, uint8_t* __restrict__ pk,
                                                                         uint8_t* __restrict__ sk,
                                                                         const uint8_t* __restrict__ coins,
                                                                         uint32_t* __restrict__ status) {

@@ -129,7 +129,7 @@ __device__ __forceinline__ bool sample_entry(uint8_t* entry, int16_t* row, const
   int chunk = 0;  // chunks written
   for (int blk = 0; blk < kMaxBlocks; ++blk) {
     if (blk >= 4 && !__any(valid && chunk < 32)) break;
-    keccakf1600_dense(A);
+    keccakf1600_two(A);
 #pragma unroll
     for (int part = 0; part < kRateShake128 / kPartWords; ++part) {
       int16_t* p = row + left;
@@ -189,7 +189,7 @@ __device__ __forceinline__ void dec_hash_wave(const Src& src, const Scratch& sc,
   const bool act = r < b.n;
   const ReqP q = src.template req<K, true>(act ? r : b.n - 1);
   uint64_t A[25];
-  sponge_absorb_dense<kRateSha3_256>(A, q.ct, P::ct_bytes / 8, 0x06);
+  sponge_absorb_two<kRateSha3_256, P::ct_bytes / 8>(A, q.ct, 0x06);
   if (act) store_words4(sc.row_of(b.grp0 + r / 16, r % 16) + kRowH, A);
 }
 
@@ -229,7 +229,7 @@ __device__ __forceinline__ void enc_open_wave(const Src& src, const Scratch& sc,
   const int rc = act ? r : b.n - 1;
   const ReqP q = src.template req<K, false>(rc);
   uint64_t A[25], m[8], c4[4];
-  sponge_absorb_dense<kRateSha3_256>(A, q.key, P::pk_bytes / 8, 0x06);
+  sponge_absorb_two<kRateSha3_256, P::pk_bytes / 8>(A, q.key, 0x06);
 #pragma unroll
   for (int i = 0; i < 4; ++i) m[4 + i] = A[i];
   load_words4(c4, q.coins);
@@ -263,7 +263,7 @@ __device__ __forceinline__ void enc_final_wave(const Src& src, const Scratch& sc
   const int rc = act ? r : b.n - 1;
   const ReqP q = src.template req<K, false>(rc);
   uint64_t A[25], m[8];
-  sponge_absorb_dense<kRateSha3_256>(A, q.ct, P::ct_bytes / 8, 0x06);
+  sponge_absorb_two<kRateSha3_256, P::ct_bytes / 8>(A, q.ct, 0x06);
   const uint8_t* row = sc.row_of(b.grp0 + rc / 16, rc % 16);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -306,7 +306,7 @@ __device__ __forceinline__ void key_final_wave(const KeySrc& src, int n, int w) 
   const int r = 64 * w + (threadIdx.x & 63);
   const int rc = r < n ? r : n - 1;
   uint64_t A[25];
-  sponge_absorb_dense<kRateSha3_256>(A, src.pk + (size_t)rc * P::pk_bytes, P::pk_bytes / 8, 0x06);
+  sponge_absorb_two<kRateSha3_256, P::pk_bytes / 8>(A, src.pk + (size_t)rc * P::pk_bytes, 0x06);
   if (r < n) store_words4(src.sk + (size_t)r * P::sk_bytes + P::hpk_off, A);
 }
 
@@ -643,8 +643,8 @@ __global__ __launch_bounds__(kProdThreads, 2) void k_open(int n, DenseSrc src, S
 }
 
 // waves: H(ct), then G and PRF (the longest chains first), then the matrix entries
-template <int K>
-__global__ __launch_bounds__(64, 4) void k_dec_sponge(int n, DenseSrc src, Scratch sc) {
+template <int K, int W>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_dec_sponge(int n, DenseSrc src, Scratch sc) {
   using P = Params<K>;
   __shared__ SponLds sh;
   const Bucket b{n, 0};
@@ -669,14 +669,14 @@ __global__ __launch_bounds__(kProdThreads, 2) void k_dec_reencrypt(int n, DenseS
   for (int tile = blockIdx.x; tile < (n + 63) / 64; tile += gridDim.x) reencrypt_tile<K, true>(src, sc, b, tile, sh);
 }
 
-template <int K>
-__global__ __launch_bounds__(64) void k_dec_kdf(int n, DenseSrc src, Scratch sc) {
+template <int K, int W>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_dec_kdf(int n, DenseSrc src, Scratch sc) {
   for (int w = blockIdx.x; w < (n + 63) / 64; w += gridDim.x) dec_kdf_wave<K>(src, sc, Bucket{n, 0}, w);
 }
 
 // encapsulation: H(pk), m, G (the longest chains first), then the matrix entries
-template <int K>
-__global__ __launch_bounds__(64, 4) void k_enc_sponge(int n, DenseSrc src, Scratch sc) {
+template <int K, int W>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_enc_sponge(int n, DenseSrc src, Scratch sc) {
   using P = Params<K>;
   __shared__ SponLds sh;
   const Bucket b{n, 0};
@@ -690,8 +690,8 @@ __global__ __launch_bounds__(64, 4) void k_enc_sponge(int n, DenseSrc src, Scrat
   }
 }
 
-template <int K>
-__global__ __launch_bounds__(64, 4) void k_enc_prf(int n, Scratch sc) {
+template <int K, int W>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_enc_prf(int n, Scratch sc) {
   const int wr = (n + 63) / 64;
   for (int w = blockIdx.x; w < wr * (2 * K + 1); w += gridDim.x) prf_wave(sc, Bucket{n, 0}, w % wr, w / wr);
 }
@@ -704,19 +704,19 @@ __global__ __launch_bounds__(kProdThreads, 2) void k_enc_encrypt(int n, DenseSrc
   for (int tile = blockIdx.x; tile < (n + 63) / 64; tile += gridDim.x) reencrypt_tile<K, false>(src, sc, b, tile, sh);
 }
 
-template <int K>
-__global__ __launch_bounds__(64, 4) void k_enc_final(int n, DenseSrc src, Scratch sc) {
+template <int K, int W>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_enc_final(int n, DenseSrc src, Scratch sc) {
   for (int w = blockIdx.x; w < (n + 63) / 64; w += gridDim.x) enc_final_wave<K>(src, sc, Bucket{n, 0}, w);
 }
 
 // key generation
-template <int K>
-__global__ __launch_bounds__(64, 4) void k_key_seed(int n, KeySrc src, Scratch sc) {
+template <int K, int W>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_key_seed(int n, KeySrc src, Scratch sc) {
   for (int w = blockIdx.x; w < (n + 63) / 64; w += gridDim.x) key_seed_wave<K>(src, sc, n, w);
 }
 
-template <int K>
-__global__ __launch_bounds__(64, 4) void k_key_sponge(int n, KeySrc src, Scratch sc) {
+template <int K, int W>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_key_sponge(int n, KeySrc src, Scratch sc) {
   using P = Params<K>;
   __shared__ SponLds sh;
   const Bucket b{n, 0};
@@ -736,8 +736,8 @@ __global__ __launch_bounds__(kProdThreads, 2) void k_key_mul(int n, KeySrc src, 
   for (int tile = blockIdx.x; tile < (n + 63) / 64; tile += gridDim.x) key_tile<K>(src, sc, Bucket{n, 0}, tile, sh);
 }
 
-template <int K>
-__global__ __launch_bounds__(64, 4) void k_key_final(int n, KeySrc src) {
+template <int K, int W>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_key_final(int n, KeySrc src) {
   for (int w = blockIdx.x; w < (n + 63) / 64; w += gridDim.x) key_final_wave<K>(src, n, w);
 }
 
@@ -834,8 +834,8 @@ __global__ __launch_bounds__(kProdThreads, 2) void k_mixed_encrypt(const uint32_
 }
 
 // KDF (DEC), or H(ct) and KDF
-template <bool DEC>
-__global__ __launch_bounds__(64, 4) void k_mixed_final(const uint32_t* counts, MixedSrc src, Scratch sc) {
+template <bool DEC, int W>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_mixed_final(const uint32_t* counts, MixedSrc src, Scratch sc) {
   const Buckets bs = buckets_of(counts);
   for (int t = blockIdx.x;; t += gridDim.x) {
     int w = t;
@@ -896,6 +896,13 @@ static int sponge_grid(const pqc_ctx* c, int waves) {
   return std::max(1, std::min(g, waves));
 }
 
+// one-wave workgroups of a kernel templated on the waves per SIMD it is compiled for
+#define LAUNCH_WAVES(c, grid, s, KERNEL, ...)                                                 \
+  with_simd_waves((c)->cu_count, grid, [&](auto w) {                                          \
+    constexpr int W = decltype(w)::value;                                                     \
+    hipLaunchKernelGGL((KERNEL), dim3(grid), dim3(64), 0, s, __VA_ARGS__);                    \
+  })
+
 template <int K>
 static int dec(pqc_ctx* c, size_t n_all, uint8_t* ss, uint8_t* ct, const uint8_t* sk, hipStream_t s) {
   using P = Params<K>;
@@ -905,9 +912,10 @@ static int dec(pqc_ctx* c, size_t n_all, uint8_t* ss, uint8_t* ct, const uint8_t
     const int tiles = (n + 63) / 64, waves = 2 * tiles + matrix_waves<K>(n);
     const DenseSrc src{ss + at * 32, ct + at * P::ct_bytes, sk + at * P::sk_bytes, nullptr, c->kprf};
     hipLaunchKernelGGL((k_open<K>), dim3(prod_grid(c, tiles)), dim3(kProdThreads), 0, s, n, src, sc);
-    hipLaunchKernelGGL((k_dec_sponge<K>), dim3(sponge_grid(c, waves)), dim3(64), 0, s, n, src, sc);
+    const int sg = sponge_grid(c, waves), kg = sponge_grid(c, tiles);
+    LAUNCH_WAVES(c, sg, s, (k_dec_sponge<K, W>), n, src, sc);
     hipLaunchKernelGGL((k_dec_reencrypt<K>), dim3(prod_grid(c, tiles)), dim3(kProdThreads), 0, s, n, src, sc);
-    hipLaunchKernelGGL((k_dec_kdf<K>), dim3(sponge_grid(c, tiles)), dim3(64), 0, s, n, src, sc);
+    LAUNCH_WAVES(c, kg, s, (k_dec_kdf<K, W>), n, src, sc);
     const int rc = hip_err(hipGetLastError());
     if (rc) return rc;
   }
@@ -923,10 +931,12 @@ static int enc(pqc_ctx* c, size_t n_all, uint8_t* ss, uint8_t* ct, const uint8_t
     const int n = (int)std::min(n_all - at, c->kstage_max);
     const int tiles = (n + 63) / 64;
     const DenseSrc src{ss + at * 32, ct + at * P::ct_bytes, pk + at * P::pk_bytes, coins + at * 32, c->kprf};
-    hipLaunchKernelGGL((k_enc_sponge<K>), dim3(sponge_grid(c, tiles + matrix_waves<K>(n))), dim3(64), 0, s, n, src, sc);
-    hipLaunchKernelGGL((k_enc_prf<K>), dim3(sponge_grid(c, tiles * (2 * K + 1))), dim3(64), 0, s, n, sc);
+    const int sg = sponge_grid(c, tiles + matrix_waves<K>(n)), pg = sponge_grid(c, tiles * (2 * K + 1)),
+              fg = sponge_grid(c, tiles);
+    LAUNCH_WAVES(c, sg, s, (k_enc_sponge<K, W>), n, src, sc);
+    LAUNCH_WAVES(c, pg, s, (k_enc_prf<K, W>), n, sc);
     hipLaunchKernelGGL((k_enc_encrypt<K>), dim3(prod_grid(c, tiles)), dim3(kProdThreads), 0, s, n, src, sc);
-    hipLaunchKernelGGL((k_enc_final<K>), dim3(sponge_grid(c, tiles)), dim3(64), 0, s, n, src, sc);
+    LAUNCH_WAVES(c, fg, s, (k_enc_final<K, W>), n, src, sc);
     const int rc = hip_err(hipGetLastError());
     if (rc) return rc;
   }
@@ -941,11 +951,11 @@ static int keypair(pqc_ctx* c, size_t n_all, uint8_t* pk, uint8_t* sk, const uin
     const int n = (int)std::min(n_all - at, c->kstage_max);
     const int tiles = (n + 63) / 64;
     const KeySrc src{pk + at * P::pk_bytes, sk + at * P::sk_bytes, coins + at * 64};
-    hipLaunchKernelGGL((k_key_seed<K>), dim3(sponge_grid(c, tiles)), dim3(64), 0, s, n, src, sc);
-    hipLaunchKernelGGL((k_key_sponge<K>), dim3(sponge_grid(c, matrix_waves<K>(n) + 2 * K * tiles)), dim3(64), 0, s, n,
-                       src, sc);
+    const int sg = sponge_grid(c, matrix_waves<K>(n) + 2 * K * tiles), fg = sponge_grid(c, tiles);
+    LAUNCH_WAVES(c, fg, s, (k_key_seed<K, W>), n, src, sc);
+    LAUNCH_WAVES(c, sg, s, (k_key_sponge<K, W>), n, src, sc);
     hipLaunchKernelGGL((k_key_mul<K>), dim3(prod_grid(c, tiles)), dim3(kProdThreads), 0, s, n, src, sc);
-    hipLaunchKernelGGL((k_key_final<K>), dim3(sponge_grid(c, tiles)), dim3(64), 0, s, n, src);
+    LAUNCH_WAVES(c, fg, s, (k_key_final<K, W>), n, src);
     const int rc = hip_err(hipGetLastError());
     if (rc) return rc;
   }
@@ -959,17 +969,18 @@ static int mixed(pqc_ctx* c, int dec, size_t n, const MixedSrc& src, hipStream_t
   const uint32_t* counts = c->kmix_counts;
   const int tiles = (int)(n / 64) + 3;  // each bucket rounds up by itself
   const int mat = ((int)((n + 15) / 16) + 3) * kmax * kmax / 4 + 3;
+  const int fg = sponge_grid(c, tiles);
   const dim3 prod(prod_grid(c, tiles)), prod_wg(kProdThreads), wg(64);
   if (dec) {
     hipLaunchKernelGGL(k_mixed_open, prod, prod_wg, 0, s, counts, src, sc);
     hipLaunchKernelGGL(k_mixed_dec_sponge, dim3(sponge_grid(c, 2 * tiles + mat)), wg, 0, s, counts, src, sc);
     hipLaunchKernelGGL(k_mixed_encrypt<true>, prod, prod_wg, 0, s, counts, src, sc);
-    hipLaunchKernelGGL(k_mixed_final<true>, dim3(sponge_grid(c, tiles)), wg, 0, s, counts, src, sc);
+    LAUNCH_WAVES(c, fg, s, (k_mixed_final<true, W>), counts, src, sc);
   } else {
     hipLaunchKernelGGL(k_mixed_enc_sponge, dim3(sponge_grid(c, tiles + mat)), wg, 0, s, counts, src, sc);
     hipLaunchKernelGGL(k_mixed_prf, dim3(sponge_grid(c, tiles * (2 * kmax + 1))), wg, 0, s, counts, sc);
     hipLaunchKernelGGL(k_mixed_encrypt<false>, prod, prod_wg, 0, s, counts, src, sc);
-    hipLaunchKernelGGL(k_mixed_final<false>, dim3(sponge_grid(c, tiles)), wg, 0, s, counts, src, sc);
+    LAUNCH_WAVES(c, fg, s, (k_mixed_final<false, W>), counts, src, sc);
   }
   return hip_err(hipGetLastError());
 }
