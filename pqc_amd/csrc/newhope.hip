@@ -95,6 +95,80 @@ __device__ __forceinline__ const Tables<1024>& tab<1024>() { return c_tab1024; }
 template <>
 __device__ __forceinline__ const Tables<512>& tab<512>() { return c_tab512; }
 
+// ---- exact FP32 arithmetic mod q for the fused kernels' transforms --------------------
+// Values are integers in floats, twiddles plain (no Montgomery factor) and centred
+// (|z| <= 6144).  x z is formed exactly inside v_fma_f32 and reduced by k = round(x z / q)
+// in two exact steps, q = 3 2^12 + 1: x z - 12288 k = r + k, then minus k.  With |x z| / q
+// <= 2^21, 12288 k = 3 k 2^12 and r + k (below 2^24) are exact, and z / q's rounding moves
+// k by at most 2^21 2^-23 = 1/4: |r| < 0.76 q.  Five full-rate instructions; the integer
+// Montgomery product is three 32-bit multiplies at half that rate and five more.
+namespace fp {
+constexpr float kQ = 12289.0f, kQinv = 1.0f / 12289.0f, kM = 12582912.0f;  // kM = 1.5 2^23
+
+// zq = z kQinv
+__device__ __forceinline__ float mul(float x, float z, float zq) {
+  const float k = __builtin_fmaf(x, zq, kM) - kM;
+  return __builtin_fmaf(x, z, k * -12288.0f) - k;
+}
+__device__ __forceinline__ float mul(float x, float z) { return mul(x, z, z * kQinv); }
+// centred residue of |x| <= 2^24
+__device__ __forceinline__ float reduce(float x) {
+  const float k = __builtin_fmaf(x, kQinv, kM) - kM;
+  return __builtin_fmaf(k, -kQ, x);
+}
+// the residue in [0, q) as an integer, |x| <= 2^19: k = floor(x / q) as the rounding of
+// x / q - 1/2 + 1 / (2 q), whose margin 1 / (2 q) exceeds the float error 2^-18
+__device__ __forceinline__ uint32_t canon(float x) {
+  const float k = (__builtin_fmaf(x, kQinv, -0.5f + 0.5f / kQ) + kM) - kM;
+  return __builtin_bit_cast(uint32_t, __builtin_fmaf(k, -kQ, x + kM)) & 0x3FFFu;
+}
+}  // namespace fp
+
+// Plain centred twiddles of the bit-reversed-input, natural-output transforms whose layer
+// L combines sub-transforms of 2^L points: entry 2^L + j belongs to output j of that layer.
+// fwd holds g^((2 j + 1) N / 2^(L+1)): the products of the reference's gammas that its
+// mul_coefficients and its layers apply one after another, as the powers they amount to.
+// inv is the cyclic inverse's g^(-2 j N / 2^(L+1)), post its output scale g^-c / N.
+template <int N>
+constexpr float twiddle(bool inv, int L, int j) {
+  const uint32_t e = (uint32_t)(N >> (L + 1)) * (uint32_t)(inv ? 2 * N - 2 * j : 2 * j + 1);
+  const uint32_t v = powmod(Par<N>::G, e % (2 * N));
+  return v > Q / 2 ? (float)((int)v - (int)Q) : (float)v;
+}
+
+template <int N>
+struct alignas(16) TablesF {
+  float fwd[N], inv[N], post[N];
+};
+
+template <int N>
+constexpr TablesF<N> make_tables_f() {
+  TablesF<N> t{};
+  for (int L = 0; L < Par<N>::LOG; L++)
+    for (int j = 0; j < (1 << L); j++) {
+      t.fwd[(1 << L) + j] = twiddle<N>(false, L, j);
+      t.inv[(1 << L) + j] = twiddle<N>(true, L, j);
+    }
+  const uint32_t ginv = powmod(Par<N>::G, Q - 2);
+  uint32_t po = powmod(N, Q - 2);
+  for (uint32_t k = 0; k < N; k++) {
+    t.post[k] = po > Q / 2 ? (float)((int)po - (int)Q) : (float)po;
+    po = (uint32_t)((uint64_t)po * ginv % Q);
+  }
+  return t;
+}
+
+__device__ const TablesF<1024> c_tabf1024 = make_tables_f<1024>();
+__device__ const TablesF<512> c_tabf512 = make_tables_f<512>();
+
+template <int N>
+__device__ __forceinline__ const TablesF<N>& tabf() {
+  if constexpr (N == 1024)
+    return c_tabf1024;
+  else
+    return c_tabf512;
+}
+
 // floor(n / q) for n < 2^21: the high word of the 24-bit product n m with
 // m = ceil(2^32 / q), one v_mul_hi_u32_u24 where the compiler's division by a
 // constant takes five instructions.  Exact: n m / 2^32 = n / q + n e / (q 2^32)
@@ -609,13 +683,14 @@ __global__ void k_tomsg(int n, uint8_t* msg, size_t msg_stride, Pv<N> p) {
 // Keypair, encryption and decryption each as one kernel.  The element's SHAKE
 // streams run on the wave's lanes (one stream per lane), its polynomials stay in
 // LDS or in VGPRs in ntt_wave's output layout, and HBM sees only the element's
-// inputs and outputs.  Every value is produced by the same operations, in the
-// same order and with the same 16-bit storage points as the per-operation
-// kernels above, so both paths give identical outputs.
+// inputs and outputs.  The per-operation kernels above keep representatives below
+// 2^16 of the residues mod q and lose none of them, these hold residues exactly in FP32,
+// and every output is a function of residues alone: both paths give identical bytes.
 
-// gen_a rows in LDS: 64 coefficients of one stream, padded to 66 so that the
-// lanes' scattered accept stores fall on different banks
-constexpr int kArow = 66;
+// gen_a rows in LDS: 64 coefficients of one stream and the sampler's 4 spare slots, an odd
+// number of words so that the lanes' stores fall on different banks
+constexpr int kArow = 70;
+static_assert(kArow >= 68 && kArow % 4 == 2, "spare slots, odd word count");
 
 __device__ __forceinline__ int arow_index(int c) { return (c >> 6) * kArow + (c & 63); }
 
@@ -624,21 +699,165 @@ __device__ __forceinline__ int brv_index(int c) {
   return (int)(__builtin_bitreverse32((uint32_t)c) >> (32 - Par<N>::LOG));
 }
 
+// The fused kernels' transforms on FP32 values, in ntt_wave's register layouts, the
+// exchanges between its register groups through an LDS buffer of floats.  Butterflies
+// multiply first (a + z b, a - z b): a layer adds 0.76 q to the bound, so nothing is
+// reduced on the way (2^14 + 10 0.76 q < 2^17), the weighting of the input is part of the
+// twiddles, those of the first register group are literals and the others serve several
+// butterflies, two polynomials at a time where there are two.  All of these kernels are
+// bound by VALU issue (a wave's Keccak-f is 4320 of its ~7000 instructions).  Keypair,
+// encryption and decryption of 16384 elements at N = 1024, us: 180, 215 and 50 with integer
+// Montgomery layers and a branch per gen_a candidate; 160, 175 and 42 with these transforms
+// and the branch-free sampler; keypair 136 with four elements per workgroup (below).
+template <int N>
+constexpr int kFxWords = N + N / 16;  // index i at i + i / 16: an exchange's lanes on different banks
+__device__ __forceinline__ int fx(int i) { return i + (i >> 4); }
+
+template <int R>
+__device__ __forceinline__ void reduce_all(float (&v)[R]) {
+#pragma unroll
+  for (int r = 0; r < R; ++r) v[r] = fp::reduce(v[r]);
+}
+
+// layer L < log2(N / 64) on index (N / 64) l + r: the twiddle depends on r alone
+template <int N, bool INV, int L, int P, int R = 0>
+__device__ __forceinline__ void layer_low(float (&v)[P][N / 64]) {
+  if constexpr (R < N / 64) {
+    if constexpr ((R & (1 << L)) == 0) {
+      constexpr float z = twiddle<N>(INV, L, R & ((1 << L) - 1));
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const float t = z == 1.0f ? v[p][R + (1 << L)] : fp::mul(v[p][R + (1 << L)], z, z * fp::kQinv);
+        v[p][R + (1 << L)] = v[p][R] - t;
+        v[p][R] += t;
+      }
+    }
+    layer_low<N, INV, L, P, R + 1>(v);
+  }
+}
+
+// layer L on index idx(r), whose bit L is register bit RB
+template <int L, int RB, int P, int R, typename IDX>
+__device__ __forceinline__ void layer_f(float (&v)[P][R], const float* __restrict__ tab, IDX idx) {
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (r & (1 << RB)) continue;
+    const float z = tab[(1 << L) + (idx(r) & ((1 << L) - 1))], zq = z * fp::kQinv;
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const float t = fp::mul(v[p][r + (1 << RB)], z, zq);
+      v[p][r + (1 << RB)] = v[p][r] - t;
+      v[p][r] += t;
+    }
+  }
+}
+
+// orders one wave's LDS accesses: the wave's own are executed in program order, so only
+// the compiler has to keep it
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// registers from index from(r) to index to(r), one polynomial after the other through buf
+// (free before and after)
+template <int P, int R, typename FROM, typename TO>
+__device__ __forceinline__ void exchange(float (&v)[P][R], float* buf, FROM from, TO to) {
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) buf[fx(from(r))] = v[p][r];
+    wave_sync();
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[p][r] = buf[fx(to(r))];
+    wave_sync();
+  }
+}
+
+// P polynomials, v[p][r] = input index (N / 64) l + r -> v[p][r] = output coefficient
+// out_index(l, r); buf is free before and after
+template <int N, bool INV, int P>
+__device__ __forceinline__ void transform_f(float (&v)[P][N / 64], float* buf, int l) {
+  constexpr int C = N / 64;
+  const float* tab = INV ? tabf<N>().inv : tabf<N>().fwd;
+  auto ia = [l](int r) { return C * l + r; };
+  auto ib = [l](int r) { return (l & (C - 1)) + C * r + C * C * (l / C); };
+  auto ic = [l](int r) { return out_index<N>(l, r); };
+  layer_low<N, INV, 0>(v);
+  layer_low<N, INV, 1>(v);
+  layer_low<N, INV, 2>(v);
+  if constexpr (N == 1024) layer_low<N, INV, 3>(v);
+  exchange(v, buf, ia, ib);
+  if constexpr (N == 1024) {
+    layer_f<4, 0>(v, tab, ib);
+    layer_f<5, 1>(v, tab, ib);
+    layer_f<6, 2>(v, tab, ib);
+    layer_f<7, 3>(v, tab, ib);
+  } else {
+    layer_f<3, 0>(v, tab, ib);
+    layer_f<4, 1>(v, tab, ib);
+    layer_f<5, 2>(v, tab, ib);
+  }
+  exchange(v, buf, ib, ic);
+  if constexpr (N == 1024) {
+    layer_f<8, 2>(v, tab, ic);
+    layer_f<9, 3>(v, tab, ic);
+  } else {
+    layer_f<6, 0>(v, tab, ic);
+    layer_f<7, 1>(v, tab, ic);
+    layer_f<8, 2>(v, tab, ic);
+  }
+}
+
+// poly_ntt's input registers from the natural-order polynomial in sm
+template <int N>
+__device__ __forceinline__ void load_ntt(float (&v)[N / 64], const uint16_t* sm, int l) {
+  constexpr int C = N / 64;
+  const uint4* p = reinterpret_cast<const uint4*>(sm + C * l);
+#pragma unroll
+  for (int h = 0; h < C / 8; ++h) {
+    const uint4 a = p[h];
+    const uint32_t aw[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[8 * h + 2 * k] = (float)(aw[k] & 0xFFFFu);
+      v[8 * h + 2 * k + 1] = (float)(aw[k] >> 16);
+    }
+  }
+}
+
+// poly_invntt of v[0][r] = coefficient out_index(l, r), |v| <= 2^14, in place
+template <int N>
+__device__ __forceinline__ void invntt_f(float (&v)[1][N / 64], float* buf, int l) {
+  wave_sync();
+  exchange(v, buf, [l](int r) { return brv_index<N>(out_index<N>(l, r)); }, [l](int r) { return (N / 64) * l + r; });
+  transform_f<N, true>(v, buf, l);
+#pragma unroll
+  for (int r = 0; r < N / 64; ++r) v[0][r] = fp::mul(v[0][r], tabf<N>().post[out_index<N>(l, r)]);
+}
+
+// canonical residues to a natural-order uint16 polynomial
+template <int N>
+__device__ __forceinline__ void put_nat_f(uint16_t* sm, const float (&v)[N / 64], int l) {
+#pragma unroll
+  for (int r = 0; r < N / 64; ++r) sm[out_index<N>(l, r)] = (uint16_t)fp::canon(v[r]);
+}
+
 // One SHAKE stream on this lane: gen_a stream i (SHAKE128(seed || i), 16-bit
 // candidates < 5q kept unreduced, poly.cu:332-366) when `uniform`, else
 // poly_sample stream i (SHAKE256(seed || nonce || i, 128 bytes), hw(a) + q -
-// hw(b), poly.cu:396-444).  Writes the stream's 64 coefficients to row[0..63].
+// hw(b), poly.cu:396-444).  Writes the stream's 64 coefficients to sm[off .. off + 63].
 // Lanes that take no part pass active = false; every lane of the wave reaches
 // the block loop's vote.
-__device__ __forceinline__ void lane_stream(uint16_t* row, const uint64_t (&seed)[4], bool active, bool uniform,
-                                            int nonce, int i) {
+__device__ __forceinline__ void lane_stream(uint16_t* sm, uint32_t off, const uint64_t (&seed)[4], bool active,
+                                            bool uniform, int nonce, int i) {
   uint64_t A[25];
 #pragma unroll
   for (int w = 0; w < 25; ++w) A[w] = w < 4 ? seed[w] : 0;
   A[4] = uniform ? ((uint64_t)i | (0x1Full << 8)) : ((uint64_t)nonce | ((uint64_t)i << 8) | (0x1Full << 16));
   A[kRateShake128 - 1] ^= uniform ? 0x8000000000000000ull : 0;
   A[kRateShake256 - 1] ^= uniform ? 0 : 0x8000000000000000ull;
-  keccakf1600(A);
+  keccakf1600_two(A);
   if (active && !uniform) {
 #pragma unroll
     for (int w = 0; w < 16; w += 2) {
@@ -646,73 +865,39 @@ __device__ __forceinline__ void lane_stream(uint16_t* row, const uint64_t (&seed
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const uint64_t word = A[w + (k >> 1)];
-        const uint32_t ab0 = (uint32_t)(word >> (32 * (k & 1))) & 0xFFFFu;
-        const uint32_t ab1 = (uint32_t)(word >> (32 * (k & 1) + 16)) & 0xFFFFu;
-        const uint32_t c0 = (__popc(ab0 & 0xFF) + Q - __popc(ab0 >> 8)) & 0xFFFFu;
-        const uint32_t c1 = (__popc(ab1 & 0xFF) + Q - __popc(ab1 >> 8)) & 0xFFFFu;
+        const uint32_t ab = (uint32_t)(word >> (32 * (k & 1)));
+        const uint32_t c0 = __popc(ab & 0xFF) + Q - __popc(ab & 0xFF00);
+        const uint32_t c1 = __popc(ab & 0xFF0000) + Q - __popc(ab & 0xFF000000);
         o[k] = c0 | (c1 << 16);
       }
-      reinterpret_cast<uint4*>(row)[w >> 1] = make_uint4(o[0], o[1], o[2], o[3]);
+      reinterpret_cast<uint4*>(sm + off)[w >> 1] = make_uint4(o[0], o[1], o[2], o[3]);
     }
   }
-  int ctr = (active && uniform) ? 0 : 64;
+  // branch-free: every candidate is written at the running position, which an accepted one
+  // advances; the position is held at 64 after each word, so a row's slots 64..67 take what
+  // comes after the 64th (a lane without a row has position 64 from the start)
+  const uint32_t end = off + 64;
+  uint32_t pos = (active && uniform) ? off : end;
   for (int blk = 0; blk < 16; ++blk) {
     if (blk > 0) {
-      if (!__any(ctr < 64)) break;
+      if (!__any(pos < end)) break;
       keccakf1600(A);
     }
-    if (ctr < 64) {
+    if (pos < end) {
 #pragma unroll
       for (int w = 0; w < kRateShake128; ++w) {
 #pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          const uint32_t val = (uint32_t)(A[w] >> (16 * h)) & 0xFFFFu;
-          if (val < 5 * Q && ctr < 64) row[ctr++] = (uint16_t)val;
+        for (int h = 0; h < 2; ++h) {  // two candidates per 32-bit half of the word
+          const uint32_t val = (uint32_t)(A[w] >> (32 * h));
+          sm[pos] = (uint16_t)val;
+          pos += val << 16 < (5 * Q) << 16 ? 1 : 0;
+          sm[pos] = (uint16_t)(val >> 16);
+          pos += val < (5 * Q) << 16 ? 1 : 0;
         }
+        pos = pos < end ? pos : end;
       }
     }
   }
-}
-
-// poly_ntt of the natural-order polynomial in sm (clobbered): v[r] = output
-// coefficient out_index(l, r), as k_ntt
-template <int N>
-__device__ __forceinline__ void ntt_lds(uint32_t (&v)[N / 64], uint16_t* sm, int l) {
-  constexpr int C = N / 64;
-  uint4* p = reinterpret_cast<uint4*>(sm + C * l);
-  const uint4* gam = reinterpret_cast<const uint4*>(tab<N>().gammas + C * l);
-#pragma unroll
-  for (int h = 0; h < C / 8; ++h) {
-    const uint4 a = p[h], g = gam[h];
-    const uint32_t aw[4] = {a.x, a.y, a.z, a.w}, gw[4] = {g.x, g.y, g.z, g.w};
-    uint32_t o[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      o[k] = mont((aw[k] & 0xFFFFu) * (gw[k] & 0xFFFFu)) | (mont((aw[k] >> 16) * (gw[k] >> 16)) << 16);
-    p[h] = make_uint4(o[0], o[1], o[2], o[3]);
-  }
-  __syncthreads();
-  ntt_wave(v, sm, l, tab<N>().gammas);
-}
-
-// poly_invntt of the polynomial held as v[r] = coefficient out_index(l, r), in
-// place, through sm (clobbered), as k_invntt
-template <int N>
-__device__ __forceinline__ void invntt_regs(uint32_t (&v)[N / 64], uint16_t* sm, int l) {
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < N / 64; ++r) sm[brv_index<N>(out_index<N>(l, r))] = (uint16_t)v[r];
-  __syncthreads();
-  ntt_wave(v, sm, l, tab<N>().omegas_inv);
-#pragma unroll
-  for (int k = 0; k < N / 64; ++k) v[k] = mont(v[k] * tab<N>().gammas_inv[out_index<N>(l, k)]);
-}
-
-// natural-order LDS polynomial <-> registers in ntt_wave's output layout
-template <int N>
-__device__ __forceinline__ void put_nat(uint16_t* sm, const uint32_t (&v)[N / 64], int l) {
-#pragma unroll
-  for (int r = 0; r < N / 64; ++r) sm[out_index<N>(l, r)] = (uint16_t)v[r];
 }
 
 // poly_frombytes of the 14-bit packing at src (8-byte aligned) into sm in
@@ -734,26 +919,40 @@ __device__ __forceinline__ void unpack14(uint16_t* sm, const uint8_t* src, int l
   }
 }
 
-// poly_tobytes of the natural-order polynomial in sm into LDS bytes bb
+// poly_tobytes of the natural-order polynomial in sm (residues in [0, q)) into LDS bytes
+// bb: lane l packs coefficients (N / 64) l .. (N / 64) (l + 1) - 1 into its 7 N / 256 bytes
 template <int N>
 __device__ __forceinline__ void pack14(uint8_t* bb, const uint16_t* sm, int l) {
+  constexpr int C = N / 64;
+  uint64_t g[C / 4];  // 56 bits of four coefficients each
 #pragma unroll
-  for (int g = l; g < N / 4; g += 64) {
-    const uint2 c = reinterpret_cast<const uint2*>(sm)[g];
-    const uint32_t t0 = freeze(c.x & 0xFFFFu), t1 = freeze(c.x >> 16), t2 = freeze(c.y & 0xFFFFu),
-                   t3 = freeze(c.y >> 16);
-    uint8_t* r = bb + 7 * g;
-    r[0] = (uint8_t)(t0 & 0xff);
-    r[1] = (uint8_t)((t0 >> 8) | (t1 << 6));
-    r[2] = (uint8_t)(t1 >> 2);
-    r[3] = (uint8_t)((t1 >> 10) | (t2 << 4));
-    r[4] = (uint8_t)(t2 >> 4);
-    r[5] = (uint8_t)((t2 >> 12) | (t3 << 2));
-    r[6] = (uint8_t)(t3 >> 6);
+  for (int h = 0; h < C / 4; ++h) {
+    const uint2 c = reinterpret_cast<const uint2*>(sm + C * l)[h];
+    const uint32_t lo = (c.x & 0xFFFFu) | (c.x >> 16 << 14), hi = (c.y & 0xFFFFu) | (c.y >> 16 << 14);
+    g[h] = lo | ((uint64_t)hi << 28);
+  }
+  if constexpr (C == 16) {
+    uint32_t* w = reinterpret_cast<uint32_t*>(bb) + 7 * l;
+    w[0] = (uint32_t)g[0];
+    w[1] = (uint32_t)(g[0] >> 32) | ((uint32_t)g[1] << 24);
+    w[2] = (uint32_t)(g[1] >> 8);
+    w[3] = (uint32_t)(g[1] >> 40) | ((uint32_t)g[2] << 16);
+    w[4] = (uint32_t)(g[2] >> 16);
+    w[5] = (uint32_t)(g[2] >> 48) | ((uint32_t)g[3] << 8);
+    w[6] = (uint32_t)(g[3] >> 24);
+  } else {
+    uint16_t* w = reinterpret_cast<uint16_t*>(bb) + 7 * l;
+    w[0] = (uint16_t)g[0];
+    w[1] = (uint16_t)(g[0] >> 16);
+    w[2] = (uint16_t)(g[0] >> 32);
+    w[3] = (uint16_t)((uint32_t)(g[0] >> 48) | ((uint32_t)g[1] << 8));
+    w[4] = (uint16_t)(g[1] >> 8);
+    w[5] = (uint16_t)(g[1] >> 24);
+    w[6] = (uint16_t)(g[1] >> 40);
   }
 }
 
-// poly_compress of the natural-order polynomial in sm into LDS bytes bb
+// poly_compress of the natural-order polynomial in sm (residues in [0, q)) into LDS bytes bb
 template <int N>
 __device__ __forceinline__ void compress3(uint8_t* bb, const uint16_t* sm, int l) {
 #pragma unroll
@@ -762,7 +961,7 @@ __device__ __forceinline__ void compress3(uint8_t* bb, const uint16_t* sm, int l
     const uint32_t cw[4] = {c.x, c.y, c.z, c.w};
     uint32_t v[8];
 #pragma unroll
-    for (int j = 0; j < 8; j++) v[j] = div_q((freeze((cw[j >> 1] >> (16 * (j & 1))) & 0xFFFFu) << 3) + Q / 2) & 7;
+    for (int j = 0; j < 8; j++) v[j] = div_q((((cw[j >> 1] >> (16 * (j & 1))) & 0xFFFFu) << 3) + Q / 2) & 7;
     uint8_t* r = bb + 3 * g;
     r[0] = (uint8_t)(v[0] | (v[1] << 3) | (v[2] << 6));
     r[1] = (uint8_t)((v[2] >> 2) | (v[3] << 1) | (v[4] << 4) | (v[5] << 7));
@@ -800,122 +999,138 @@ __device__ __forceinline__ void copy_out(uint8_t* dst, const uint8_t* bb, int by
   for (int w = l; w < bytes / 8; w += 64) store_u64(dst + 8 * w, reinterpret_cast<const uint64_t*>(bb)[w]);
 }
 
-// cpapke_keypair (cpapke.cu:265-338) for element blockIdx.x, from z =
-// publicseed || noiseseed = SHAKE256(seed, 64) at z + 64 x (k_seed_expand: the
-// one serial permutation stays on one lane per element).  Lanes 0..S-1 run the
-// gen_a streams, S..2S-1 the streams of s (nonce 0), 2S..3S-1 those of e
-// (nonce 1); S = N / 64.
-template <int N>
-__global__ __launch_bounds__(64) void k_keypair_fused(int n, uint8_t* pk, uint8_t* sk, size_t sk_stride,
-                                                      const uint8_t* z) {
-  using P = Par<N>;
-  constexpr int C = N / 64, S = P::STREAMS;
-  __shared__ __align__(16) uint16_t sa[S * kArow];
-  __shared__ __align__(16) uint16_t ss[N];
-  __shared__ __align__(16) uint16_t se[N];
-  const int x = blockIdx.x, l = threadIdx.x;
-  if (x >= n) return;
-  const uint8_t* zx = z + (size_t)x * 64;
-  {
-    const int kind = l / S, i = l % S;
-    const bool pub = kind == 0;
-    uint64_t sd[4];
-#pragma unroll
-    for (int w = 0; w < 4; ++w) sd[w] = load_u64(zx + (pub ? 0 : 32) + 8 * w);
-    uint16_t* row = pub ? sa + i * kArow : (kind == 1 ? ss : se) + 64 * i;
-    lane_stream(row, sd, kind < 3, pub, kind - 1, i);
-  }
-  __syncthreads();
-  uint32_t vs[C], vb[C];
-  ntt_lds<N>(vs, ss, l);
-  ntt_lds<N>(vb, se, l);
-  // b = e + s o a (k_pointwise(AS, SHAT, AHAT), k_addsub(BHAT, EHAT, AS))
-#pragma unroll
-  for (int r = 0; r < C; ++r) {
-    const uint32_t ahat = sa[arow_index(out_index<N>(l, r))];
-    vb[r] = mod_q(vb[r] + mont(vs[r] * mont(3186u * ahat)));
-  }
-  __syncthreads();
-  put_nat<N>(ss, vs, l);
-  put_nat<N>(se, vb, l);
-  __syncthreads();
-  pack14<N>(reinterpret_cast<uint8_t*>(sa), ss, l);
-  __syncthreads();
-  copy_out(sk + (size_t)x * sk_stride, reinterpret_cast<const uint8_t*>(sa), P::POLYBYTES, l);
-  __syncthreads();
-  pack14<N>(reinterpret_cast<uint8_t*>(sa), se, l);
-  __syncthreads();
-  uint8_t* pkx = pk + (size_t)x * P::PK;
-  copy_out(pkx, reinterpret_cast<const uint8_t*>(sa), P::POLYBYTES, l);
-  if (l < 4) store_u64(pkx + P::POLYBYTES + 8 * l, load_u64(zx + 8 * l));
-}
+// Keypair and encryption run in workgroups of four waves, four elements.  A wave's
+// transforms are its own element's; the SHAKE streams of the four lie side by side on the
+// workgroup's lanes, ordered by kind, so that a wave's lanes are all in use (alone, an
+// element fills 48 or 64 of them at N = 1024, 24 or 32 at N = 512) and only the waves that
+// hold gen_a streams step through its candidates.  The waves left without streams rotate
+// with the workgroup, whose waves sit on the same SIMDs each time.
+constexpr int kElems = 4;
 
-// cpapke_enc (cpapke.cu:353-429) for element blockIdx.x.  Lanes 0..S-1 run the
-// gen_a streams of the public seed, S..4S-1 the streams of s', e', e'' (coin,
-// nonces 0, 1, 2).
-template <int N>
-__global__ __launch_bounds__(64) void k_enc_fused(int n, uint8_t* ct, size_t ct_stride, const uint8_t* m,
-                                                  size_t m_stride, const uint8_t* pk, size_t pk_stride,
-                                                  const uint8_t* coin, size_t coin_stride) {
-  using P = Par<N>;
-  constexpr int C = N / 64, S = P::STREAMS;
-  __shared__ __align__(16) uint16_t sa[S * kArow];
-  __shared__ __align__(16) uint16_t s1[N];
-  __shared__ __align__(16) uint16_t s2[N];
-  __shared__ __align__(16) uint16_t s3[N];
-  const int x = blockIdx.x, l = threadIdx.x;
-  if (x >= n) return;
-  const uint8_t* pkx = pk + (size_t)x * pk_stride;
-  {
-    const int kind = l / S, i = l % S;
-    const bool pub = kind == 0;
-    const uint8_t* src = pub ? pkx + P::POLYBYTES : coin + (size_t)x * coin_stride;
+// Runs the workgroup's streams: stream t is stream i of kind `kind` (0 gen_a, then the
+// KINDS - 1 nonces) of element el, whose coefficients go to sm[el ES + off(kind, i)];
+// seed(x, kind) is its seed.  Elements past n take part with the last one's seed and write
+// nothing.
+template <int N, int KINDS, int ES, typename SEED, typename OFF>
+__device__ __forceinline__ void run_streams(uint16_t* sm, int n, SEED seed, OFF off) {
+  constexpr int S = Par<N>::STREAMS, T = kElems * S * KINDS;
+  const int t = (threadIdx.x + 64 * (blockIdx.x % kElems)) % (64 * kElems);
+  if ((t & ~63) < T) {
+    const int kind = t / (kElems * S), el = t / S % kElems, i = t % S;
+    const int x = (int)blockIdx.x * kElems + el;
+    const uint8_t* src = seed(x < n ? x : n - 1, kind < KINDS ? kind : 0);
     uint64_t sd[4];
 #pragma unroll
     for (int w = 0; w < 4; ++w) sd[w] = load_u64(src + 8 * w);
-    uint16_t* row = pub ? sa + i * kArow : (kind == 1 ? s1 : kind == 2 ? s2 : s3) + 64 * i;
-    lane_stream(row, sd, kind < 4, pub, kind - 1, i);
+    lane_stream(sm, (uint32_t)(el * ES + off(kind, i)), sd, t < T && x < n, kind == 0, kind - 1, i);
   }
   __syncthreads();
-  uint32_t vsp[C], vv[C];
-  ntt_lds<N>(vsp, s1, l);
+}
+
+// cpapke_keypair (cpapke.cu:265-338) for element kElems blockIdx.x + wave, from z =
+// publicseed || noiseseed = SHAKE256(seed, 64) at z + 64 x (k_seed_expand: the one serial
+// permutation stays on one lane per element).  Streams: gen_a, s (nonce 0), e (nonce 1).
+template <int N>
+__global__ __launch_bounds__(64 * kElems, 4) void k_keypair_fused(int n, uint8_t* pk, uint8_t* sk, size_t sk_stride,
+                                                                  const uint8_t* z) {
+  using P = Par<N>;
+  constexpr int C = N / 64, S = P::STREAMS;
+  // per element: gen_a rows | s | e; the transforms' buffer lies over s and e
+  constexpr int ES = S * kArow + 2 * kFxWords<N>;
+  static_assert(S * kArow % 8 == 0 && ES % 8 == 0, "16-byte rows");
+  __shared__ __align__(16) uint16_t sm[kElems * ES];
+  run_streams<N, 3, ES>(
+      sm, n, [z](int x, int kind) { return z + (size_t)x * 64 + (kind ? 32 : 0); },
+      [](int kind, int i) { return kind ? S * kArow + N * (kind - 1) + 64 * i : kArow * i; });
+  const int l = threadIdx.x & 63, el = threadIdx.x >> 6, x = (int)blockIdx.x * kElems + el;
+  if (x >= n) return;
+  uint16_t *const sa = sm + el * ES, *const ss = sa + S * kArow, *const se = ss + N;
+  float* const buf = reinterpret_cast<float*>(ss);
+  float v[2][C];  // s, then e + s o a
+  load_ntt<N>(v[0], ss, l);
+  load_ntt<N>(v[1], se, l);
+  wave_sync();
+  transform_f<N, false>(v, buf, l);
+  reduce_all(v[0]);
+  // b = e + s o a (k_pointwise(AS, SHAT, AHAT), k_addsub(BHAT, EHAT, AS))
+#pragma unroll
+  for (int r = 0; r < C; ++r) v[1][r] += fp::mul((float)sa[arow_index(out_index<N>(l, r))], v[0][r]);
+  put_nat_f<N>(ss, v[0], l);
+  put_nat_f<N>(se, v[1], l);
+  wave_sync();
+  uint8_t* const bb = reinterpret_cast<uint8_t*>(sa);
+  pack14<N>(bb, ss, l);
+  wave_sync();
+  copy_out(sk + (size_t)x * sk_stride, bb, P::POLYBYTES, l);
+  wave_sync();
+  pack14<N>(bb, se, l);
+  wave_sync();
+  uint8_t* pkx = pk + (size_t)x * P::PK;
+  copy_out(pkx, bb, P::POLYBYTES, l);
+  if (l < 4) store_u64(pkx + P::POLYBYTES + 8 * l, load_u64(z + (size_t)x * 64 + 8 * l));
+}
+
+// cpapke_enc (cpapke.cu:353-429) for element kElems blockIdx.x + wave.  Streams: gen_a of
+// the public seed, then s', e', e'' (coin, nonces 0, 1, 2).
+template <int N>
+__global__ __launch_bounds__(64 * kElems, 4) void k_enc_fused(int n, uint8_t* ct, size_t ct_stride, const uint8_t* m,
+                                                              size_t m_stride, const uint8_t* pk, size_t pk_stride,
+                                                              const uint8_t* coin, size_t coin_stride) {
+  using P = Par<N>;
+  constexpr int C = N / 64, S = P::STREAMS;
+  // per element: gen_a rows | e'' | s' | e'; the transforms' buffer lies over s' and e'
+  constexpr int ES = S * kArow + N + 2 * kFxWords<N>;
+  static_assert(S * kArow % 8 == 0 && ES % 8 == 0, "16-byte rows");
+  __shared__ __align__(16) uint16_t sm[kElems * ES];
+  run_streams<N, 4, ES>(
+      sm, n,
+      [=](int x, int kind) {
+        return kind ? coin + (size_t)x * coin_stride : pk + (size_t)x * pk_stride + P::POLYBYTES;
+      },
+      [](int kind, int i) { return kind ? S * kArow + N * (kind % 3) + 64 * i : kArow * i; });
+  const int l = threadIdx.x & 63, el = threadIdx.x >> 6, x = (int)blockIdx.x * kElems + el;
+  if (x >= n) return;
+  uint16_t *const sa = sm + el * ES, *const s3 = sa + S * kArow, *const s1 = s3 + N, *const s2 = s1 + N;
+  float* const buf = reinterpret_cast<float*>(s1);
+  float vv[1][C];
   {
     // u = a o s' + e' (k_pointwise(UHAT, AHAT, SP), k_addsub(UHAT, UHAT, EP)),
     // parked in natural order over the gen_a rows once every lane has read them
-    uint32_t vu[C];
-    ntt_lds<N>(vu, s2, l);
+    float v[2][C];  // s', then u
+    load_ntt<N>(v[0], s1, l);
+    load_ntt<N>(v[1], s2, l);
+    wave_sync();
+    transform_f<N, false>(v, buf, l);
+    reduce_all(v[0]);
 #pragma unroll
-    for (int r = 0; r < C; ++r) {
-      const uint32_t ahat = sa[arow_index(out_index<N>(l, r))];
-      vu[r] = mod_q(mont(ahat * mont(3186u * vsp[r])) + vu[r]);
-    }
-    __syncthreads();
-    put_nat<N>(sa, vu, l);
+    for (int r = 0; r < C; ++r) v[1][r] += fp::mul((float)sa[arow_index(out_index<N>(l, r))], v[0][r]);
+    wave_sync();
+    put_nat_f<N>(sa, v[1], l);
+    unpack14<N>(s1, pk + (size_t)x * pk_stride, l);  // b (decode_pk)
+    wave_sync();
+    // v' = invntt(b o s') (k_pointwise(VP, BHAT, SP), k_invntt)
+#pragma unroll
+    for (int r = 0; r < C; ++r) vv[0][r] = fp::mul((float)s1[out_index<N>(l, r)], v[0][r]);
   }
-  unpack14<N>(s1, pkx, l);  // b (decode_pk)
-  __syncthreads();
-  // v' = invntt(b o s') (k_pointwise(VP, BHAT, SP), k_invntt)
-#pragma unroll
-  for (int r = 0; r < C; ++r) vv[r] = mont((uint32_t)s1[out_index<N>(l, r)] * mont(3186u * vsp[r]));
-  invntt_regs<N>(vv, s2, l);
+  invntt_f<N>(vv, buf, l);
   // v = v' + e'' + frommsg(m) (k_addsub twice, k_frommsg)
-  uint64_t mw[4];
+  // Coefficient c takes message bit c mod 256: at N = 1024 a lane's bits are one nibble
+  const uint8_t* mx = m + (size_t)x * m_stride;
+  uint64_t mw[N == 1024 ? 1 : 4];
 #pragma unroll
-  for (int w = 0; w < 4; ++w) mw[w] = load_u64(m + (size_t)x * m_stride + 8 * w);
+  for (int w = 0; w < (N == 1024 ? 1 : 4); ++w) mw[w] = load_u64(mx + 8 * (N == 1024 ? l >> 4 : w));
 #pragma unroll
   for (int r = 0; r < C; ++r) {
-    const int c = out_index<N>(l, r), b = c & 255;
-    const uint64_t word = (b >> 6) == 0 ? mw[0] : (b >> 6) == 1 ? mw[1] : (b >> 6) == 2 ? mw[2] : mw[3];
-    const uint32_t bit = (uint32_t)(word >> (b & 63)) & 1u;
-    const uint32_t t = mod_q(vv[r] + s3[c]);
-    vv[r] = mod_q(t + ((0u - bit) & (Q / 2)));
+    const int c = out_index<N>(l, r);
+    const uint32_t bit = (uint32_t)(N == 1024 ? mw[0] >> (4 * (l & 15) + (r & 3)) : mw[r & 3] >> l) & 1u;
+    vv[0][r] += (float)(s3[c] + ((0u - bit) & (Q / 2)));
   }
-  __syncthreads();
-  put_nat<N>(s3, vv, l);
-  __syncthreads();
+  wave_sync();
+  put_nat_f<N>(s3, vv[0], l);
+  wave_sync();
   pack14<N>(reinterpret_cast<uint8_t*>(s2), sa, l);
   compress3<N>(reinterpret_cast<uint8_t*>(s1), s3, l);
-  __syncthreads();
+  wave_sync();
   uint8_t* ctx_ = ct + (size_t)x * ct_stride;
   copy_out(ctx_, reinterpret_cast<const uint8_t*>(s2), P::POLYBYTES, l);
   copy_out(ctx_ + P::POLYBYTES, reinterpret_cast<const uint8_t*>(s1), P::CBYTES, l);
@@ -927,9 +1142,9 @@ __global__ __launch_bounds__(64) void k_dec_fused(int n, uint8_t* m, size_t m_st
                                                   size_t ct_stride, const uint8_t* sk, size_t sk_stride) {
   using P = Par<N>;
   constexpr int C = N / 64;
-  __shared__ __align__(16) uint16_t s1[N];
-  __shared__ __align__(16) uint16_t s2[N];
+  __shared__ __align__(16) float buf[kFxWords<N>];  // over s1 and s2
   __shared__ __align__(16) uint16_t s3[N];
+  uint16_t *const s1 = reinterpret_cast<uint16_t*>(buf), *const s2 = s1 + N;
   const int x = blockIdx.x, l = threadIdx.x;
   if (x >= n) return;
   const uint8_t* ctx_ = ct + (size_t)x * ct_stride;
@@ -938,17 +1153,17 @@ __global__ __launch_bounds__(64) void k_dec_fused(int n, uint8_t* m, size_t m_st
   decompress3<N>(s3, ctx_ + P::POLYBYTES, l);
   __syncthreads();
   // tmp = invntt(s o u) - v (k_pointwise(TMP, SHAT, UHAT), k_invntt, k_addsub(TMP, TMP, VP, 1))
-  uint32_t vt[C];
+  float vt[1][C];
 #pragma unroll
   for (int r = 0; r < C; ++r) {
     const int c = out_index<N>(l, r);
-    vt[r] = mont((uint32_t)s1[c] * mont(3186u * (uint32_t)s2[c]));
+    vt[0][r] = fp::mul((float)s1[c], (float)s2[c]);
   }
-  invntt_regs<N>(vt, s1, l);
+  invntt_f<N>(vt, buf, l);
 #pragma unroll
-  for (int r = 0; r < C; ++r) vt[r] = mod_q(vt[r] + 3 * Q - (uint32_t)s3[out_index<N>(l, r)]);
+  for (int r = 0; r < C; ++r) vt[0][r] -= (float)s3[out_index<N>(l, r)];
   __syncthreads();
-  put_nat<N>(s2, vt, l);
+  put_nat_f<N>(s2, vt[0], l);
   __syncthreads();
   // poly_tomsg: byte i from the N / 256 copies of coefficients 8 i + j
   if (l < 32) {
@@ -1061,6 +1276,7 @@ struct Launch {
   int block;
   dim3 grid(size_t threads) const { return dim3((unsigned)((threads + block - 1) / block)); }
 };
+inline dim3 elem_grid(int n) { return dim3((unsigned)((n + kElems - 1) / kElems)); }
 #define LAUNCH(kern, threads, ...) hipLaunchKernelGGL(kern, L.grid(threads), dim3(L.block), 0, s, __VA_ARGS__)
 #define LAUNCH_NTT(kern, ...) hipLaunchKernelGGL(kern, dim3(n), dim3(64), 0, s, __VA_ARGS__)
 
@@ -1073,7 +1289,7 @@ int keypair_impl(pqc_ctx* c, int n, uint8_t* pk, uint8_t* sk, size_t sk_stride, 
   if (!plain) {
     const size_t n1 = n;
     LAUNCH(k_seed_expand, n1, n, c->nhbytes, seed, seed_stride);
-    hipLaunchKernelGGL(k_keypair_fused<N>, dim3((unsigned)n), dim3(64), 0, s, n, pk, sk, sk_stride,
+    hipLaunchKernelGGL(k_keypair_fused<N>, elem_grid(n), dim3(64 * kElems), 0, s, n, pk, sk, sk_stride,
                        (const uint8_t*)c->nhbytes);
     return hip_err(hipGetLastError());
   }
@@ -1100,7 +1316,7 @@ template <int N>
 int enc_impl(pqc_ctx* c, int n, uint8_t* ct, size_t ct_stride, const uint8_t* m, size_t m_stride, const uint8_t* pk,
              size_t pk_stride, const uint8_t* coin, size_t coin_stride, bool plain, hipStream_t s) {
   if (!plain) {
-    hipLaunchKernelGGL(k_enc_fused<N>, dim3((unsigned)n), dim3(64), 0, s, n, ct, ct_stride, m, m_stride, pk, pk_stride,
+    hipLaunchKernelGGL(k_enc_fused<N>, elem_grid(n), dim3(64 * kElems), 0, s, n, ct, ct_stride, m, m_stride, pk, pk_stride,
                        coin, coin_stride);
     return hip_err(hipGetLastError());
   }
