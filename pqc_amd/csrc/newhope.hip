@@ -20,6 +20,7 @@
 // (precomp.cu:75-190 tables, ntt.cu:130-180, poly.cu:244,279), which its
 // batched GPU path never compiled.
 #include "internal.h"
+#include "keccak_wide.cuh"
 #include "sponge.cuh"
 
 namespace pqc {
@@ -1263,6 +1264,138 @@ __global__ void k_cmov32(int n, uint8_t* k, size_t k_stride, const uint8_t* z, s
   store_u64(pk, (load_u64(pk) & ~mask) | (load_u64(z + x * z_stride + 8 * w) & mask));
 }
 
+// Per-element CCA scratch row (one size for both N): mu or m' | H(pk) |
+// K || coin || d | H(c) | fail | re-encrypted ct
+constexpr int KM_MU = 0, KM_HPK = 32, KM_KCD = 64, KM_HC = 160, KM_FAIL = 192, KM_CT2 = 224;
+static_assert(KM_CT2 + Par<1024>::CCA_CT == kNewhopeKemBytes, "scratch row size");
+
+// ---- the CCA-KEM's hashes on 16 lanes per element (keccak_wide.cuh) ----------------
+// Up to kWideMax elements the sponges above are serial chains on a few waves, and every
+// step between two of them is a launch of its own.  Here four elements share a wave, and
+// the copies, the comparison and the selection belong to the kernel that hashes next to
+// them.  One encapsulation and decapsulation per element, us, lane-pair form -> this one:
+// N = 512: 308 -> 141 (7 elements), 325 -> 189 (3001), 368 -> 292 (8192), 490 -> 548
+// (16384: the pair form's 512 waves are still one per SIMD, these would be four);
+// N = 1024: 506 -> 211, 533 -> 286, 585 -> 456, 753 -> 905.
+constexpr int kWideMax = 8192;
+
+struct Wide4 {
+  wide::Consts consts;
+  wide::States states;
+  alignas(16) uint32_t dig[4][16];  // per element: the words of its next short message
+};
+
+// out[x] = SHAKE256(in[x], 8 words bytes), 32 bytes
+template <int W>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_shake256_wide(int n, uint8_t* out, size_t out_stride,
+                                                                        const uint8_t* in, size_t in_stride,
+                                                                        int words) {
+  __shared__ Wide4 sh;
+  wide::init_consts(sh.consts);
+  __syncthreads();
+  wide::Sponge s;
+  s.init(sh.states, sh.consts);
+  const int rq = 4 * blockIdx.x + s.st, r = rq < n ? rq : n - 1;
+  s.absorb17<24>(reinterpret_cast<const uint32_t*>(in + (size_t)r * in_stride), words, 0x1F, 0, words / 17 + 1);
+  uint32_t* o = reinterpret_cast<uint32_t*>(out + (size_t)r * out_stride);
+  s.squeeze<4>([&](int x, uint32_t v) {
+    if (rq < n && s.y == 0) o[2 * x + s.h] = v;
+  });
+}
+
+// (K || coin || d) = SHAKE256(mu || H(pk), 96).  Encapsulation (ENC): mu = H(in[x], 32
+// bytes), kept in the row, and H(pk) of the public key key[x] (words 64-bit words);
+// decapsulation: m' of the row and the H(pk) that key[x] holds.
+template <int W, bool ENC>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_cca_open_wide(int n, uint8_t* km, const uint8_t* in,
+                                                                        const uint8_t* key, size_t key_stride,
+                                                                        int words) {
+  __shared__ Wide4 sh;
+  wide::init_consts(sh.consts);
+  __syncthreads();
+  wide::Sponge s;
+  s.init(sh.states, sh.consts);
+  const int rq = 4 * blockIdx.x + s.st, r = rq < n ? rq : n - 1;
+  const bool act = rq < n;
+  uint32_t* row = reinterpret_cast<uint32_t*>(km + (size_t)r * kNewhopeKemBytes);
+  const uint32_t* kp = reinterpret_cast<const uint32_t*>(key + (size_t)r * key_stride);
+  uint32_t* dig = sh.dig[s.st];
+  if constexpr (ENC) {
+    s.absorb17(reinterpret_cast<const uint32_t*>(in + (size_t)r * 32), 4, 0x1F, 0, 1);
+    s.squeeze<4>([&](int x, uint32_t v) {
+      if (s.y == 0) dig[2 * x + s.h] = v;
+      if (act && s.y == 0) row[KM_MU / 4 + 2 * x + s.h] = v;
+    });
+    s.clear();
+    s.absorb17<24>(kp, words, 0x1F, 0, words / 17 + 1);
+    s.squeeze<4>([&](int x, uint32_t v) {
+      if (s.y == 0) dig[8 + 2 * x + s.h] = v;
+    });
+    s.clear();
+  } else {
+    const int i = threadIdx.x & 15;
+    dig[i] = i < 8 ? row[KM_MU / 4 + i] : kp[i - 8];
+  }
+  wide::sync();
+  s.absorb17(dig, 8, 0x1F, 0, 1);
+  s.squeeze<5>([&](int x, uint32_t v) {
+    const int w = s.word(x);
+    if (act && w < 12) row[KM_KCD / 4 + 2 * w + s.h] = v;
+  });
+}
+
+// ss = SHAKE256(K || H(c), 32).  Encapsulation: d goes to the end of ct[x] and H(c) is made
+// here.  Decapsulation: H(c) is in the row, and the element's 16 lanes compare ct[x] with
+// the re-encryption and d, all of it (verify.cu:15-28 without its data-dependent branch);
+// on any difference z[x] takes the place of K by mask (verify.cu:40-50).
+template <int W, bool ENC, int N>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_cca_close_wide(
+    int n, uint8_t* ss, const uint8_t* km, std::conditional_t<ENC, uint8_t*, const uint8_t*> ct, const uint8_t* z,
+    size_t z_stride) {
+  using P = Par<N>;
+  __shared__ Wide4 sh;
+  wide::init_consts(sh.consts);
+  __syncthreads();
+  wide::Sponge s;
+  s.init(sh.states, sh.consts);
+  const int rq = 4 * blockIdx.x + s.st, r = rq < n ? rq : n - 1;
+  const bool act = rq < n;
+  const uint32_t* row = reinterpret_cast<const uint32_t*>(km + (size_t)r * kNewhopeKemBytes);
+  const uint32_t* d = row + KM_KCD / 4 + 16;
+  auto* c = reinterpret_cast<std::conditional_t<ENC, uint32_t*, const uint32_t*>>(ct + (size_t)r * P::CCA_CT);
+  uint32_t* dig = sh.dig[s.st];
+  const int i = threadIdx.x & 15;
+  if constexpr (ENC) {
+    static_assert(P::CT % 136 == 0, "d starts a block");
+    if (act && i < 8) c[P::CT / 4 + i] = d[i];
+    if (i < 8) dig[i] = row[KM_KCD / 4 + i];
+    s.absorb17<24>((const uint32_t*)c, P::CT / 8, 0x1F, 0, P::CT / 136);
+    s.absorb17(d, 4, 0x1F, 0, 1);
+    s.squeeze<4>([&](int x, uint32_t v) {
+      if (s.y == 0) dig[8 + 2 * x + s.h] = v;
+    });
+    s.clear();
+  } else {
+    const uint64_t* a = reinterpret_cast<const uint64_t*>(c);
+    const uint64_t* b = reinterpret_cast<const uint64_t*>(row + KM_CT2 / 4);
+    uint64_t diff = 0;
+#pragma unroll 4
+    for (int w = i; w < P::CT / 8; w += 16) diff |= a[w] ^ b[w];
+    if (i < 4) diff |= a[P::CT / 8 + i] ^ reinterpret_cast<const uint64_t*>(d)[i];
+    const uint64_t lanes = __ballot(diff != 0);
+    const uint32_t mask = ((lanes >> (16 * s.st)) & 0xFFFFu) != 0 ? 0xFFFFFFFFu : 0u;
+    const uint32_t kw = i < 8 ? row[KM_KCD / 4 + i] : row[KM_HC / 4 + i - 8];
+    const uint32_t zw = reinterpret_cast<const uint32_t*>(z + (size_t)r * z_stride)[i & 7];
+    dig[i] = i < 8 ? (kw & ~mask) | (zw & mask) : kw;
+  }
+  wide::sync();
+  s.absorb17(dig, 8, 0x1F, 0, 1);
+  uint32_t* o = reinterpret_cast<uint32_t*>(ss + (size_t)r * 32);
+  s.squeeze<4>([&](int x, uint32_t v) {
+    if (act && s.y == 0) o[2 * x + s.h] = v;
+  });
+}
+
 // ---- orchestration (cpapke.cu:265-476) -------------------------------------------
 
 template <int N>
@@ -1279,6 +1412,13 @@ struct Launch {
 inline dim3 elem_grid(int n) { return dim3((unsigned)((n + kElems - 1) / kElems)); }
 #define LAUNCH(kern, threads, ...) hipLaunchKernelGGL(kern, L.grid(threads), dim3(L.block), 0, s, __VA_ARGS__)
 #define LAUNCH_NTT(kern, ...) hipLaunchKernelGGL(kern, dim3(n), dim3(64), 0, s, __VA_ARGS__)
+
+// kernel template NAME<W, ...> on a wave per four elements
+#define LAUNCH_WIDE(NAME, TARGS, st, ...)                                                                  \
+  with_simd_waves(c->cu_count, (n + 3) / 4, [&](auto w_) {                                                 \
+    hipLaunchKernelGGL((NAME<decltype(w_)::value PQC_UNPAREN TARGS>), dim3((n + 3) / 4), dim3(64), 0, st, __VA_ARGS__); \
+  })
+#define PQC_UNPAREN(...) __VA_OPT__(,) __VA_ARGS__
 
 // cpapke_keypair (cpapke.cu:265-338) with pk at stride PK and sk at sk_stride
 // (the CCA-KEM's sk holds sk_cpa first), seeds at seed_stride
@@ -1367,10 +1507,15 @@ int dec_impl(pqc_ctx* c, int n, uint8_t* m, size_t m_stride, const uint8_t* ct, 
   return hip_err(hipGetLastError());
 }
 
-// Per-element CCA scratch row (one size for both N): mu or m' | H(pk) |
-// K || coin || d | H(c) | fail | re-encrypted ct
-constexpr int KM_MU = 0, KM_HPK = 32, KM_KCD = 64, KM_HC = 160, KM_FAIL = 192, KM_CT2 = 224;
-static_assert(KM_CT2 + Par<1024>::CCA_CT == kNewhopeKemBytes, "scratch row size");
+// out[x] = SHAKE256(in[x], 8 words bytes), 32 bytes, of a public key or a ciphertext
+inline void hash32(pqc_ctx* c, int n, uint8_t* out, size_t out_stride, const uint8_t* in, size_t in_stride, int words,
+                   hipStream_t s) {
+  const Launch L{c->tune.newhope_block};
+  if (n <= kWideMax)
+    LAUNCH_WIDE(k_shake256_wide, (), s, n, out, out_stride, in, in_stride, words);
+  else
+    LAUNCH(k_shake256_pair<4>, 2 * (size_t)n, n, out, out_stride, in, in_stride, words);
+}
 
 // NewHope CCA-KEM, the NewHope specification's transform over the CPA-PKE
 // (SHAKE256 for every hash).  Keypair coins: CPA seed || s, 64 bytes.
@@ -1382,8 +1527,7 @@ int cca_keypair(pqc_ctx* c, size_t n_, uint8_t* pk, uint8_t* sk, const uint8_t* 
   int rc = keypair_impl<N>(c, n, pk, sk, P::CCA_SK, coins, 64, plain, s);
   if (rc) return rc;
   LAUNCH(k_copy_words, n_ * (P::PK / 8), n, sk + P::SK, (size_t)P::CCA_SK, (const uint8_t*)pk, (size_t)P::PK, P::PK / 8);
-  LAUNCH(k_shake256_pair<4>, 2 * n_, n, sk + P::SK + P::PK, (size_t)P::CCA_SK, (const uint8_t*)pk, (size_t)P::PK,
-         P::PK / 8);
+  hash32(c, n, sk + P::SK + P::PK, P::CCA_SK, pk, P::PK, P::PK / 8, s);
   LAUNCH(k_copy_words, n_ * 4, n, sk + P::CCA_SK - SYM, (size_t)P::CCA_SK, coins + SYM, (size_t)64, 4);
   return hip_err(hipGetLastError());
 }
@@ -1396,14 +1540,24 @@ int cca_enc(pqc_ctx* c, size_t n_, uint8_t* ct, uint8_t* ss, const uint8_t* pk, 
   const int n = (int)n_;
   uint8_t* km = c->nhkem;
   const size_t kb = kNewhopeKemBytes;
-  LAUNCH(k_shake256_words<4>, n_, n, km + KM_MU, kb, coins, (size_t)32, 4);              // mu = H(coins)
-  LAUNCH(k_shake256_pair<4>, 2 * n_, n, km + KM_HPK, kb, pk, (size_t)P::PK, P::PK / 8);  // H(pk)
-  LAUNCH(k_shake256_2x32<12>, n_, n, km + KM_KCD, kb, (const uint8_t*)km + KM_MU, kb, (const uint8_t*)km + KM_HPK, kb);
+  const bool few = n <= kWideMax;
+  if (few) {
+    LAUNCH_WIDE(k_cca_open_wide, (true), s, n, km, coins, pk, (size_t)P::PK, P::PK / 8);
+  } else {
+    LAUNCH(k_shake256_words<4>, n_, n, km + KM_MU, kb, coins, (size_t)32, 4);  // mu = H(coins)
+    hash32(c, n, km + KM_HPK, kb, pk, P::PK, P::PK / 8, s);
+    LAUNCH(k_shake256_2x32<12>, n_, n, km + KM_KCD, kb, (const uint8_t*)km + KM_MU, kb, (const uint8_t*)km + KM_HPK,
+           kb);
+  }
   int rc = enc_impl<N>(c, n, ct, P::CCA_CT, km + KM_MU, kb, pk, P::PK, km + KM_KCD + SYM, kb, plain, s);
   if (rc) return rc;
-  LAUNCH(k_copy_words, n_ * 4, n, ct + P::CT, (size_t)P::CCA_CT, (const uint8_t*)km + KM_KCD + 2 * SYM, kb, 4);  // d
-  LAUNCH(k_shake256_pair<4>, 2 * n_, n, km + KM_HC, kb, (const uint8_t*)ct, (size_t)P::CCA_CT, P::CCA_CT / 8);  // H(c)
-  LAUNCH(k_shake256_2x32<4>, n_, n, ss, (size_t)32, (const uint8_t*)km + KM_KCD, kb, (const uint8_t*)km + KM_HC, kb);
+  if (few) {
+    LAUNCH_WIDE(k_cca_close_wide, (true, N), s, n, ss, (const uint8_t*)km, ct, (const uint8_t*)nullptr, (size_t)0);
+  } else {
+    LAUNCH(k_copy_words, n_ * 4, n, ct + P::CT, (size_t)P::CCA_CT, (const uint8_t*)km + KM_KCD + 2 * SYM, kb, 4);  // d
+    hash32(c, n, km + KM_HC, kb, ct, P::CCA_CT, P::CCA_CT / 8, s);
+    LAUNCH(k_shake256_2x32<4>, n_, n, ss, (size_t)32, (const uint8_t*)km + KM_KCD, kb, (const uint8_t*)km + KM_HC, kb);
+  }
   return hip_err(hipGetLastError());
 }
 
@@ -1415,24 +1569,32 @@ int cca_dec(pqc_ctx* c, size_t n_, uint8_t* ss, const uint8_t* ct, const uint8_t
   uint8_t* km = c->nhkem;
   const size_t kb = kNewhopeKemBytes;
   // H(c) depends only on the input ciphertext: it runs on the context's side
-  // stream (two lanes per element, half a wave per SIMD at 16384 elements)
-  // beside the decryption and re-encryption, and joins before the key selection
+  // stream beside the decryption and re-encryption, and joins before the key selection
   if (hipEventRecord(c->nh_fork, s) != hipSuccess || hipStreamWaitEvent(c->nh_side, c->nh_fork, 0) != hipSuccess)
     return PQC_ERR_DEVICE;
-  hipLaunchKernelGGL(k_shake256_pair<4>, L.grid(2 * n_), dim3(L.block), 0, c->nh_side, n, km + KM_HC, kb, ct,
-                     (size_t)P::CCA_CT, P::CCA_CT / 8);  // H(c)
+  hash32(c, n, km + KM_HC, kb, ct, P::CCA_CT, P::CCA_CT / 8, c->nh_side);
   if (hipGetLastError() != hipSuccess || hipEventRecord(c->nh_join, c->nh_side) != hipSuccess) return PQC_ERR_DEVICE;
   int rc = dec_impl<N>(c, n, km + KM_MU, kb, ct, P::CCA_CT, sk, P::CCA_SK, plain, s);  // m'
   if (rc) {
     (void)hipStreamWaitEvent(s, c->nh_join, 0);
     return rc;
   }
-  LAUNCH(k_copy_words, n_ * 4, n, km + KM_HPK, kb, sk + P::SK + P::PK, (size_t)P::CCA_SK, 4);
-  LAUNCH(k_shake256_2x32<12>, n_, n, km + KM_KCD, kb, (const uint8_t*)km + KM_MU, kb, (const uint8_t*)km + KM_HPK, kb);
+  const uint8_t* hpk = sk + P::SK + P::PK;
+  const bool few = n <= kWideMax;
+  if (few)
+    LAUNCH_WIDE(k_cca_open_wide, (false), s, n, km, (const uint8_t*)nullptr, hpk, (size_t)P::CCA_SK, 0);
+  else
+    LAUNCH(k_shake256_2x32<12>, n_, n, km + KM_KCD, kb, (const uint8_t*)km + KM_MU, kb, hpk, (size_t)P::CCA_SK);
   rc = enc_impl<N>(c, n, km + KM_CT2, kb, km + KM_MU, kb, sk + P::SK, P::CCA_SK, km + KM_KCD + SYM, kb, plain, s);
   if (rc) {
     (void)hipStreamWaitEvent(s, c->nh_join, 0);
     return rc;
+  }
+  if (few) {
+    if (hipStreamWaitEvent(s, c->nh_join, 0) != hipSuccess) return PQC_ERR_DEVICE;
+    LAUNCH_WIDE(k_cca_close_wide, (false, N), s, n, ss, (const uint8_t*)km, ct, sk + P::CCA_SK - SYM,
+                (size_t)P::CCA_SK);
+    return hip_err(hipGetLastError());
   }
   LAUNCH(k_copy_words, n_ * 4, n, km + KM_CT2 + P::CT, kb, (const uint8_t*)km + KM_KCD + 2 * SYM, kb, 4);  // d'
   hipLaunchKernelGGL(k_verify_words, dim3((unsigned)n), dim3(64), 0, s, n, reinterpret_cast<uint32_t*>(km + KM_FAIL),

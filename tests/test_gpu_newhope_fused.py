@@ -33,3 +33,32 @@ def test_fused_equals_plain_at_workgroup_edges(N):
         for a, b in zip(*out):
             assert (a == b).all()
     ctx.close()
+
+
+@pytest.mark.parametrize("N", [1024, 512])
+def test_cca_16_lane_hashes_equal_larger_call(N):
+    """Calls whose hashes run on 16 lanes per element against the rows of a call above that
+    form's limit, a differing byte in every part of the ciphertext included."""
+    import pqc_amd
+    n, alg = 8200, f"newhope{N}"
+    rng = np.random.default_rng(N + 1)
+    kc = rng.integers(0, 256, (n, 64), dtype=np.uint8)
+    ec = rng.integers(0, 256, (n, 32), dtype=np.uint8)
+    ctx = pqc_amd.Context([alg], max_batch=n)
+    print("newhope cca large", N, flush=True)
+    pk, sk = ctx.keypair_host(alg, kc)
+    ct, ss = ctx.enc_host(alg, pk, ec)
+    bad = ct.copy()
+    for i, col in enumerate((0, 14 * N // 8 - 1, 14 * N // 8, 17 * N // 8 - 1, 17 * N // 8, 17 * N // 8 + 31)):
+        bad[i::7, col] ^= 0x80 >> i
+    want = ctx.dec_host(alg, bad, sk)
+    ok = (bad == ct).all(axis=1)
+    assert ok.any() and (want[ok] == ss[ok]).all() and (want[~ok] != ss[~ok]).any(axis=1).all()
+    for m in (1, 3, 4, 5, 63, 1025, 4097, 8192):
+        print("newhope cca 16 lanes", N, m, flush=True)
+        pk2, sk2 = ctx.keypair_host(alg, kc[:m])
+        ct2, ss2 = ctx.enc_host(alg, pk[:m], ec[:m])
+        assert (pk2 == pk[:m]).all() and (sk2 == sk[:m]).all()
+        assert (ct2 == ct[:m]).all() and (ss2 == ss[:m]).all()
+        assert (ctx.dec_host(alg, bad[:m], sk[:m]) == want[:m]).all()
+    ctx.close()
