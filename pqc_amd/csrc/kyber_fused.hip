@@ -679,12 +679,17 @@ static int launch_fused(pqc_ctx* c, size_t n, uint8_t* ss, uint8_t* ct, const ui
 }
 
 // Kyber batches of at most this many requests take the one-workgroup-per-request kernels
-// (kyber_lowlat.hip), larger ones the stages (kyber_staged.hip).  Measured on MI355X,
-// per-request against staged, us: Kyber-768 decapsulation 92 / 155 at 1000, 149 / 159 at
-// 1500, 186 / 160 at 2000; encapsulation 124 / 238 at 1000, 264 / 245 at 2000; key
-// generation 89 / 164 at 1000, 181 / 169 at 2000; Kyber-1024 decapsulation 124 / 193 at
-// 1000, 196 / 200 at 1500.  tuning.lowlat_max overrides them all (-1 = never).
-constexpr int kLowLatDec = 1280, kLowLatEnc = 1280, kLowLatKey = 1280;
+// (kyber_lowlat.hip), larger ones the stages (kyber_staged.hip).  A request's workgroup of
+// four to six waves brings the time up in steps of one workgroup per CU (256 requests); the
+// line is the last step at which the stages are slower.  Measured on MI355X, per-request /
+// staged, us: Kyber-512 encapsulation 101 / 104 at 1280; Kyber-768 decapsulation 91 / 102 at
+// 1024 and 127 / 104 at 1280, encapsulation 121 / 123 and 170 / 128, key generation 91 / 116
+// and 122 / 118; Kyber-1024 decapsulation 122 / 126 and 172 / 135, key generation 134 / 150
+// and 171 / 154, encapsulation 132 / 159 at 768 and 198 / 158 at 1024.  Mixed batches (the
+// stages read their sizes on the device) 149 / 159 at 1500 requests of decapsulation.
+// tuning.lowlat_max overrides them all (-1 = never).
+constexpr int kLowLatMixed = 1280;
+constexpr int lowlat_limit(int k, bool enc) { return k == 2 ? 1280 : k == 4 && enc ? 768 : 1024; }
 
 inline bool use_lowlat(const pqc_ctx* c, size_t n, int dflt) {
   const int lim = c->tune.lowlat_max != 0 ? c->tune.lowlat_max : dflt;
@@ -707,7 +712,7 @@ static int launch_fused_keypair(pqc_ctx* c, size_t n, uint8_t* pk, uint8_t* sk, 
 }  // namespace kyber
 
 int kyber_fused_keypair(pqc_ctx* c, int k, size_t n, uint8_t* pk, uint8_t* sk, const uint8_t* coins, hipStream_t s) {
-  if (c->tune.fused_key_tile != 64 && kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatKey))
+  if (c->tune.fused_key_tile != 64 && kyber::fused::use_lowlat(c, n, kyber::fused::lowlat_limit(k, false)))
     return kyber_lowlat_keypair(k, n, pk, sk, coins, c->status, s);
   if (n > 0 && c->tune.fused_key_tile != 64) return kyber_staged_keypair(c, k, n, pk, sk, coins, s);
   switch (k) {
@@ -720,7 +725,7 @@ int kyber_fused_keypair(pqc_ctx* c, int k, size_t n, uint8_t* pk, uint8_t* sk, c
 
 int kyber_fused_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct, const uint8_t* sk, hipStream_t s) {
   uint8_t* ctm = const_cast<uint8_t*>(ct);  // read-only in the decaps instantiation
-  if (kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatDec)) return kyber_lowlat_dec(k, n, ss, ct, sk, c->status, s);
+  if (kyber::fused::use_lowlat(c, n, kyber::fused::lowlat_limit(k, false))) return kyber_lowlat_dec(k, n, ss, ct, sk, c->status, s);
   if (n > 0 && c->tune.fused_dec_tile != 64) return kyber_staged_dec(c, k, n, ss, ct, sk, s);
   switch (k) {
     case 2: return kyber::fused::launch_fused<2, true>(c, n, ss, ctm, sk, nullptr, s);
@@ -732,7 +737,7 @@ int kyber_fused_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct,
 
 int kyber_fused_enc(pqc_ctx* c, int k, size_t n, uint8_t* ct, uint8_t* ss, const uint8_t* pk, const uint8_t* coins,
                     hipStream_t s) {
-  if (kyber::fused::use_lowlat(c, n, kyber::fused::kLowLatEnc))
+  if (kyber::fused::use_lowlat(c, n, kyber::fused::lowlat_limit(k, true)))
     return kyber_lowlat_enc(k, n, ct, ss, pk, coins, c->status, s);
   if (n > 0 && c->tune.fused_enc_tile != 64) return kyber_staged_enc(c, k, n, ct, ss, pk, coins, s);
   switch (k) {
@@ -752,7 +757,7 @@ int kyber_fused_mixed(pqc_ctx* c, int dec, size_t n, const pqc_kem_req* reqs, ui
   using namespace kyber::fused;
   if (n == 0) return PQC_OK;
   if (!c->kmix_order || !c->kprf) return PQC_ERR_UNSUPPORTED;
-  if (use_lowlat(c, n, dec ? kLowLatDec : kLowLatEnc))  // one workgroup per descriptor, no bucketing
+  if (use_lowlat(c, n, kLowLatMixed))  // one workgroup per descriptor, no bucketing
     return kyber_lowlat_mixed(c, dec, n, reqs, ct, ct_bytes, key, key_bytes, ss, ss_bytes, coins, coins_bytes, s);
   const int cap = (int)c->max_batch;
   auto classify = [&](const pqc_kem_req* r, size_t m) {

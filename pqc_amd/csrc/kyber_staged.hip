@@ -14,6 +14,7 @@
 //   encapsulation  k_enc_sponge (H(pk), m, G; A^T) -> k_enc_prf -> k_enc_encrypt
 //                  (indcpa_enc) -> k_enc_final (H(ct), KDF)
 //   key generation k_key_seed (G) -> k_key_sponge (A; PRF) -> k_key_mul -> k_key_final (H(pk))
+//   the ..._few and ..._pair kernels are the same stages for fewer requests
 //
 // Scratch, by group of 16 requests (request r of a bucket: group r / 16, slot r % 16;
 // dense batches have one bucket, mixed batches three whose groups follow each other):
@@ -28,13 +29,14 @@
 // Measured on MI355X, us per call, this path and the 32-request tiles (two waves per
 // SIMD, butterfly transforms) or per-request workgroups it replaced:
 //   Kyber-768 decapsulation, 65536 requests    623    714
-//   Kyber-1024 decapsulation, 6000 requests    233    675 (a workgroup per request)
+//   Kyber-1024 decapsulation, 6000 requests    189    675 (a workgroup per request)
 // At 65536 the sponge stage takes ~370 us (53 permutations per request at 9.4 G/s, the
 // rate of the VALU on this mix), the product stages ~65 and ~140, the KDF ~15.
 #include <algorithm>
 #include <type_traits>
 
 #include "internal.h"
+#include "keccak_wide.cuh"
 #include "kyber_mfma.cuh"
 #include "kyber_src.cuh"
 #include "sponge.cuh"
@@ -308,6 +310,196 @@ __device__ __forceinline__ void key_final_wave(const KeySrc& src, int n, int w) 
   uint64_t A[25];
   sponge_absorb_two<kRateSha3_256, P::pk_bytes / 8>(A, src.pk + (size_t)rc * P::pk_bytes, 0x06);
   if (r < n) store_words4(src.sk + (size_t)r * P::sk_bytes + P::hpk_off, A);
+}
+
+// ---- dense batches of at most kFewMax requests: the long chains shortened ------------------
+// A stage lasts as long as its longest chain: on one lane the hash of a ciphertext or a
+// public key (6 to 12 permutations at ~8 us) and decapsulation's G and 2K + 1 noise streams
+// of a request.  With few requests the chip has room to shorten them: the hashes run on 16
+// lanes per request (keccak_wide.cuh, 3.3 us per permutation), and every noise stream of
+// decapsulation has a lane that makes its own G.  Decapsulation's H(ct) is not needed
+// before the KDF and runs beside the re-encryption.  us per call, one lane per request ->
+// this: Kyber-512 encapsulation 174 -> 109 (2501 requests), 182 -> 152 (8192), 205 -> 230
+// (16384); Kyber-1024 decapsulation 217 -> 143 (2501), 218 -> 189 (6000), 259 -> 222 (8192),
+// 309 -> 390 (16384); Kyber-768 key generation 168 -> 126 (2501), 187 -> 162 (8192).
+constexpr int kFewMax = 8192;
+
+struct WideLds {
+  wide::Consts consts;
+  wide::States states;
+  alignas(16) uint32_t dig[4][16];  // per request: the words of its next short message
+};
+
+// this lane's request of wave w, four to a wave (past the batch's end: the last one)
+struct WideReq {
+  int r;
+  bool act;
+  uint8_t* row;
+  __device__ __forceinline__ WideReq(const Scratch& sc, int n, int w, const wide::Sponge& s) {
+    const int rq = 4 * w + s.st;
+    act = rq < n;
+    r = act ? rq : n - 1;
+    row = sc.row_of(r / 16, r % 16);
+  }
+};
+
+// the first 32 bytes of the state to o
+__device__ __forceinline__ void wide_digest(const wide::Sponge& s, bool act, uint32_t* o) {
+  s.squeeze<4>([&](int x, uint32_t v) {
+    if (act && s.y == 0) o[2 * x + s.h] = v;
+  });
+}
+
+__device__ __forceinline__ const uint32_t* words32(const uint8_t* p) { return reinterpret_cast<const uint32_t*>(p); }
+__device__ __forceinline__ uint32_t* words32(uint8_t* p) { return reinterpret_cast<uint32_t*>(p); }
+
+// SHA3-256 of NWORDS 64-bit words
+template <int NWORDS>
+__device__ __forceinline__ void wide_h(wide::Sponge& s, const uint32_t* p) {
+  s.clear();
+  s.absorb17<(NWORDS > 17 ? 24 : 4)>(p, NWORDS, 0x06, 0, NWORDS / 17 + 1);
+}
+
+template <int K>
+__device__ __forceinline__ void dec_hash_wide(const DenseSrc& src, const Scratch& sc, int n, int w, wide::Sponge& s) {
+  using P = Params<K>;
+  const WideReq x(sc, n, w, s);
+  wide_h<P::ct_bytes / 8>(s, words32(src.template req<K, true>(x.r).ct));
+  wide_digest(s, x.act, words32(x.row + kRowH));
+}
+
+// G of 64 requests and noise stream `nonce`
+template <int K>
+__device__ __forceinline__ void dec_prf_one(const DenseSrc& src, const Scratch& sc, int n, int w, int nonce) {
+  using P = Params<K>;
+  const int r = 64 * w + (threadIdx.x & 63);
+  if (r >= n) return;
+  uint8_t* row = sc.row_of(r / 16, r % 16);
+  uint64_t m[8], A[25], seed[4];
+  load_words4(*reinterpret_cast<uint64_t(*)[4]>(m), row + kRowM);
+  load_words4(*reinterpret_cast<uint64_t(*)[4]>(m + 4), src.template req<K, true>(r).key + P::hpk_off);
+  absorb_fixed<kRateSha3_512, 8, true>(A, m, 0x06);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) seed[i] = A[4 + i];
+  if (nonce == 0) store_words4(row + kRowKbar, A);
+  prf_store(sc, r / 16, r % 16, seed, nonce);
+}
+
+template <int K>
+__device__ __forceinline__ void enc_open_wide(const DenseSrc& src, const Scratch& sc, int n, int w, wide::Sponge& s,
+                                              WideLds& sh) {
+  using P = Params<K>;
+  const WideReq x(sc, n, w, s);
+  const ReqP q = src.template req<K, false>(x.r);
+  uint32_t* dig = sh.dig[s.st];
+  wide_h<4>(s, words32(q.coins));
+  wide_digest(s, true, dig);
+  wide_digest(s, x.act, words32(x.row + kRowM));
+  wide_h<P::pk_bytes / 8>(s, words32(q.key));
+  wide_digest(s, true, dig + 8);
+  wide::sync();
+  s.clear();
+  uint32_t m[5];
+#pragma unroll
+  for (int c = 0; c < 5; ++c) {
+    const int word = s.word(c);
+    m[c] = word < 8 ? dig[2 * (word & 7) + s.h] : 0;
+    if (word == 8) m[c] = s.h ? 0x80000000u : 0x06u;  // the last word of SHA3-512's rate
+  }
+  wide::sync();
+  s.absorb(m);
+  s.permute();
+  s.squeeze<5>([&](int c, uint32_t v) {  // Kbar, then the noise seed
+    const int word = s.word(c);
+    if (x.act && word < 8) words32(x.row + (word < 4 ? kRowKbar : kRowH - 32))[2 * word + s.h] = v;
+  });
+}
+
+// ss = SHAKE256(first || second, 32), the two in dig
+__device__ __forceinline__ void wide_kdf(wide::Sponge& s, const WideReq& x, const uint32_t* dig, uint8_t* ss) {
+  wide::sync();
+  s.clear();
+  s.absorb17(dig, 8, 0x1F, 0, 1);
+  wide::sync();
+  wide_digest(s, x.act, words32(ss));
+}
+
+template <int K>
+__device__ __forceinline__ void enc_final_wide(const DenseSrc& src, const Scratch& sc, int n, int w, wide::Sponge& s,
+                                               WideLds& sh) {
+  using P = Params<K>;
+  const WideReq x(sc, n, w, s);
+  const ReqP q = src.template req<K, false>(x.r);
+  uint32_t* dig = sh.dig[s.st];
+  wide_h<P::ct_bytes / 8>(s, words32(q.ct));
+  wide_digest(s, true, dig + 8);
+  const int i = threadIdx.x & 15;
+  if (i < 8) dig[i] = words32(x.row + kRowKbar)[i];
+  wide_kdf(s, x, dig, q.ss);
+}
+
+template <int K>
+__device__ __forceinline__ void dec_kdf_wide(const DenseSrc& src, const Scratch& sc, int n, int w, wide::Sponge& s,
+                                             WideLds& sh) {
+  using P = Params<K>;
+  const WideReq x(sc, n, w, s);
+  const ReqP q = src.template req<K, true>(x.r);
+  uint32_t* dig = sh.dig[s.st];
+  const int i = threadIdx.x & 15;
+  const uint32_t f = *words32(x.row + kRowFail), mask = 0u - ((f | (0u - f)) >> 31);
+  const uint32_t v = words32(x.row + (i < 8 ? kRowKbar : kRowH - 32))[i];
+  const uint32_t z = words32(q.key + P::z_off)[i & 7];
+  dig[i] = i < 8 ? v ^ (mask & (z ^ v)) : v;
+  wide_kdf(s, x, dig, q.ss);
+}
+
+template <int K>
+__device__ __forceinline__ void key_final_wide(const KeySrc& src, const Scratch& sc, int n, int w, wide::Sponge& s) {
+  using P = Params<K>;
+  const WideReq x(sc, n, w, s);
+  wide_h<P::pk_bytes / 8>(s, words32(src.pk + (size_t)x.r * P::pk_bytes));
+  wide_digest(s, x.act, words32(src.sk + (size_t)x.r * P::sk_bytes + P::hpk_off));
+}
+
+// ---- dense batches of up to kPairMax requests: the last stage's hashes on lane pairs -------
+// One lane per request would leave half of the SIMDs or more without a wave; a pair's chain
+// is shorter (6.3 us per permutation against 7.65).  us per call, lane -> pair: Kyber-768
+// encapsulation 302 -> 286 at 16384 requests, 378 -> 364 at 32768, 642 -> 666 at 65536;
+// Kyber-1024 key generation 331 -> 321, 525 -> 524 and 922 -> 968.
+constexpr int kPairMax = 32768;
+
+__device__ __forceinline__ void digest_pair(const uint32_t (&S)[25], uint32_t half, uint8_t* o) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) words32(o)[2 * i + half] = S[i];
+}
+
+template <int K>
+__device__ __forceinline__ void enc_final_pair(const DenseSrc& src, const Scratch& sc, int n, int w) {
+  using P = Params<K>;
+  const int r = 32 * w + ((threadIdx.x & 63) >> 1);
+  const uint32_t half = threadIdx.x & 1;
+  if (r >= n) return;  // both lanes of a pair
+  const ReqP q = src.template req<K, false>(r);
+  const uint32_t* kbar = words32(sc.row_of(r / 16, r % 16) + kRowKbar);
+  uint32_t S[25], A[25];
+  absorb_range_pair(S, q.ct, P::ct_bytes / 8, 0, P::ct_bytes / 136 + 1, 0x06, half);
+#pragma unroll
+  for (int i = 0; i < 25; ++i) A[i] = i < 4 ? kbar[2 * i + half] : i < 8 ? S[i - 4] : 0;
+  A[8] = half ? 0u : 0x1Fu;
+  A[kRateShake256 - 1] = half ? 0x80000000u : 0u;
+  keccakf1600_pair(A, half);
+  digest_pair(A, half, q.ss);
+}
+
+template <int K>
+__device__ __forceinline__ void key_final_pair(const KeySrc& src, int n, int w) {
+  using P = Params<K>;
+  const int r = 32 * w + ((threadIdx.x & 63) >> 1);
+  const uint32_t half = threadIdx.x & 1;
+  if (r >= n) return;
+  uint32_t S[25];
+  absorb_range_pair(S, src.pk + (size_t)r * P::pk_bytes, P::pk_bytes / 8, 0, P::pk_bytes / 136 + 1, 0x06, half);
+  digest_pair(S, half, src.sk + (size_t)r * P::sk_bytes + P::hpk_off);
 }
 
 // ---- product stages ----------------------------------------------------------------------
@@ -661,6 +853,22 @@ __global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_dec_sponge(int n, Dens
   }
 }
 
+// at most kFewMax requests: a wave per 64 noise streams, then the matrix entries
+template <int K, int W>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_dec_sponge_few(int n, DenseSrc src, Scratch sc) {
+  using P = Params<K>;
+  __shared__ SponLds sh;
+  const int wr = (n + 63) / 64, wp = wr * (2 * K + 1), total = wp + matrix_waves<K>(n);
+  for (int w = blockIdx.x; w < total; w += gridDim.x) {
+    if (w < wp)
+      dec_prf_one<K>(src, sc, n, w % wr, w / wr);
+    else
+      matrix_wave<K, true>(sc, Bucket{n, 0}, w - wp, sh, [&](int r) {
+        return src.template req<K, true>(r).key + P::sk_cpa_bytes + P::polyvec_bytes;
+      });
+  }
+}
+
 template <int K>
 __global__ __launch_bounds__(kProdThreads, 2) void k_dec_reencrypt(int n, DenseSrc src, Scratch sc) {
   __shared__ DftLds<true, true> sh;
@@ -669,10 +877,55 @@ __global__ __launch_bounds__(kProdThreads, 2) void k_dec_reencrypt(int n, DenseS
   for (int tile = blockIdx.x; tile < (n + 63) / 64; tile += gridDim.x) reencrypt_tile<K, true>(src, sc, b, tile, sh);
 }
 
+// at most kFewMax requests: the first `prod` workgroups re-encrypt, 64 requests each at a
+// time, which leaves most CUs without work; the others hash ciphertexts, 16 requests each,
+// for the KDF after this stage
+template <int K>
+__global__ __launch_bounds__(kProdThreads, 2) void k_dec_reencrypt_few(int n, int prod, DenseSrc src, Scratch sc) {
+  constexpr int kWaves = kProdThreads / 64;
+  __shared__ union {
+    DftLds<true, true> dft;
+    struct {
+      wide::Consts consts;
+      wide::States states[kWaves];
+    } h;
+  } sh;
+  if ((int)blockIdx.x < prod) {
+    load_tables<true, true, kProdThreads>(sh.dft, &c_dft);
+    for (int tile = blockIdx.x; tile < (n + 63) / 64; tile += prod)
+      reencrypt_tile<K, true>(src, sc, Bucket{n, 0}, tile, sh.dft);
+    return;
+  }
+  wide::init_consts(sh.h.consts);
+  __syncthreads();
+  wide::Sponge s;
+  const int wave = threadIdx.x >> 6;
+  s.init(sh.h.states[wave], sh.h.consts);
+  const int w = ((int)blockIdx.x - prod) * kWaves + wave;
+  if (w < (n + 3) / 4) dec_hash_wide<K>(src, sc, n, w, s);
+}
+
 template <int K, int W>
 __global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_dec_kdf(int n, DenseSrc src, Scratch sc) {
   for (int w = blockIdx.x; w < (n + 63) / 64; w += gridDim.x) dec_kdf_wave<K>(src, sc, Bucket{n, 0}, w);
 }
+
+// a kernel of one wave per four requests: NAME(n, source, scratch) runs the statement for
+// each wave w of the batch
+#define WIDE_KERNEL(NAME, SRC, ...)                                                                       \
+  template <int K, int W>                                                                                 \
+  __global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void NAME(int n, SRC src, Scratch sc) {              \
+    __shared__ WideLds sh;                                                                                \
+    wide::init_consts(sh.consts);                                                                         \
+    __syncthreads();                                                                                      \
+    wide::Sponge s;                                                                                       \
+    s.init(sh.states, sh.consts);                                                                         \
+    for (int w = blockIdx.x; w < (n + 3) / 4; w += gridDim.x) __VA_ARGS__;                                \
+  }
+WIDE_KERNEL(k_dec_kdf_few, DenseSrc, dec_kdf_wide<K>(src, sc, n, w, s, sh))
+WIDE_KERNEL(k_enc_final_few, DenseSrc, enc_final_wide<K>(src, sc, n, w, s, sh))
+WIDE_KERNEL(k_key_final_few, KeySrc, key_final_wide<K>(src, sc, n, w, s))
+#undef WIDE_KERNEL
 
 // encapsulation: H(pk), m, G (the longest chains first), then the matrix entries
 template <int K, int W>
@@ -687,6 +940,30 @@ __global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_enc_sponge(int n, Dens
     else
       matrix_wave<K, true>(sc, b, w - wr, sh,
                            [&](int r) { return src.template req<K, false>(r).key + P::polyvec_bytes; });
+  }
+}
+
+template <int K, int W>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_enc_sponge_few(int n, DenseSrc src, Scratch sc) {
+  using P = Params<K>;
+  __shared__ union {
+    SponLds m;
+    WideLds h;
+  } sh;
+  const int wh = (n + 3) / 4, total = wh + matrix_waves<K>(n);
+  for (int w = blockIdx.x; w < total; w += gridDim.x) {
+    if (w < wh) {
+      wide::Sponge s;
+      __syncthreads();
+      wide::init_consts(sh.h.consts);
+      __syncthreads();
+      s.init(sh.h.states, sh.h.consts);
+      enc_open_wide<K>(src, sc, n, w, s, sh.h);
+      __syncthreads();
+    } else {
+      matrix_wave<K, true>(sc, Bucket{n, 0}, w - wh, sh.m,
+                           [&](int r) { return src.template req<K, false>(r).key + P::polyvec_bytes; });
+    }
   }
 }
 
@@ -739,6 +1016,16 @@ __global__ __launch_bounds__(kProdThreads, 2) void k_key_mul(int n, KeySrc src, 
 template <int K, int W>
 __global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_key_final(int n, KeySrc src) {
   for (int w = blockIdx.x; w < (n + 63) / 64; w += gridDim.x) key_final_wave<K>(src, n, w);
+}
+
+// up to kPairMax requests
+template <int K, int W>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_enc_final_pair(int n, DenseSrc src, Scratch sc) {
+  for (int w = blockIdx.x; w < (n + 31) / 32; w += gridDim.x) enc_final_pair<K>(src, sc, n, w);
+}
+template <int K, int W>
+__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_key_final_pair(int n, KeySrc src) {
+  for (int w = blockIdx.x; w < (n + 31) / 32; w += gridDim.x) key_final_pair<K>(src, n, w);
 }
 
 // ---- mixed kernels ------------------------------------------------------------------------------
@@ -909,13 +1196,25 @@ static int dec(pqc_ctx* c, size_t n_all, uint8_t* ss, uint8_t* ct, const uint8_t
   const Scratch sc = scratch_of(c, K);
   for (size_t at = 0; at < n_all; at += c->kstage_max) {
     const int n = (int)std::min(n_all - at, c->kstage_max);
-    const int tiles = (n + 63) / 64, waves = 2 * tiles + matrix_waves<K>(n);
+    const bool few = n <= kFewMax;
+    const int tiles = (n + 63) / 64, fours = (n + 3) / 4;
+    const int waves = tiles * (few ? 2 * K + 1 : 2) + matrix_waves<K>(n), prod = prod_grid(c, tiles);
     const DenseSrc src{ss + at * 32, ct + at * P::ct_bytes, sk + at * P::sk_bytes, nullptr, c->kprf};
-    hipLaunchKernelGGL((k_open<K>), dim3(prod_grid(c, tiles)), dim3(kProdThreads), 0, s, n, src, sc);
-    const int sg = sponge_grid(c, waves), kg = sponge_grid(c, tiles);
-    LAUNCH_WAVES(c, sg, s, (k_dec_sponge<K, W>), n, src, sc);
-    hipLaunchKernelGGL((k_dec_reencrypt<K>), dim3(prod_grid(c, tiles)), dim3(kProdThreads), 0, s, n, src, sc);
-    LAUNCH_WAVES(c, kg, s, (k_dec_kdf<K, W>), n, src, sc);
+    hipLaunchKernelGGL((k_open<K>), dim3(prod), dim3(kProdThreads), 0, s, n, src, sc);
+    const int sg = sponge_grid(c, waves), kg = sponge_grid(c, few ? fours : tiles);
+    if (few)
+      LAUNCH_WAVES(c, sg, s, (k_dec_sponge_few<K, W>), n, src, sc);
+    else
+      LAUNCH_WAVES(c, sg, s, (k_dec_sponge<K, W>), n, src, sc);
+    if (few)
+      hipLaunchKernelGGL((k_dec_reencrypt_few<K>), dim3(prod + (fours + 3) / 4), dim3(kProdThreads), 0, s, n, prod, src,
+                         sc);
+    else
+      hipLaunchKernelGGL((k_dec_reencrypt<K>), dim3(prod), dim3(kProdThreads), 0, s, n, src, sc);
+    if (few)
+      LAUNCH_WAVES(c, kg, s, (k_dec_kdf_few<K, W>), n, src, sc);
+    else
+      LAUNCH_WAVES(c, kg, s, (k_dec_kdf<K, W>), n, src, sc);
     const int rc = hip_err(hipGetLastError());
     if (rc) return rc;
   }
@@ -929,14 +1228,23 @@ static int enc(pqc_ctx* c, size_t n_all, uint8_t* ss, uint8_t* ct, const uint8_t
   const Scratch sc = scratch_of(c, K);
   for (size_t at = 0; at < n_all; at += c->kstage_max) {
     const int n = (int)std::min(n_all - at, c->kstage_max);
-    const int tiles = (n + 63) / 64;
+    const bool few = n <= kFewMax;
+    const int tiles = (n + 63) / 64, hash = few ? (n + 3) / 4 : tiles;
     const DenseSrc src{ss + at * 32, ct + at * P::ct_bytes, pk + at * P::pk_bytes, coins + at * 32, c->kprf};
-    const int sg = sponge_grid(c, tiles + matrix_waves<K>(n)), pg = sponge_grid(c, tiles * (2 * K + 1)),
-              fg = sponge_grid(c, tiles);
-    LAUNCH_WAVES(c, sg, s, (k_enc_sponge<K, W>), n, src, sc);
+    const int sg = sponge_grid(c, hash + matrix_waves<K>(n)), pg = sponge_grid(c, tiles * (2 * K + 1)),
+              fg = sponge_grid(c, hash), qg = sponge_grid(c, (n + 31) / 32);
+    if (few)
+      LAUNCH_WAVES(c, sg, s, (k_enc_sponge_few<K, W>), n, src, sc);
+    else
+      LAUNCH_WAVES(c, sg, s, (k_enc_sponge<K, W>), n, src, sc);
     LAUNCH_WAVES(c, pg, s, (k_enc_prf<K, W>), n, sc);
     hipLaunchKernelGGL((k_enc_encrypt<K>), dim3(prod_grid(c, tiles)), dim3(kProdThreads), 0, s, n, src, sc);
-    LAUNCH_WAVES(c, fg, s, (k_enc_final<K, W>), n, src, sc);
+    if (few)
+      LAUNCH_WAVES(c, fg, s, (k_enc_final_few<K, W>), n, src, sc);
+    else if (n <= kPairMax)
+      LAUNCH_WAVES(c, qg, s, (k_enc_final_pair<K, W>), n, src, sc);
+    else
+      LAUNCH_WAVES(c, fg, s, (k_enc_final<K, W>), n, src, sc);
     const int rc = hip_err(hipGetLastError());
     if (rc) return rc;
   }
@@ -951,11 +1259,18 @@ static int keypair(pqc_ctx* c, size_t n_all, uint8_t* pk, uint8_t* sk, const uin
     const int n = (int)std::min(n_all - at, c->kstage_max);
     const int tiles = (n + 63) / 64;
     const KeySrc src{pk + at * P::pk_bytes, sk + at * P::sk_bytes, coins + at * 64};
-    const int sg = sponge_grid(c, matrix_waves<K>(n) + 2 * K * tiles), fg = sponge_grid(c, tiles);
+    const bool few = n <= kFewMax;
+    const int sg = sponge_grid(c, matrix_waves<K>(n) + 2 * K * tiles), fg = sponge_grid(c, tiles),
+              hg = sponge_grid(c, (n + 3) / 4), qg = sponge_grid(c, (n + 31) / 32);
     LAUNCH_WAVES(c, fg, s, (k_key_seed<K, W>), n, src, sc);
     LAUNCH_WAVES(c, sg, s, (k_key_sponge<K, W>), n, src, sc);
     hipLaunchKernelGGL((k_key_mul<K>), dim3(prod_grid(c, tiles)), dim3(kProdThreads), 0, s, n, src, sc);
-    LAUNCH_WAVES(c, fg, s, (k_key_final<K, W>), n, src);
+    if (few)
+      LAUNCH_WAVES(c, hg, s, (k_key_final_few<K, W>), n, src, sc);
+    else if (n <= kPairMax)
+      LAUNCH_WAVES(c, qg, s, (k_key_final_pair<K, W>), n, src);
+    else
+      LAUNCH_WAVES(c, fg, s, (k_key_final<K, W>), n, src);
     const int rc = hip_err(hipGetLastError());
     if (rc) return rc;
   }

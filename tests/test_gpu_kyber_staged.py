@@ -88,3 +88,30 @@ def test_per_request_kernels_vs_oracle(pqc, k):
         assert all((a == b).all() for a, b in zip(ctx.enc_host(ALG[k], pk, c32), O.kyber_batch("enc", k, [pk, c32])))
         assert (ctx.dec_host(ALG[k], ct, sk) == O.kyber_batch("dec", k, [ct, sk])).all()
     ctx.close()
+
+
+@pytest.mark.parametrize("k", [2, 3, 4])
+def test_hash_forms_agree_across_batch_sizes(pqc, k):
+    """The stages hash on one lane, a lane pair or 16 lanes per request, by batch size: the
+    rows of a call in one form against calls in the others, and against the oracle."""
+    n, rng = 32800, np.random.default_rng(40 + k)
+    ctx = staged_ctx(pqc, k, n, 0)
+    kc = rng.integers(0, 256, (n, 64), dtype=np.uint8)
+    ec = rng.integers(0, 256, (n, 32), dtype=np.uint8)
+    print("hash forms k", k, "n", n, flush=True)
+    pk, sk = ctx.keypair_host(ALG[k], kc)
+    ct, ss = ctx.enc_host(ALG[k], pk, ec)
+    bad = ct.copy()
+    bad[::5, int(rng.integers(0, ct.shape[1]))] ^= 4
+    want = ctx.dec_host(ALG[k], bad, sk)
+    ok = (bad == ct).all(axis=1)
+    assert (want[ok] == ss[ok]).all() and (want[~ok] != ss[~ok]).any(axis=1).all()
+    for m in (5, 1027, 8192, 8193, 32768):
+        print("hash forms k", k, "n", m, flush=True)
+        pk2, sk2 = ctx.keypair_host(ALG[k], kc[:m])
+        ct2, ss2 = ctx.enc_host(ALG[k], pk[:m], ec[:m])
+        assert (pk2 == pk[:m]).all() and (sk2 == sk[:m]).all()
+        assert (ct2 == ct[:m]).all() and (ss2 == ss[:m]).all()
+        assert (ctx.dec_host(ALG[k], bad[:m], sk[:m]) == want[:m]).all()
+    assert (O.kyber_batch("dec", k, [bad[:8], sk[:8]]) == want[:8]).all()
+    ctx.close()
