@@ -714,7 +714,7 @@ static int launch_fused_keypair(pqc_ctx* c, size_t n, uint8_t* pk, uint8_t* sk, 
 int kyber_fused_keypair(pqc_ctx* c, int k, size_t n, uint8_t* pk, uint8_t* sk, const uint8_t* coins, hipStream_t s) {
   if (c->tune.fused_key_tile != 64 && kyber::fused::use_lowlat(c, n, kyber::fused::lowlat_limit(k, false)))
     return kyber_lowlat_keypair(k, n, pk, sk, coins, c->status, s);
-  if (n > 0 && c->tune.fused_key_tile != 64) return kyber_staged_keypair(c, k, n, pk, sk, coins, s);
+  if (n > 0 && c->kat && c->tune.fused_key_tile != 64) return kyber_staged_keypair(c, k, n, pk, sk, coins, s);
   switch (k) {
     case 2: return kyber::fused::launch_fused_keypair<2>(c, n, pk, sk, coins, s);
     case 3: return kyber::fused::launch_fused_keypair<3>(c, n, pk, sk, coins, s);
@@ -726,7 +726,7 @@ int kyber_fused_keypair(pqc_ctx* c, int k, size_t n, uint8_t* pk, uint8_t* sk, c
 int kyber_fused_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct, const uint8_t* sk, hipStream_t s) {
   uint8_t* ctm = const_cast<uint8_t*>(ct);  // read-only in the decaps instantiation
   if (kyber::fused::use_lowlat(c, n, kyber::fused::lowlat_limit(k, false))) return kyber_lowlat_dec(k, n, ss, ct, sk, c->status, s);
-  if (n > 0 && c->tune.fused_dec_tile != 64) return kyber_staged_dec(c, k, n, ss, ct, sk, s);
+  if (n > 0 && c->kat && c->tune.fused_dec_tile != 64) return kyber_staged_dec(c, k, n, ss, ct, sk, s);
   switch (k) {
     case 2: return kyber::fused::launch_fused<2, true>(c, n, ss, ctm, sk, nullptr, s);
     case 3: return kyber::fused::launch_fused<3, true>(c, n, ss, ctm, sk, nullptr, s);
@@ -739,7 +739,7 @@ int kyber_fused_enc(pqc_ctx* c, int k, size_t n, uint8_t* ct, uint8_t* ss, const
                     hipStream_t s) {
   if (kyber::fused::use_lowlat(c, n, kyber::fused::lowlat_limit(k, true)))
     return kyber_lowlat_enc(k, n, ct, ss, pk, coins, c->status, s);
-  if (n > 0 && c->tune.fused_enc_tile != 64) return kyber_staged_enc(c, k, n, ct, ss, pk, coins, s);
+  if (n > 0 && c->kat && c->tune.fused_enc_tile != 64) return kyber_staged_enc(c, k, n, ct, ss, pk, coins, s);
   switch (k) {
     case 2: return kyber::fused::launch_fused<2, false>(c, n, ss, ct, pk, coins, s);
     case 3: return kyber::fused::launch_fused<3, false>(c, n, ss, ct, pk, coins, s);
@@ -768,7 +768,7 @@ int kyber_fused_mixed(pqc_ctx* c, int dec, size_t n, const pqc_kem_req* reqs, ui
                        c->status);
   };
   kyber::MixedSrc src{reqs, c->kmix_order, cap, ss, ct, key, coins, c->kprf, c->kprf_per_elem};
-  if ((dec ? c->tune.fused_dec_tile : c->tune.fused_enc_tile) != 64) {
+  if (c->kat && (dec ? c->tune.fused_dec_tile : c->tune.fused_enc_tile) != 64) {
     // in stages, kstage_max requests at a time (their scratch)
     for (size_t at = 0; at < n; at += c->kstage_max) {
       const size_t m = std::min(n - at, c->kstage_max);

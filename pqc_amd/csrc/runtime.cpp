@@ -353,6 +353,33 @@ int single(int alg, Op op, uint8_t* o0, uint8_t* o1, const uint8_t* i0, const ui
 
 extern "C" {
 
+// Noise rows of the Kyber kernels and the scratch of the staged path for up to kstage_max
+// requests (groups of 16 of each parameter set, read in tiles of 64: under 128 rows of
+// padding); larger batches run in passes.  A budget that leaves less room gets shorter
+// passes, and one that holds the noise rows alone none: batches then run in 64-request
+// tiles.
+static int alloc_kyber_stage(pqc_ctx* c, int kmax) {
+  const size_t at = pqc::kyber_stage_at_bytes(kmax);
+  for (size_t stage = std::min<size_t>(c->ld, 65536);; stage = stage > 64 ? stage / 2 & ~(size_t)63 : 0) {
+    const size_t rows = stage ? stage + 128 : 0;
+    const size_t prf = c->kprf_per_elem * std::max(c->ld, rows);
+    if (stage && c->hbm_budget && c->allocated + prf + rows * (at + 128) > c->hbm_budget) continue;
+    void* p = nullptr;
+    int rc = ctx_alloc(c, &p, prf);
+    if (rc) return rc;
+    c->kprf = (uint8_t*)p;
+    if (!stage) return PQC_OK;
+    rc = ctx_alloc(c, &p, rows * at);
+    if (rc) return rc;
+    c->kat = (uint8_t*)p;
+    rc = ctx_alloc(c, &p, rows * 128);
+    if (rc) return rc;
+    c->krow = (uint8_t*)p;
+    c->kstage_max = stage;
+    return PQC_OK;
+  }
+}
+
 int pqc_ctx_create(pqc_ctx** out, unsigned alg_mask, size_t max_batch, size_t hbm_budget) {
   if (!out || max_batch == 0 || max_batch > (1u << 26)) return PQC_ERR_INVALID_ARG;
   *out = nullptr;
@@ -392,19 +419,6 @@ int pqc_ctx_create(pqc_ctx** out, unsigned alg_mask, size_t max_batch, size_t hb
     if (rc) goto fail;
     c->kbytes = (uint8_t*)p;
     c->kprf_per_elem = (size_t)(2 * kmax + 1) * 128;
-    rc = ctx_alloc(c, &p, c->kprf_per_elem * (c->ld + 128));
-    if (rc) goto fail;
-    c->kprf = (uint8_t*)p;
-    // scratch of the staged path for up to kstage_max requests (groups of 16 of each
-    // parameter set, read in tiles of 64: under 128 rows of padding); larger batches run
-    // in passes
-    c->kstage_max = std::min<size_t>(c->ld, 65536);
-    rc = ctx_alloc(c, &p, pqc::kyber_stage_at_bytes(kmax) * (c->kstage_max + 128));
-    if (rc) goto fail;
-    c->kat = (uint8_t*)p;
-    rc = ctx_alloc(c, &p, (size_t)128 * (c->kstage_max + 128));
-    if (rc) goto fail;
-    c->krow = (uint8_t*)p;
     rc = ctx_alloc(c, &p, (size_t)3 * c->ld * sizeof(uint32_t) + 256);
     if (rc) goto fail;
     c->kmix_order = (uint32_t*)p;
@@ -466,6 +480,10 @@ int pqc_ctx_create(pqc_ctx** out, unsigned alg_mask, size_t max_batch, size_t hb
   rc = ctx_alloc(c, &p, 256);
   if (rc) goto fail;
   c->status = (uint32_t*)p;
+  if (kmax) {
+    rc = alloc_kyber_stage(c, kmax);
+    if (rc) goto fail;
+  }
   if (hipMemset(c->status, 0, 256) != hipSuccess) {
     rc = PQC_ERR_DEVICE;
     goto fail;

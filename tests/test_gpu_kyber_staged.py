@@ -115,3 +115,29 @@ def test_hash_forms_agree_across_batch_sizes(pqc, k):
         assert (ctx.dec_host(ALG[k], bad[:m], sk[:m]) == want[:m]).all()
     assert (O.kyber_batch("dec", k, [bad[:8], sk[:8]]) == want[:8]).all()
     ctx.close()
+
+
+@pytest.mark.parametrize("k", [2, 4])
+def test_budget_limits_staged_scratch(pqc, k):
+    """A budget below the full scratch gets shorter passes, one that holds only the noise
+    rows 64-request tiles, with the same bytes; less is refused."""
+    n = 2000
+    _, sk, ct = inputs(k, n, 70 + k)
+    full = pqc.Context([ALG[k]], max_batch=n)
+    total = full.device_bytes
+    want = full.dec_host(ALG[k], ct, sk)
+    full.close()
+    d_ct, d_sk = pqc.DeviceBuffer.from_array(ct), pqc.DeviceBuffer.from_array(sk)
+    ld = (n + 63) // 64 * 64
+    stage = (ld + 128) * (512 * k * k + 128) + 128 * 128 * (2 * k + 1)
+    for budget in (total, total - 1, total - stage // 3, total - stage):
+        print("budget k", k, budget, flush=True)
+        ctx = pqc.Context([ALG[k]], max_batch=n, hbm_budget=budget)
+        assert ctx.device_bytes <= budget
+        d_ss = pqc.DeviceBuffer(n * 32)
+        ctx.dec(ALG[k], n, d_ss, d_ct, d_sk)
+        ctx.take_status()
+        assert (d_ss.download((n, 32)) == want).all()
+        ctx.close()
+    with pytest.raises(Exception):
+        pqc.Context([ALG[k]], max_batch=n, hbm_budget=total - stage - 1)
