@@ -40,18 +40,18 @@ BYTES_PER_DECAPS = 1088 + 2400 + 32  # compulsory: ct in, sk in, ss out
 # measures the sustained issue rate on the box (pqc_valu_issue_rate).
 VALU_PEAK_TOPS = 256 * 4 * 64 / 2 * 2.4e9 / 1e12
 HBM_PEAK_GBPS = 8000.0
-# Bytes between L2 and memory per fused decapsulation launch at batch 65536
-# (k_fused_dec32<3>) from rocprofv3 FETCH_SIZE and WRITE_SIZE runs, each scaled
-# by the same counter's reading of a 256 MiB device copy
-# (profiles/kyber768_decaps_b65536.md): 786.8 MB read + 515.1 MB written.  Most of
-# it is the A^T scratch of the 32-request tiles, written and read back per wave.
-MEASURED_TRAFFIC_BYTES_B65536 = 1301.9e6
+# Bytes between L2 and memory per decapsulation call at batch 65536 (k_open, k_dec_sponge,
+# k_dec_reencrypt and k_dec_kdf together) from rocprofv3 FETCH_SIZE and WRITE_SIZE runs, each
+# scaled by the same counter's reading of a 256 MiB device copy
+# (profiles/stages_and_small_batches.md): 853 MB read + 378 MB written.  Most of it is the
+# sampled matrix entries and noise that the sponge stage writes and the next one reads.
+MEASURED_TRAFFIC_BYTES_B65536 = 1231e6
 # HBM bytes per Frodo-976 decapsulation GEMM launch at batch 4096, same method
 # (profiles/frodo976_decaps_b4096.md): 186.2 MB read + 0.07 MB written.
 MEASURED_TRAFFIC_FRODO_GEMM_B4096 = 186.3e6
 # HBM bytes per NewHope-1024 fused encryption launch at batch 16384, same method
-# (profiles/newhope1024_cpa_triples_b16384.md): 35.86 MB read + 35.65 MB written.
-MEASURED_TRAFFIC_NEWHOPE_ENC_B16384 = 71.5e6
+# (profiles/stages_and_small_batches.md): 31.5 MB read + 35.65 MB written.
+MEASURED_TRAFFIC_NEWHOPE_ENC_B16384 = 67.2e6
 
 
 def log(*a):
@@ -404,7 +404,7 @@ def main():
         },
         "roofline": {
             "bound": "valu",
-            "kernel": "k_fused_dec32<3> (fused Kyber-768 decaps, 32-request tiles, two waves per SIMD)",
+            "kernel": "k_open, k_dec_sponge, k_dec_reencrypt, k_dec_kdf (Kyber-768 decaps in stages)",
             "achieved": round(achieved, 3),
             "peak": round(VALU_PEAK_TOPS, 2),
             "unit": "Tops/s (int32)",
@@ -866,8 +866,8 @@ def run_mixed(args):
         off, cnt = lay.region["ss"][a]
         return _Slice(ss_dec, off, cnt * 32)
 
-    # the dominant kernel, k_fused_mixed_dec32, timed alone on the stream (with the
-    # descriptor classification it needs: two small kernels of ~40 us together)
+    # decapsulation's stages timed alone on the stream (with the descriptor
+    # classification they need: two small kernels of ~10 us together)
     dec_ms = timed_run(lambda: ctx.kem_dec_mixed(n, ar.dec_reqs, ar.buf["ct"], ar.buf["sk"], ss_dec, stream=stream),
                        stream, 10, 2, pqc)
     dec_ops = sum(lay.count[a] * MIXED_KECCAK_PER_DECAPS[a] for a in (1, 2, 3)) * OPS_PER_KECCAK
@@ -901,7 +901,7 @@ def run_mixed(args):
                    "batch_latency_ms_p50": round(float(np.percentile(per, 50)), 4),
                    "batch_latency_ms_p99": round(float(np.percentile(per, 99)), 4),
                    "bitexact_fused_plain": bitexact},
-        "roofline": {"bound": "valu", "kernel": "k_fused_mixed_dec32 (mixed decaps, 32-request tiles of all three parameter sets, two waves per SIMD)",
+        "roofline": {"bound": "valu", "kernel": "k_mixed_open, k_mixed_dec_sponge, k_mixed_encrypt, k_mixed_final (mixed decaps in stages)",
                      "achieved": round(dec_ops / dec_ms / 1e9, 3), "peak": VALU_PEAK_TOPS, "unit": "T int32 ops/s",
                      "frac": round(dec_ops / dec_ms / 1e9 / VALU_PEAK_TOPS, 4),
                      "work_per_launch": "Keccak-f per decaps 29 / 54 / 87 (Kyber-512 / 768 / 1024) x 7440 ops, "

@@ -83,7 +83,8 @@ typedef struct pqc_tuning {
                                  or lanes (calls above 4096 requests): 64, 128 or 256 */
   int32_t lowlat_max;         /* Kyber batches of at most this many requests run one
                                  workgroup per request (latency) instead of the throughput forms
-                                 below: 0 = library default (1280), -1 = never, else 1..65536;
+                                 below: 0 = library default (1280 for Kyber-512 and mixed, 1024, or 768
+                                 for Kyber-1024 encapsulation), -1 = never, else 1..65536;
                                  key generation with fused_key_tile = 64 never does */
   int32_t frodo_chunk;        /* FrodoKEM-976 batches under one key above this many requests are cut
                                  into chunks of this many, run on four streams: 0 = library default
@@ -231,7 +232,8 @@ int pqc_ctx_take_status(pqc_ctx *ctx, void *stream, uint32_t *status);
  * memory or call hipMalloc (code under HIP graph capture, tight serving loops,
  * harnesses that forbid allocation): Kyber-512/768/1024 decapsulation of n
  * ciphertexts with no context, bit-identical to crypto_kem_dec_batch with the
- * default tuning (the same kernels).  The tile kernel's scratch (PRF rows,
+ * default tuning (the per-request kernels up to 8192 requests, 64-request tiles
+ * above).  The tile kernel's scratch (PRF rows,
  * (2K+1) x 128 bytes per request) lives in a library-owned device array of
  * 256 + PQC_NOALLOC_MAX_BATCH x 1152 bytes (18.9 MB), one per GPU, held until
  * the process ends; nothing is allocated or freed per call.  n above

@@ -1,4 +1,6 @@
-// Fused persistent Kyber encapsulation / decapsulation.
+// Kyber dispatch, mixed-batch classification, and the fused persistent kernels over
+// 64-request tiles (tuning.fused_*_tile = 64, the allocation-free entry above 8192 requests,
+// contexts whose budget has no room for the staged path's scratch).
 //
 // One workgroup = one wave64; a persistent grid walks tiles of up to 64
 // requests.  Inside a tile the work is split two ways:
@@ -748,8 +750,8 @@ int kyber_fused_enc(pqc_ctx* c, int k, size_t n, uint8_t* ct, uint8_t* ss, const
   }
 }
 
-// Mixed Kyber-512/768/1024 batch: classify into buckets, then one persistent
-// launch.  Every launch has a fixed shape (the bucket sizes are read on the
+// Mixed Kyber-512/768/1024 batch: classify into buckets, then the stages (or one persistent
+// launch over 64-request tiles).  Every launch has a fixed shape (the bucket sizes are read on the
 // device), so the sequence can be captured into a graph and replayed.
 int kyber_fused_mixed(pqc_ctx* c, int dec, size_t n, const pqc_kem_req* reqs, uint8_t* ct, size_t ct_bytes,
                       const uint8_t* key, size_t key_bytes, uint8_t* ss, size_t ss_bytes, const uint8_t* coins,
