@@ -371,24 +371,34 @@ __global__ __launch_bounds__(256) void k_shake(int n, int npad, int with_f, FrKe
 
 // The same on 16 lanes per request (keccak_wide.cuh), four requests per wave: calls of
 // up to kWideMax requests, which leave SIMDs idle on lane pairs and are bound by the
-// serial chain.  Waves [0, ceil(n / 4)) are streams, written as k_shake writes them; waves
-// from there on (decapsulation) absorb the F prefixes.
-template <int W>
-__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_shake_wide(int n, FrKeys keys, const uint8_t* mu, int mu_stride,
-                                                   uint8_t* raw, uint8_t* kout, const uint8_t* ct, uint32_t* fstate) {
+// serial chain.  Streams are written as k_shake writes them; with_f (decapsulation), as many
+// waves absorb the F prefixes: behind the streams with one wave per workgroup, else half
+// of each workgroup, so that every CU has the same work.
+template <int WG>
+__global__ PQC_WIDE_KERNEL(WG) void k_shake_wide(int n, int with_f, FrKeys keys, const uint8_t* mu, int mu_stride,
+                                                 uint8_t* raw, uint8_t* kout, const uint8_t* ct, uint32_t* fstate) {
   __shared__ wide::Consts consts;
-  __shared__ wide::States states;
-  __shared__ uint32_t seed[4][8];
-  const int waves = (n + 3) / 4;
-  const int w0 = blockIdx.x;
+  __shared__ wide::States states[WG];
+  __shared__ uint32_t seeds[WG][4][8];
+  const int waves = (n + 3) / 4, wave = wide::wg_wave<WG>();
+  int w0 = wide::wave_of<WG>();
+  bool prefix = w0 >= waves;
+  if constexpr (WG == 1) {
+    w0 = prefix ? w0 - waves : w0;
+  } else if (with_f) {
+    prefix = wave >= WG / 2;
+    w0 = (int)blockIdx.x * (WG / 2) + wave % (WG / 2);
+  }
   wide::init_consts(consts);
   __syncthreads();
+  if (WG > 1 && w0 >= waves) return;
+  auto& seed = seeds[wave];
   wide::Sponge s;
-  s.init(states, consts);
-  const int rq = 4 * (w0 < waves ? w0 : w0 - waves) + s.st;
+  s.init(states[wave], consts);
+  const int rq = 4 * w0 + s.st;
   const bool act = rq < n;
   const int r = act ? rq : n - 1;
-  if (w0 >= waves) {
+  if (prefix) {
     s.absorb17<24>(reinterpret_cast<const uint32_t*>(ct + (size_t)r * CT), CT / 8, 0x1F, 0, (CT + SS) / 136);
     s.squeeze<5>([&](int x, uint32_t v) {
       const int w = s.word(x);
@@ -431,11 +441,18 @@ __global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_shake_wide(int n, FrKe
   s.absorb(m);
   // word x + 5 y of block b: its even-bit, then its odd-bit half
   uint32_t* out = reinterpret_cast<uint32_t*>(raw + (size_t)r * RAWB) + 2 * (5 * s.y) + s.h;
+  const bool col1 = act && s.word(1) < kRateShake256, col4 = act && s.word(4) < kRateShake256;
+  static_assert(kRateShake256 == 17, "17 words: three planes and two columns of the fourth");
   for (int blk = 0; blk < 231; ++blk) {
     s.permute<24>();
+    if (col1) {  // planes 0..3, then 0..2: a branch around each store costs a lone wave 2% of the stream
+      out[0] = s.a[0];
+      out[2] = s.a[1];
+      if (col4) {
 #pragma unroll
-    for (int x = 0; x < 5; ++x)
-      if (act && s.word(x) < kRateShake256) out[2 * x] = s.a[x];
+        for (int x = 2; x < 5; ++x) out[2 * x] = s.a[x];
+      }
+    }
     out += 2 * kRateShake256;
   }
 }
@@ -912,15 +929,16 @@ __global__ __launch_bounds__(64) void k_f_full(int n, uint8_t* ss, const uint8_t
 }
 
 // The same on 16 lanes per request
-template <int W>
-__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_f_full_wide(int n, uint8_t* ss, const uint8_t* ct, const uint8_t* kp) {
+template <int WG>
+__global__ PQC_WIDE_KERNEL(WG) void k_f_full_wide(int n, uint8_t* ss, const uint8_t* ct, const uint8_t* kp) {
   __shared__ wide::Consts consts;
-  __shared__ wide::States states;
+  __shared__ wide::States states[WG];
   wide::init_consts(consts);
   __syncthreads();
+  if (WG > 1 && 4 * wide::wave_of<WG>() >= n) return;
   wide::Sponge s;
-  s.init(states, consts);
-  const int rq = 4 * blockIdx.x + s.st;
+  s.init(states[wide::wg_wave<WG>()], consts);
+  const int rq = 4 * wide::wave_of<WG>() + s.st;
   const int r = rq < n ? rq : n - 1;
   const uint32_t* c = reinterpret_cast<const uint32_t*>(ct + (size_t)r * CT);
   const uint32_t* k = reinterpret_cast<const uint32_t*>(kp + (size_t)r * 32);
@@ -1064,16 +1082,17 @@ __global__ __launch_bounds__(64) void k_pkh_many(int n, uint8_t* pkh, size_t out
 }
 
 // The same on 16 lanes per key (a loaded public key; small batches)
-template <int W>
-__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_pkh_wide(int n, uint8_t* pkh, size_t out_stride, const uint8_t* pk,
-                                                 size_t pk_stride) {
+template <int WG>
+__global__ PQC_WIDE_KERNEL(WG) void k_pkh_wide(int n, uint8_t* pkh, size_t out_stride, const uint8_t* pk,
+                                               size_t pk_stride) {
   __shared__ wide::Consts consts;
-  __shared__ wide::States states;
+  __shared__ wide::States states[WG];
   wide::init_consts(consts);
   __syncthreads();
+  if (WG > 1 && 4 * wide::wave_of<WG>() >= n) return;
   wide::Sponge s;
-  s.init(states, consts);
-  const int rq = 4 * blockIdx.x + s.st;
+  s.init(states[wide::wg_wave<WG>()], consts);
+  const int rq = 4 * wide::wave_of<WG>() + s.st;
   const int r = rq < n ? rq : n - 1;
   s.absorb17<24>(reinterpret_cast<const uint32_t*>(pk + (size_t)r * pk_stride), PK / 8, 0x1F, 0, PK / 8 / 17 + 1);
   uint32_t* o = reinterpret_cast<uint32_t*>(pkh + (size_t)r * out_stride);
@@ -1248,17 +1267,20 @@ static FrKeys loaded_key(pqc_ctx* c) {
 
 // Calls of up to this many requests run their sponges on 16 lanes per request: one stream
 // wave per SIMD at 4096 (two with the F prefixes).  Measured on MI355X, us per call, lane
-// pairs and 16 lanes: decapsulation of 1 / 501 / 2048 / 4096 requests 1394 / 1182 / 1225 /
-// 1284 -> 769 / 790 / 871 / 950; encapsulation 2086 / 1912 / 1960 / 2019 -> 1122 / 1147 /
-// 1232 / 1286.  At 6000, pairs (one wave per SIMD or less) take 1361, about what 16 lanes
-// would at three waves per SIMD.
+// pairs and 16 lanes: decapsulation of 1 / 500 / 2048 / 4096 requests 1162 / 1186 / 1226 /
+// 1286 -> 764 / 788 / 865 / 941; encapsulation 2090 / 1918 / 1963 / 2023 -> 1118 / 1142 /
+// 1247 / 1265.  At 6000, pairs (one wave per SIMD or less) take 1361, about what 16 lanes
+// would at three waves per SIMD.  16 lanes cost more of the chip's time per permutation, so
+// four such calls side by side gain less: 2932 -> 3162 for decapsulations of 4096 (slower),
+// 2367 -> 1897 for 2048, 3886 -> 2985 for encapsulations of 4096.
 constexpr int kWideMax = 4096;
 
 static void launch_f_full(const pqc_ctx* c, int ni, uint8_t* ss, const uint8_t* ct, const uint8_t* kp, hipStream_t s) {
   const int waves = (ni + 3) / 4;
   if (ni <= kWideMax)
-    with_simd_waves(c->cu_count, waves, [&](auto w) {
-      hipLaunchKernelGGL(k_f_full_wide<decltype(w)::value>, dim3(waves), dim3(64), 0, s, ni, ss, ct, kp);
+    wide::with_wg(c->cu_count, waves, [&](auto wg) {
+      constexpr int WG = decltype(wg)::value;
+      hipLaunchKernelGGL(k_f_full_wide<WG>, wide::wg_grid(waves, WG), dim3(64 * WG), 0, s, ni, ss, ct, kp);
     });
   else
     hipLaunchKernelGGL(k_f_full, dim3((2 * ni + 63) / 64), dim3(64), 0, s, ni, ss, ct, kp);
@@ -1267,8 +1289,9 @@ static void launch_f_full(const pqc_ctx* c, int ni, uint8_t* ss, const uint8_t* 
 static void launch_pkh(const pqc_ctx* c, int m, uint8_t* pkh, size_t out_stride, const uint8_t* pk, size_t pk_stride, hipStream_t s) {
   const int waves = (m + 3) / 4;
   if (m <= kWideMax)
-    with_simd_waves(c->cu_count, waves, [&](auto w) {
-      hipLaunchKernelGGL(k_pkh_wide<decltype(w)::value>, dim3(waves), dim3(64), 0, s, m, pkh, out_stride, pk,
+    wide::with_wg(c->cu_count, waves, [&](auto wg) {
+      constexpr int WG = decltype(wg)::value;
+      hipLaunchKernelGGL(k_pkh_wide<WG>, wide::wg_grid(waves, WG), dim3(64 * WG), 0, s, m, pkh, out_stride, pk,
                          pk_stride);
     });
   else
@@ -1294,9 +1317,10 @@ static void launch_stream(pqc_ctx* c, const FrScratch& f, int ni, int with_f, co
   }
   if (ni <= kWideMax) {
     const int waves = (with_f ? 2 : 1) * ((ni + 3) / 4);
-    with_simd_waves(c->cu_count, waves, [&](auto w) {
-      hipLaunchKernelGGL(k_shake_wide<decltype(w)::value>, dim3(waves), dim3(64), 0, s, ni, keys, mu, mu_stride, f.raw,
-                         f.kp, ct, with_f ? f.fstate : (uint32_t*)nullptr);
+    wide::with_wg(c->cu_count, waves, [&](auto wg) {
+      constexpr int WG = decltype(wg)::value;
+      hipLaunchKernelGGL(k_shake_wide<WG>, wide::wg_grid(waves, WG), dim3(64 * WG), 0, s, ni, with_f, keys, mu,
+                         mu_stride, f.raw, f.kp, ct, with_f ? f.fstate : (uint32_t*)nullptr);
     });
     hipLaunchKernelGGL((k_sample<ROWS, true>), dim3((nt + 255) / 256), dim3(256), 0, s, ni, (const uint8_t*)f.raw,
                        f.sfrag, f.efrag);

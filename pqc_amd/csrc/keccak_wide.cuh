@@ -19,6 +19,8 @@
 #pragma once
 #include <stddef.h>
 
+#include <type_traits>
+
 #include "keccak.cuh"
 
 namespace pqc {
@@ -219,6 +221,45 @@ struct Sponge {
     }
   }
 };
+
+// ---- workgroups of the kernels with four chains per wave ----------------------------
+// WG waves per workgroup.  Chains finish soonest on SIMDs that hold as few of them as
+// possible.  The hardware spreads workgroups over CUs and a workgroup's waves over the
+// CU's four SIMDs, but not the waves of several one-wave workgroups on one CU.  So a
+// launch that needs a wave on most SIMDs takes four waves per workgroup, one of two waves
+// per SIMD eight: a workgroup per CU.  Launches of up to two waves per CU take one-wave
+// workgroups whose register allocation leaves no second place on a SIMD (as PQC_SIMD_WAVES
+// in internal.h): they fill at most half of the SIMDs, and up to four of them side by side
+// spread better than by workgroups (four calls of 500 FrodoKEM decapsulations 860 us,
+// 1209 with four waves per workgroup).  A larger launch must not take whole SIMDs: it
+// shuts out whatever runs beside it on other streams.  Measured, four contexts on four
+// streams, us per round of calls, registers rounded up to one or two waves per SIMD ->
+// this: FrodoKEM-976 encapsulation of 4096 5061 -> 2985 (one call 1295 -> 1260),
+// decapsulation of 2048 2618 -> 1897 and of 4096 3418 -> 3162; NewHope-1024 CCA
+// encapsulation of 3000 408 -> 320 and of 8000 836 -> 770.
+#define PQC_WIDE_KERNEL(WG) \
+  __launch_bounds__(64 * (WG)) __attribute__((amdgpu_waves_per_eu((WG) == 1 ? 1 : 4, (WG) == 1 ? 1 : 8)))
+
+template <int WG>
+__device__ __forceinline__ int wg_wave() {
+  return WG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+}
+template <int WG>
+__device__ __forceinline__ int wave_of() {
+  return (int)blockIdx.x * WG + wg_wave<WG>();
+}
+
+// f(std::integral_constant<int, WG>) for a launch of `waves` waves on `cus` CUs
+template <class F>
+inline void with_wg(int cus, int waves, F&& f) {
+  if (waves <= 2 * cus)
+    f(std::integral_constant<int, 1>{});
+  else if (waves <= 4 * cus)
+    f(std::integral_constant<int, 4>{});
+  else
+    f(std::integral_constant<int, 8>{});
+}
+inline dim3 wg_grid(int waves, int wg) { return dim3((unsigned)((waves + wg - 1) / wg)); }
 
 }  // namespace wide
 }  // namespace pqc

@@ -19,6 +19,8 @@
 // out-of-range ones.  N = 512 follows the reference's NEWHOPE_N == 512 branches
 // (precomp.cu:75-190 tables, ntt.cu:130-180, poly.cu:244,279), which its
 // batched GPU path never compiled.
+#include <type_traits>
+
 #include "internal.h"
 #include "keccak_wide.cuh"
 #include "sponge.cuh"
@@ -1274,28 +1276,34 @@ static_assert(KM_CT2 + Par<1024>::CCA_CT == kNewhopeKemBytes, "scratch row size"
 // step between two of them is a launch of its own.  Here four elements share a wave, and
 // the copies, the comparison and the selection belong to the kernel that hashes next to
 // them.  One encapsulation and decapsulation per element, us, lane-pair form -> this one:
-// N = 512: 308 -> 141 (7 elements), 325 -> 189 (3001), 368 -> 292 (8192), 490 -> 548
+// N = 512: 308 -> 141 (7 elements), 323 -> 161 (3001), 368 -> 274 (8192), 490 -> 548
 // (16384: the pair form's 512 waves are still one per SIMD, these would be four);
-// N = 1024: 506 -> 211, 533 -> 286, 585 -> 456, 753 -> 905.
+// N = 1024: 506 -> 211, 530 -> 260, 585 -> 439, 753 -> 905.
 constexpr int kWideMax = 8192;
+// Decapsulation's H(c) runs beside the decryption and re-encryption.  Above this the
+// lane-pair form still ends before they do and leaves them more of the chip: N = 1024, 8000
+// elements, one call 189 us either way, two calls side by side 428 -> 344.
+constexpr int kSideWideMax = 4096;
 
-struct Wide4 {
-  wide::Consts consts;
+struct Wide4 {  // one wave's
   wide::States states;
   alignas(16) uint32_t dig[4][16];  // per element: the words of its next short message
 };
 
 // out[x] = SHAKE256(in[x], 8 words bytes), 32 bytes
-template <int W>
-__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_shake256_wide(int n, uint8_t* out, size_t out_stride,
+template <int WG>
+__global__ PQC_WIDE_KERNEL(WG) void k_shake256_wide(int n, uint8_t* out, size_t out_stride,
                                                                         const uint8_t* in, size_t in_stride,
                                                                         int words) {
-  __shared__ Wide4 sh;
-  wide::init_consts(sh.consts);
+  __shared__ wide::Consts consts;
+  __shared__ Wide4 lds[WG];
+  wide::init_consts(consts);
   __syncthreads();
+  if (WG > 1 && 4 * wide::wave_of<WG>() >= n) return;
+  Wide4& sh = lds[wide::wg_wave<WG>()];
   wide::Sponge s;
-  s.init(sh.states, sh.consts);
-  const int rq = 4 * blockIdx.x + s.st, r = rq < n ? rq : n - 1;
+  s.init(sh.states, consts);
+  const int rq = 4 * wide::wave_of<WG>() + s.st, r = rq < n ? rq : n - 1;
   s.absorb17<24>(reinterpret_cast<const uint32_t*>(in + (size_t)r * in_stride), words, 0x1F, 0, words / 17 + 1);
   uint32_t* o = reinterpret_cast<uint32_t*>(out + (size_t)r * out_stride);
   s.squeeze<4>([&](int x, uint32_t v) {
@@ -1306,16 +1314,19 @@ __global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_shake256_wide(int n, u
 // (K || coin || d) = SHAKE256(mu || H(pk), 96).  Encapsulation (ENC): mu = H(in[x], 32
 // bytes), kept in the row, and H(pk) of the public key key[x] (words 64-bit words);
 // decapsulation: m' of the row and the H(pk) that key[x] holds.
-template <int W, bool ENC>
-__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_cca_open_wide(int n, uint8_t* km, const uint8_t* in,
+template <int WG, bool ENC>
+__global__ PQC_WIDE_KERNEL(WG) void k_cca_open_wide(int n, uint8_t* km, const uint8_t* in,
                                                                         const uint8_t* key, size_t key_stride,
                                                                         int words) {
-  __shared__ Wide4 sh;
-  wide::init_consts(sh.consts);
+  __shared__ wide::Consts consts;
+  __shared__ Wide4 lds[WG];
+  wide::init_consts(consts);
   __syncthreads();
+  if (WG > 1 && 4 * wide::wave_of<WG>() >= n) return;
+  Wide4& sh = lds[wide::wg_wave<WG>()];
   wide::Sponge s;
-  s.init(sh.states, sh.consts);
-  const int rq = 4 * blockIdx.x + s.st, r = rq < n ? rq : n - 1;
+  s.init(sh.states, consts);
+  const int rq = 4 * wide::wave_of<WG>() + s.st, r = rq < n ? rq : n - 1;
   const bool act = rq < n;
   uint32_t* row = reinterpret_cast<uint32_t*>(km + (size_t)r * kNewhopeKemBytes);
   const uint32_t* kp = reinterpret_cast<const uint32_t*>(key + (size_t)r * key_stride);
@@ -1348,17 +1359,20 @@ __global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_cca_open_wide(int n, u
 // here.  Decapsulation: H(c) is in the row, and the element's 16 lanes compare ct[x] with
 // the re-encryption and d, all of it (verify.cu:15-28 without its data-dependent branch);
 // on any difference z[x] takes the place of K by mask (verify.cu:40-50).
-template <int W, bool ENC, int N>
-__global__ __launch_bounds__(64) PQC_SIMD_WAVES(W) void k_cca_close_wide(
+template <int WG, bool ENC, int N>
+__global__ PQC_WIDE_KERNEL(WG) void k_cca_close_wide(
     int n, uint8_t* ss, const uint8_t* km, std::conditional_t<ENC, uint8_t*, const uint8_t*> ct, const uint8_t* z,
     size_t z_stride) {
   using P = Par<N>;
-  __shared__ Wide4 sh;
-  wide::init_consts(sh.consts);
+  __shared__ wide::Consts consts;
+  __shared__ Wide4 lds[WG];
+  wide::init_consts(consts);
   __syncthreads();
+  if (WG > 1 && 4 * wide::wave_of<WG>() >= n) return;
+  Wide4& sh = lds[wide::wg_wave<WG>()];
   wide::Sponge s;
-  s.init(sh.states, sh.consts);
-  const int rq = 4 * blockIdx.x + s.st, r = rq < n ? rq : n - 1;
+  s.init(sh.states, consts);
+  const int rq = 4 * wide::wave_of<WG>() + s.st, r = rq < n ? rq : n - 1;
   const bool act = rq < n;
   const uint32_t* row = reinterpret_cast<const uint32_t*>(km + (size_t)r * kNewhopeKemBytes);
   const uint32_t* d = row + KM_KCD / 4 + 16;
@@ -1413,10 +1427,11 @@ inline dim3 elem_grid(int n) { return dim3((unsigned)((n + kElems - 1) / kElems)
 #define LAUNCH(kern, threads, ...) hipLaunchKernelGGL(kern, L.grid(threads), dim3(L.block), 0, s, __VA_ARGS__)
 #define LAUNCH_NTT(kern, ...) hipLaunchKernelGGL(kern, dim3(n), dim3(64), 0, s, __VA_ARGS__)
 
-// kernel template NAME<W, ...> on a wave per four elements
-#define LAUNCH_WIDE(NAME, TARGS, st, ...)                                                                  \
-  with_simd_waves(c->cu_count, (n + 3) / 4, [&](auto w_) {                                                 \
-    hipLaunchKernelGGL((NAME<decltype(w_)::value PQC_UNPAREN TARGS>), dim3((n + 3) / 4), dim3(64), 0, st, __VA_ARGS__); \
+// kernel template NAME<WG, ...> on a wave per four elements
+#define LAUNCH_WIDE(NAME, TARGS, st, ...)                                                                            \
+  wide::with_wg(c->cu_count, (n + 3) / 4, [&](auto wg_) {                                                            \
+    constexpr int WG = decltype(wg_)::value;                                                                         \
+    hipLaunchKernelGGL((NAME<WG PQC_UNPAREN TARGS>), wide::wg_grid((n + 3) / 4, WG), dim3(64 * WG), 0, st, __VA_ARGS__); \
   })
 #define PQC_UNPAREN(...) __VA_OPT__(,) __VA_ARGS__
 
@@ -1508,10 +1523,10 @@ int dec_impl(pqc_ctx* c, int n, uint8_t* m, size_t m_stride, const uint8_t* ct, 
 }
 
 // out[x] = SHAKE256(in[x], 8 words bytes), 32 bytes, of a public key or a ciphertext
-inline void hash32(pqc_ctx* c, int n, uint8_t* out, size_t out_stride, const uint8_t* in, size_t in_stride, int words,
-                   hipStream_t s) {
+inline void hash32(const pqc_ctx* c, int n, uint8_t* out, size_t out_stride, const uint8_t* in, size_t in_stride,
+                   int words, hipStream_t s, int wide_max = kWideMax) {
   const Launch L{c->tune.newhope_block};
-  if (n <= kWideMax)
+  if (n <= wide_max)
     LAUNCH_WIDE(k_shake256_wide, (), s, n, out, out_stride, in, in_stride, words);
   else
     LAUNCH(k_shake256_pair<4>, 2 * (size_t)n, n, out, out_stride, in, in_stride, words);
@@ -1572,7 +1587,7 @@ int cca_dec(pqc_ctx* c, size_t n_, uint8_t* ss, const uint8_t* ct, const uint8_t
   // stream beside the decryption and re-encryption, and joins before the key selection
   if (hipEventRecord(c->nh_fork, s) != hipSuccess || hipStreamWaitEvent(c->nh_side, c->nh_fork, 0) != hipSuccess)
     return PQC_ERR_DEVICE;
-  hash32(c, n, km + KM_HC, kb, ct, P::CCA_CT, P::CCA_CT / 8, c->nh_side);
+  hash32(c, n, km + KM_HC, kb, ct, P::CCA_CT, P::CCA_CT / 8, c->nh_side, kSideWideMax);
   if (hipGetLastError() != hipSuccess || hipEventRecord(c->nh_join, c->nh_side) != hipSuccess) return PQC_ERR_DEVICE;
   int rc = dec_impl<N>(c, n, km + KM_MU, kb, ct, P::CCA_CT, sk, P::CCA_SK, plain, s);  // m'
   if (rc) {
