@@ -693,6 +693,20 @@ static int launch_fused(pqc_ctx* c, size_t n, uint8_t* ss, uint8_t* ct, const ui
 constexpr int kLowLatMixed = 1280;
 constexpr int lowlat_limit(int k, bool enc) { return k == 2 ? 1280 : k == 4 && enc ? 768 : 1024; }
 
+// Larger batches run in stages unless `tile` (a fused_*_tile knob) says 64-request tiles or
+// the context's budget left no scratch for the stages, or so little that the batch would
+// take many passes of them: a pass lasts ~95 (Kyber-512) to ~160 us however short it is, 230
+// to 320 mixed, where one tile launch does up to 65536 requests in 510, 880, 1290 us (mixed
+// 1320).  Measured on MI355X, us, 2 / 4 / 8 passes and tiles: 65536 Kyber-768
+// encapsulations 746 / 1147 / 1664 and 885, 16384 of them 418 / 597 / 1061 and 871; Kyber-512
+// 501 / 764 / 1192 and 508, 298 / 481 / 855 and 496; mixed 970 / 1403 / 2566 and 1313, 643 /
+// 1280 / 2513 and 1293.
+inline bool use_stages(const pqc_ctx* c, size_t n, int tile) {
+  if (!c->kat || tile == 64 || n == 0) return false;
+  const size_t block = std::min<size_t>(n, 65536);  // no pass is longer
+  return (block + c->kstage_max - 1) / c->kstage_max <= (block <= 16384 ? 4 : 2);
+}
+
 inline bool use_lowlat(const pqc_ctx* c, size_t n, int dflt) {
   const int lim = c->tune.lowlat_max != 0 ? c->tune.lowlat_max : dflt;
   return n > 0 && (long long)n <= (long long)lim;
@@ -716,7 +730,7 @@ static int launch_fused_keypair(pqc_ctx* c, size_t n, uint8_t* pk, uint8_t* sk, 
 int kyber_fused_keypair(pqc_ctx* c, int k, size_t n, uint8_t* pk, uint8_t* sk, const uint8_t* coins, hipStream_t s) {
   if (c->tune.fused_key_tile != 64 && kyber::fused::use_lowlat(c, n, kyber::fused::lowlat_limit(k, false)))
     return kyber_lowlat_keypair(k, n, pk, sk, coins, c->status, s);
-  if (n > 0 && c->kat && c->tune.fused_key_tile != 64) return kyber_staged_keypair(c, k, n, pk, sk, coins, s);
+  if (kyber::fused::use_stages(c, n, c->tune.fused_key_tile)) return kyber_staged_keypair(c, k, n, pk, sk, coins, s);
   switch (k) {
     case 2: return kyber::fused::launch_fused_keypair<2>(c, n, pk, sk, coins, s);
     case 3: return kyber::fused::launch_fused_keypair<3>(c, n, pk, sk, coins, s);
@@ -728,7 +742,7 @@ int kyber_fused_keypair(pqc_ctx* c, int k, size_t n, uint8_t* pk, uint8_t* sk, c
 int kyber_fused_dec(pqc_ctx* c, int k, size_t n, uint8_t* ss, const uint8_t* ct, const uint8_t* sk, hipStream_t s) {
   uint8_t* ctm = const_cast<uint8_t*>(ct);  // read-only in the decaps instantiation
   if (kyber::fused::use_lowlat(c, n, kyber::fused::lowlat_limit(k, false))) return kyber_lowlat_dec(k, n, ss, ct, sk, c->status, s);
-  if (n > 0 && c->kat && c->tune.fused_dec_tile != 64) return kyber_staged_dec(c, k, n, ss, ct, sk, s);
+  if (kyber::fused::use_stages(c, n, c->tune.fused_dec_tile)) return kyber_staged_dec(c, k, n, ss, ct, sk, s);
   switch (k) {
     case 2: return kyber::fused::launch_fused<2, true>(c, n, ss, ctm, sk, nullptr, s);
     case 3: return kyber::fused::launch_fused<3, true>(c, n, ss, ctm, sk, nullptr, s);
@@ -741,7 +755,7 @@ int kyber_fused_enc(pqc_ctx* c, int k, size_t n, uint8_t* ct, uint8_t* ss, const
                     hipStream_t s) {
   if (kyber::fused::use_lowlat(c, n, kyber::fused::lowlat_limit(k, true)))
     return kyber_lowlat_enc(k, n, ct, ss, pk, coins, c->status, s);
-  if (n > 0 && c->kat && c->tune.fused_enc_tile != 64) return kyber_staged_enc(c, k, n, ct, ss, pk, coins, s);
+  if (kyber::fused::use_stages(c, n, c->tune.fused_enc_tile)) return kyber_staged_enc(c, k, n, ct, ss, pk, coins, s);
   switch (k) {
     case 2: return kyber::fused::launch_fused<2, false>(c, n, ss, ct, pk, coins, s);
     case 3: return kyber::fused::launch_fused<3, false>(c, n, ss, ct, pk, coins, s);
@@ -770,7 +784,7 @@ int kyber_fused_mixed(pqc_ctx* c, int dec, size_t n, const pqc_kem_req* reqs, ui
                        c->status);
   };
   kyber::MixedSrc src{reqs, c->kmix_order, cap, ss, ct, key, coins, c->kprf, c->kprf_per_elem};
-  if (c->kat && (dec ? c->tune.fused_dec_tile : c->tune.fused_enc_tile) != 64) {
+  if (use_stages(c, n, dec ? c->tune.fused_dec_tile : c->tune.fused_enc_tile)) {
     // in stages, kstage_max requests at a time (their scratch)
     for (size_t at = 0; at < n; at += c->kstage_max) {
       const size_t m = std::min(n - at, c->kstage_max);

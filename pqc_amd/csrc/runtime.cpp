@@ -356,8 +356,8 @@ extern "C" {
 // Noise rows of the Kyber kernels and the scratch of the staged path for up to kstage_max
 // requests (groups of 16 of each parameter set, read in tiles of 64: under 128 rows of
 // padding); larger batches run in passes.  A budget that leaves less room gets shorter
-// passes, and one that holds the noise rows alone none: batches then run in 64-request
-// tiles.
+// passes, and one that holds the noise rows alone none: batches that no stage or too many
+// passes are left for run in 64-request tiles (use_stages, kyber_fused.hip).
 static int alloc_kyber_stage(pqc_ctx* c, int kmax) {
   const size_t at = pqc::kyber_stage_at_bytes(kmax);
   for (size_t stage = std::min<size_t>(c->ld, 65536);; stage = stage > 64 ? stage / 2 & ~(size_t)63 : 0) {
