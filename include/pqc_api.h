@@ -83,8 +83,9 @@ typedef struct pqc_tuning {
                                  or lanes (calls above 4096 requests): 64, 128 or 256 */
   int32_t lowlat_max;         /* Kyber batches of at most this many requests run one
                                  workgroup per request (latency) instead of the throughput forms
-                                 below: 0 = library default (1280 for Kyber-512 and mixed, 1024, or 768
-                                 for Kyber-1024 encapsulation), -1 = never, else 1..65536;
+                                 below: 0 = library default (1280 for Kyber-512 and mixed encapsulation,
+                                 1536 for mixed decapsulation, 768 for Kyber-1024 encapsulation, else
+                                 1024), -1 = never, else 1..65536;
                                  key generation with fused_key_tile = 64 never does */
   int32_t frodo_chunk;        /* FrodoKEM-976 batches under one key above this many requests are cut
                                  into chunks of this many, run on four streams: 0 = library default

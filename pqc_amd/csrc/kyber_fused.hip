@@ -687,10 +687,12 @@ static int launch_fused(pqc_ctx* c, size_t n, uint8_t* ss, uint8_t* ct, const ui
 // staged, us: Kyber-512 encapsulation 101 / 104 at 1280; Kyber-768 decapsulation 91 / 102 at
 // 1024 and 127 / 104 at 1280, encapsulation 121 / 123 and 170 / 128, key generation 91 / 116
 // and 122 / 118; Kyber-1024 decapsulation 122 / 126 and 172 / 135, key generation 134 / 150
-// and 171 / 154, encapsulation 132 / 159 at 768 and 198 / 158 at 1024.  Mixed batches (the
-// stages read their sizes on the device) 149 / 159 at 1500 requests of decapsulation.
+// and 171 / 154, encapsulation 132 / 159 at 768 and 198 / 158 at 1024.  Mixed batches, whose
+// stages hash on one lane per request: decapsulation 181 / 213 at 1536 (1:2:1; Kyber-512
+// alone 109 / 116 at 1500) and 230 / 220 at 2048, encapsulation 253 / 308 at 1281 and 323 /
+// 311 at 1800, but Kyber-512 alone 174 / 179 and 193 / 178 at 1500.
 // tuning.lowlat_max overrides them all (-1 = never).
-constexpr int kLowLatMixed = 1280;
+constexpr int lowlat_mixed(bool dec) { return dec ? 1536 : 1280; }
 constexpr int lowlat_limit(int k, bool enc) { return k == 2 ? 1280 : k == 4 && enc ? 768 : 1024; }
 
 // Larger batches run in stages unless `tile` (a fused_*_tile knob) says 64-request tiles or
@@ -773,7 +775,7 @@ int kyber_fused_mixed(pqc_ctx* c, int dec, size_t n, const pqc_kem_req* reqs, ui
   using namespace kyber::fused;
   if (n == 0) return PQC_OK;
   if (!c->kmix_order || !c->kprf) return PQC_ERR_UNSUPPORTED;
-  if (use_lowlat(c, n, kLowLatMixed))  // one workgroup per descriptor, no bucketing
+  if (use_lowlat(c, n, lowlat_mixed(dec != 0)))  // one workgroup per descriptor, no bucketing
     return kyber_lowlat_mixed(c, dec, n, reqs, ct, ct_bytes, key, key_bytes, ss, ss_bytes, coins, coins_bytes, s);
   const int cap = (int)c->max_batch;
   auto classify = [&](const pqc_kem_req* r, size_t m) {
