@@ -91,7 +91,7 @@ struct Slot {
   std::vector<size_t> out_a, out_b, len_a, len_b;  // where each request's output lies in h_out
   std::vector<size_t> in_at;                       // where each request's input goes in h_in
   uint32_t* h_status = nullptr;  // pinned: status of ctx and ctx_fd after the batch; [2]: ctx after the Kyber part
-  std::map<uint32_t, hipGraphExec_t> graphs;  // graph mode: one executable per batch shape (groups present)
+  std::map<uint64_t, hipGraphExec_t> graphs;  // graph mode: one executable per sequence of nodes (graph_key)
   size_t bytes = 0;
   bool busy = false;
   int cls = kAnyClass;  // which requests the slot takes (split pools: Kyber or Frodo only)
@@ -135,10 +135,14 @@ namespace {
 
 constexpr size_t kCopyPer = 128;  // requests per copy thread (about 140 KB of Kyber-768 ciphertexts)
 
-void free_slot(Slot& sl) {
+void free_graphs(Slot& sl) {
   for (auto& g : sl.graphs)
     if (g.second) (void)hipGraphExecDestroy(g.second);
   sl.graphs.clear();
+}
+
+void free_slot(Slot& sl) {
+  free_graphs(sl);
   if (sl.ctx) pqc_ctx_destroy(sl.ctx);
   if (sl.ctx_fd) pqc_ctx_destroy(sl.ctx_fd);
   for (hipStream_t t : {sl.s, sl.s2, sl.s3})
@@ -158,13 +162,45 @@ void free_server(pqc_server* v) {
   delete v;
 }
 
-// Graph mode: the slot's executable graph for this batch shape takes the new
-// batch's parameters (sizes, counts, grids) by an in-place update; a first batch
-// of a shape, or an update the runtime refuses (a different kernel, say), makes
-// a new executable.  The slot's previous batch has finished before the slot is
-// reused, so no update touches a graph in flight.
-int launch_graph(Slot& sl, uint32_t shape, hipGraph_t g, hipStream_t st) {
-  hipGraphExec_t& ex = sl.graphs[shape];
+constexpr size_t kMaxGraphs = 64;
+
+// A hash of the captured nodes' types and kernels.  Batches of different sizes take
+// different kernels (per request, in stages, workgroup shapes): one executable per batch
+// shape alone would be made anew whenever the size crosses such a line (50 to 70 us a time
+// in batches of 900 and 2000 Kyber-768 decapsulations in turn).
+bool graph_key(hipGraph_t g, uint64_t* key) {
+  hipGraphNode_t nodes[256];
+  size_t n = 0;
+  if (hipGraphGetNodes(g, nullptr, &n) != hipSuccess || n > 256) return false;
+  if (n && hipGraphGetNodes(g, nodes, &n) != hipSuccess) return false;
+  uint64_t h = 0xCBF29CE484222325ull + n;
+  for (size_t i = 0; i < n; ++i) {
+    hipGraphNodeType type;
+    if (hipGraphNodeGetType(nodes[i], &type) != hipSuccess) return false;
+    uint64_t v = (uint64_t)type;
+    if (type == hipGraphNodeTypeKernel) {
+      hipKernelNodeParams p{};
+      if (hipGraphKernelNodeGetParams(nodes[i], &p) != hipSuccess) return false;
+      v ^= (uint64_t)(uintptr_t)p.func;
+    }
+    h = (h ^ v) * 0x100000001B3ull;
+  }
+  *key = h;
+  return true;
+}
+
+// Graph mode: the slot's executable for these nodes takes the new batch's parameters
+// (sizes, counts, grids) by an in-place update; a first batch of them, or an update the
+// runtime refuses, makes a new executable.  The slot's previous batch has finished
+// before the slot is reused, so no update touches a graph in flight.
+int launch_graph(Slot& sl, hipGraph_t g, hipStream_t st) {
+  uint64_t key = 0;
+  if (!graph_key(g, &key)) {
+    (void)hipGetLastError();
+    key = 0;
+  }
+  if (sl.graphs.size() >= kMaxGraphs && !sl.graphs.count(key)) free_graphs(sl);
+  hipGraphExec_t& ex = sl.graphs[key];
   if (ex) {
     hipGraphNode_t bad = nullptr;
     hipGraphExecUpdateResult res = hipGraphExecUpdateSuccess;
@@ -369,9 +405,7 @@ int launch(pqc_server* v, Slot& sl) {
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(st, &g);
     if (!rc && (e != hipSuccess || !g)) rc = PQC_ERR_DEVICE;
-    uint32_t shape = 0;
-    for (int k = 0; k < kGroups; ++k) shape |= cnt[k] ? 1u << k : 0u;
-    if (!rc) rc = launch_graph(sl, shape, g, st);
+    if (!rc) rc = launch_graph(sl, g, st);
     if (g) (void)hipGraphDestroy(g);
   }
   if (rc) return rc;
