@@ -140,7 +140,9 @@ int crypto_kem_enc_batch(pqc_ctx *ctx, int alg, size_t n, uint8_t *ct, uint8_t *
  * Times the candidate configurations of one workload family (the knobs that
  * family uses) with HIP events and keeps every measurement as a sample
  * (14 features, log ms) in the context.  `run` launches the workload once,
- * asynchronously, on the given stream and returns 0 or a PQC_ERR code.
+ * asynchronously, on the given stream and returns 0 or a PQC_ERR code.  It first
+ * runs for ~30 ms as configured, then the candidates take turns, so that clocks
+ * that settle or drift meanwhile favour none of them.
  * use_model = 0: candidates in a fixed order (the configuration in use first)
  * up to `budget` (0 = all).  use_model = 1: once the context's learned cost
  * model has been fitted (after the first use_model call), it ranks all

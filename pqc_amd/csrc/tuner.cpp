@@ -4,9 +4,10 @@
 //
 // A tuning request names a workload family (which knobs apply), its batch size
 // and parameter set, and a callback that runs the workload once on a stream.
-// Each candidate configuration is timed with HIP events (median of `reps`
-// runs after one warm-up) and kept as a sample (features, log ms) in the
-// context.  Without the cost model the candidates are measured in a fixed order
+// The GPU runs the configuration in use until its clocks have settled, then the
+// candidates take turns, one run each, timed with HIP events: whatever drifts
+// during the measurement meets all of them alike.  The median of a candidate's
+// `reps` runs is kept as a sample (features, log ms) in the context.  Without the cost model the candidates are measured in a fixed order
 // (current configuration first) up to the budget; with it, the model trained on
 // every sample so far ranks all candidates and only the best-ranked `budget` are
 // measured, after which the model is refitted with the new samples.
@@ -127,33 +128,58 @@ static bool same(const pqc_tuning& a, const pqc_tuning& b) {
          lane_min_of(a.frodo_lane_min) == lane_min_of(b.frodo_lane_min);
 }
 
-// median of reps timed runs (one untimed warm-up first)
-static int measure(pqc_ctx* c, const pqc_tuning& t, pqc_workload_fn run, void* user, hipStream_t s, int reps,
-                   float* ms) {
-  c->tune = t;
-  int rc = run(user, (void*)s);
-  if (rc) return rc;
-  hipEvent_t a, b;
-  if (hipEventCreate(&a) != hipSuccess) return PQC_ERR_DEVICE;
-  if (hipEventCreate(&b) != hipSuccess) {
-    (void)hipEventDestroy(a);
-    return PQC_ERR_DEVICE;
+struct Timer {
+  hipEvent_t a = nullptr, b = nullptr;
+  int create() {
+    return hipEventCreate(&a) == hipSuccess && hipEventCreate(&b) == hipSuccess ? PQC_OK : PQC_ERR_DEVICE;
   }
-  std::vector<float> v;
-  for (int i = 0; i < reps && rc == PQC_OK; ++i) {
-    if (hipEventRecord(a, s) != hipSuccess) rc = PQC_ERR_DEVICE;
-    if (!rc) rc = run(user, (void*)s);
-    if (!rc && hipEventRecord(b, s) != hipSuccess) rc = PQC_ERR_DEVICE;
-    if (!rc && hipEventSynchronize(b) != hipSuccess) rc = PQC_ERR_DEVICE;
-    float e = 0.f;
-    if (!rc && hipEventElapsedTime(&e, a, b) != hipSuccess) rc = PQC_ERR_DEVICE;
-    v.push_back(e);
+  ~Timer() {
+    if (a) (void)hipEventDestroy(a);
+    if (b) (void)hipEventDestroy(b);
   }
-  (void)hipEventDestroy(a);
-  (void)hipEventDestroy(b);
+  // one run, its time in ms
+  int run(pqc_workload_fn fn, void* user, hipStream_t s, float* ms) {
+    if (hipEventRecord(a, s) != hipSuccess) return PQC_ERR_DEVICE;
+    const int rc = fn(user, (void*)s);
+    if (rc) return rc;
+    if (hipEventRecord(b, s) != hipSuccess || hipEventSynchronize(b) != hipSuccess ||
+        hipEventElapsedTime(ms, a, b) != hipSuccess)
+      return PQC_ERR_DEVICE;
+    return PQC_OK;
+  }
+};
+
+// After an idle phase the GPU's first tens of milliseconds of work run up to ~10% slower:
+// about what the candidates differ by (mixed batches of 65536: 1.68 ms were chosen over the
+// 1.49 of the configuration in use, which had been measured by itself right after the
+// model's predictions).
+constexpr float kWarmMs = 30.f;
+constexpr int kWarmRuns = 1000;
+
+// ms[i]: median time of cand[order[i]], i < n
+static int measure(pqc_ctx* c, const std::vector<pqc_tuning>& cand, const std::vector<size_t>& order, size_t n,
+                   pqc_workload_fn run, void* user, hipStream_t s, int reps, std::vector<float>& ms) {
+  Timer t;
+  int rc = t.create();
+  float e = 0.f, warm = 0.f;
+  for (int i = 0; !rc && i < kWarmRuns && warm < kWarmMs; ++i) {
+    rc = t.run(run, user, s, &e);
+    warm += e;
+  }
+  std::vector<std::vector<float>> v(n);
+  for (int r = 0; !rc && r < reps; ++r)
+    for (size_t i = 0; !rc && i < n; ++i) {
+      c->tune = cand[order[i]];
+      if (r == 0) rc = run(user, (void*)s);  // untimed: a configuration's first run
+      if (!rc) rc = t.run(run, user, s, &e);
+      v[i].push_back(e);
+    }
   if (rc) return rc;
-  std::sort(v.begin(), v.end());
-  *ms = v[v.size() / 2];
+  ms.clear();
+  for (auto& x : v) {
+    std::sort(x.begin(), x.end());
+    ms.push_back(x[x.size() / 2]);
+  }
   return PQC_OK;
 }
 
@@ -244,23 +270,21 @@ int pqc_autotune(pqc_ctx* c, const pqc_tune_request* r, pqc_workload_fn run, voi
   const size_t budget = r->budget == 0 ? cand.size() : std::min<size_t>(r->budget, cand.size());
   float best_ms = 0.f;
   size_t best = order[0];
-  int rc = PQC_OK;
-  for (size_t j = 0; j < budget; ++j) {
-    float ms = 0.f;
-    rc = measure(c, cand[order[j]], run, user, s, r->reps, &ms);
-    if (rc) break;
-    float f[kFeatures];
-    features(*r, cand[order[j]], f);
-    S->x.insert(S->x.end(), f, f + kFeatures);
-    S->y.push_back(std::log(std::max(ms, 1e-4f)));
-    if (j == 0 || ms < best_ms) {
-      best_ms = ms;
-      best = order[j];
-    }
-  }
+  std::vector<float> ms;
+  int rc = measure(c, cand, order, budget, run, user, s, r->reps, ms);
   if (rc) {
     c->tune = start;
     return rc;
+  }
+  for (size_t j = 0; j < budget; ++j) {
+    float f[kFeatures];
+    features(*r, cand[order[j]], f);
+    S->x.insert(S->x.end(), f, f + kFeatures);
+    S->y.push_back(std::log(std::max(ms[j], 1e-4f)));
+    if (j == 0 || ms[j] < best_ms) {
+      best_ms = ms[j];
+      best = order[j];
+    }
   }
   c->tune = cand[best];
   out->best = cand[best];
