@@ -79,8 +79,9 @@ typedef struct pqc_tuning {
                                  many sponge waves per SIMD and half as many product workgroups per CU */
   int32_t mixed_order;        /* mixed-batch tile order: 0 = K 4,3,2; 1 = K 2,3,4; 2 = round-robin over K;
                                  3 = K 4,3,2 with 32-request tiles for K = 4 and K = 2 */
-  int32_t frodo_stream_block; /* threads per workgroup of the Frodo noise-stream kernel on lane pairs
-                                 or lanes (calls above 4096 requests): 64, 128 or 256 */
+  int32_t frodo_stream_block; /* threads per workgroup of the Frodo noise-stream kernel on lane pairs or
+                                 single lanes (not on 16 lanes, the default up to 4096 requests): 64,
+                                 128 or 256 */
   int32_t lowlat_max;         /* Kyber batches of at most this many requests run one
                                  workgroup per request (latency) instead of the throughput forms
                                  below: 0 = library default (1280 for Kyber-512 and mixed encapsulation,
@@ -100,7 +101,8 @@ typedef struct pqc_tuning {
                                  shared-key decapsulation: calls of at least this many requests run one state
                                  per lane (throughput), smaller ones one state per lane pair, or up to 4096
                                  requests on 16 lanes (latency);
-                                 0 = library default (49152), -1 = lane pairs always, else >= 1 */
+                                 0 = library default (49152), -1 = lane pairs always (also up to 4096),
+                                 else >= 1 */
 } pqc_tuning;
 int pqc_ctx_get_tuning(const pqc_ctx *ctx, pqc_tuning *t);
 int pqc_ctx_put_tuning(pqc_ctx *ctx, const pqc_tuning *t); /* PQC_ERR_INVALID_ARG outside the ranges */

@@ -1273,7 +1273,7 @@ static FrKeys loaded_key(pqc_ctx* c) {
 // would at three waves per SIMD.  16 lanes cost more of the chip's time per permutation, so
 // four such calls side by side gain less: 2932 -> 3162 for decapsulations of 4096 (slower),
 // 2367 -> 1897 for 2048, 3886 -> 2985 for encapsulations of 4096.
-constexpr int kWideMax = 4096;
+constexpr int kWideMax = kFrodoWideMax;
 
 static void launch_f_full(const pqc_ctx* c, int ni, uint8_t* ss, const uint8_t* ct, const uint8_t* kp, hipStream_t s) {
   const int waves = (ni + 3) / 4;
@@ -1298,8 +1298,8 @@ static void launch_pkh(const pqc_ctx* c, int m, uint8_t* pkh, size_t out_stride,
     hipLaunchKernelGGL(k_pkh_many, dim3((2 * m + 63) / 64), dim3(64), 0, s, m, pkh, out_stride, pk, pk_stride);
 }
 
-// G2 and the S'/E'/E'' stream of n requests (lane pairs; with_f adds the F prefix
-// of each ciphertext), then its sampling into the ROWS or fragment layouts.
+// G2 and the S'/E'/E'' stream of n requests (with_f adds the F prefix of each
+// ciphertext), then its sampling into the ROWS or fragment layouts.
 template <bool ROWS>
 static void launch_stream(pqc_ctx* c, const FrScratch& f, int ni, int with_f, const FrKeys& keys, const uint8_t* mu,
                           int mu_stride, const uint8_t* ct, hipStream_t s) {
@@ -1307,7 +1307,9 @@ static void launch_stream(pqc_ctx* c, const FrScratch& f, int ni, int with_f, co
   // shared-key decapsulation: its F-prefix lanes share the SIMDs with the stream
   // lanes.  Encapsulation on single lanes runs one wave per SIMD (4.4 against 3.4 ms
   // on pairs at 32768, no faster at 65536); the keyed paths run at most a server batch
-  if (!ROWS && with_f && frodo_lanes(c->tune, (uint64_t)ni)) {
+  const FrodoLayout layout =
+      !ROWS && with_f ? frodo_layout(c->tune, (uint64_t)ni) : ni <= kWideMax ? kFrodoWide : kFrodoPairs;
+  if (layout == kFrodoLanes) {
     const int nlane = (ni + 63) / 64 * 64, lanes = nlane + (with_f ? ni : 0);
     hipLaunchKernelGGL(k_shake_lane, dim3((lanes + sb - 1) / sb), dim3(sb), 0, s, ni, nlane, with_f, keys, mu,
                        mu_stride, f.raw, f.kp, ct, with_f ? reinterpret_cast<uint64_t*>(f.fstate) : nullptr);
@@ -1315,7 +1317,7 @@ static void launch_stream(pqc_ctx* c, const FrScratch& f, int ni, int with_f, co
                        f.sfrag, f.efrag);
     return;
   }
-  if (ni <= kWideMax) {
+  if (layout == kFrodoWide) {
     const int waves = (with_f ? 2 : 1) * ((ni + 3) / 4);
     wide::with_wg(c->cu_count, waves, [&](auto wg) {
       constexpr int WG = decltype(wg)::value;

@@ -10,12 +10,16 @@
 
 constexpr int kFrSideStreams = 3;
 
-// FrodoKEM-976 shared-key calls of at least this many requests run the noise
-// stream with one Keccak state per lane (tuning.frodo_lane_min = 0)
-constexpr int kFrodoLaneMinDefault = 49152;
-inline bool frodo_lanes(const pqc_tuning& t, uint64_t n) {
+// Keccak lane layout of the noise stream and F prefix in FrodoKEM-976 shared-key
+// decapsulations of n requests (tuning.frodo_lane_min): one state per lane from
+// frodo_lane_min on, 16 lanes per state up to kFrodoWideMax, else, or with -1 always,
+// lane pairs
+constexpr int kFrodoLaneMinDefault = 49152, kFrodoWideMax = 4096;
+enum FrodoLayout { kFrodoWide, kFrodoPairs, kFrodoLanes };
+inline FrodoLayout frodo_layout(const pqc_tuning& t, uint64_t n) {
   const int m = t.frodo_lane_min == 0 ? kFrodoLaneMinDefault : t.frodo_lane_min;
-  return m > 0 && n >= (uint64_t)m;
+  if (m < 0) return kFrodoPairs;
+  return n >= (uint64_t)m ? kFrodoLanes : n <= (uint64_t)kFrodoWideMax ? kFrodoWide : kFrodoPairs;
 }
 
 struct pqc_ctx {

@@ -42,8 +42,9 @@ static int mixed_layout(const pqc_tuning& t) {
 }
 
 // one-hot family (5), K / 4, op / 2, log2(n) / 17, log2(block) / 10, waves / 4,
-// mixed tile layout one-hot (4); for the Frodo family, slot 10 is the stream's
-// Keccak lane layout at this n (1 = one state per lane)
+// mixed tile layout one-hot (4); for the Frodo family, the stream's Keccak lane
+// layout at this n: slot 9 = 16 lanes per state (the block size plays no part
+// then), slot 10 = one state per lane
 static void features(const pqc_tune_request& r, const pqc_tuning& t, float* f) {
   for (int i = 0; i < kFeatures; ++i) f[i] = 0.f;
   if (r.family >= 0 && r.family < 5) f[r.family] = 1.f;
@@ -61,7 +62,10 @@ static void features(const pqc_tune_request& r, const pqc_tuning& t, float* f) {
   const bool fused = r.family == PQC_TUNE_FUSED_KYBER || r.family == PQC_TUNE_MIXED_KYBER;
   f[9] = fused ? (float)t.fused_waves_per_cu / 4.f : 0.f;
   if (r.family == PQC_TUNE_MIXED_KYBER) f[10 + mixed_layout(t)] = 1.f;
-  if (r.family == PQC_TUNE_FRODO) f[10] = frodo_lanes(t, r.n) ? 1.f : 0.f;
+  if (r.family == PQC_TUNE_FRODO) {
+    f[9] = frodo_layout(t, r.n) == kFrodoWide ? 1.f : 0.f;
+    f[10] = frodo_layout(t, r.n) == kFrodoLanes ? 1.f : 0.f;
+  }
 }
 
 static std::vector<pqc_tuning> candidates(const pqc_tune_request& r, const pqc_tuning& base) {
@@ -99,17 +103,27 @@ static std::vector<pqc_tuning> candidates(const pqc_tune_request& r, const pqc_t
           add(t);
         }
       break;
-    case PQC_TUNE_FRODO:
-      // block size x Keccak lane layout at this n (lane pairs or one state per lane);
-      // the layout in use keeps its threshold, so the configuration in use is a candidate
-      for (int lanes = 0; lanes < 2; ++lanes)
+    case PQC_TUNE_FRODO: {
+      // Keccak lane layout at this n x block size where it plays a part (not on 16 lanes per
+      // state, which there is up to kFrodoWideMax requests).  Six candidates either way:
+      // below, where one state per lane is far off, it gets two block sizes.  The layout
+      // in use keeps its threshold and its block size is among those measured, so the
+      // configuration in use is a candidate.
+      const FrodoLayout used = frodo_layout(base, r.n);
+      const bool wide = r.n <= (uint64_t)kFrodoWideMax;
+      for (FrodoLayout l : {kFrodoWide, kFrodoPairs, kFrodoLanes}) {
+        if (l == kFrodoWide && !wide) continue;
         for (int b : {64, 128, 256}) {
+          if (l == kFrodoWide && b != base.frodo_stream_block) continue;
+          if (l == kFrodoLanes && wide && b == (base.frodo_stream_block == 128 ? 256 : 128)) continue;
           pqc_tuning t = base;
           t.frodo_stream_block = b;
-          if (frodo_lanes(base, r.n) != (lanes != 0)) t.frodo_lane_min = lanes ? 1 : -1;
+          if (l != used) t.frodo_lane_min = l == kFrodoWide ? 0 : l == kFrodoPairs ? -1 : 1;
           add(t);
         }
+      }
       break;
+    }
     default: break;
   }
   return out;
