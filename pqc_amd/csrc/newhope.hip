@@ -23,6 +23,7 @@
 
 #include "internal.h"
 #include "keccak_wide.cuh"
+#include "newhope_f32.h"
 #include "sponge.cuh"
 
 namespace pqc {
@@ -97,35 +98,6 @@ template <>
 __device__ __forceinline__ const Tables<1024>& tab<1024>() { return c_tab1024; }
 template <>
 __device__ __forceinline__ const Tables<512>& tab<512>() { return c_tab512; }
-
-// ---- exact FP32 arithmetic mod q for the fused kernels' transforms --------------------
-// Values are integers in floats, twiddles plain (no Montgomery factor) and centred
-// (|z| <= 6144).  x z is formed exactly inside v_fma_f32 and reduced by k = round(x z / q)
-// in two exact steps, q = 3 2^12 + 1: x z - 12288 k = r + k, then minus k.  With |x z| / q
-// <= 2^21, 12288 k = 3 k 2^12 and r + k (below 2^24) are exact, and z / q's rounding moves
-// k by at most 2^21 2^-23 = 1/4: |r| < 0.76 q.  Five full-rate instructions; the integer
-// Montgomery product is three 32-bit multiplies at half that rate and five more.
-namespace fp {
-constexpr float kQ = 12289.0f, kQinv = 1.0f / 12289.0f, kM = 12582912.0f;  // kM = 1.5 2^23
-
-// zq = z kQinv
-__device__ __forceinline__ float mul(float x, float z, float zq) {
-  const float k = __builtin_fmaf(x, zq, kM) - kM;
-  return __builtin_fmaf(x, z, k * -12288.0f) - k;
-}
-__device__ __forceinline__ float mul(float x, float z) { return mul(x, z, z * kQinv); }
-// centred residue of |x| <= 2^24
-__device__ __forceinline__ float reduce(float x) {
-  const float k = __builtin_fmaf(x, kQinv, kM) - kM;
-  return __builtin_fmaf(k, -kQ, x);
-}
-// the residue in [0, q) as an integer, |x| <= 2^19: k = floor(x / q) as the rounding of
-// x / q - 1/2 + 1 / (2 q), whose margin 1 / (2 q) exceeds the float error 2^-18
-__device__ __forceinline__ uint32_t canon(float x) {
-  const float k = (__builtin_fmaf(x, kQinv, -0.5f + 0.5f / kQ) + kM) - kM;
-  return __builtin_bit_cast(uint32_t, __builtin_fmaf(k, -kQ, x + kM)) & 0x3FFFu;
-}
-}  // namespace fp
 
 // Plain centred twiddles of the bit-reversed-input, natural-output transforms whose layer
 // L combines sub-transforms of 2^L points: entry 2^L + j belongs to output j of that layer.
@@ -704,10 +676,11 @@ __device__ __forceinline__ int brv_index(int c) {
 
 // The fused kernels' transforms on FP32 values, in ntt_wave's register layouts, the
 // exchanges between its register groups through an LDS buffer of floats.  Butterflies
-// multiply first (a + z b, a - z b): a layer adds 0.76 q to the bound, so nothing is
-// reduced on the way (2^14 + 10 0.76 q < 2^17), the weighting of the input is part of the
-// twiddles, those of the first register group are literals and the others serve several
-// butterflies, two polynomials at a time where there are two.  All of these kernels are
+// multiply first (a + z b, a - z b) and nothing is reduced on the way: a layer adds the
+// bound of a product (the inverse's first register group, whose j = 0 butterflies take
+// z = 1 without a product, doubles; newhope_f32.h has the bounds).  The weighting of the
+// input is part of the twiddles, those of the first register group are literals and the
+// others serve several butterflies, two polynomials at a time where there are two.  All of these kernels are
 // bound by VALU issue (a wave's Keccak-f is 4320 of its ~7000 instructions).  Keypair,
 // encryption and decryption of 16384 elements at N = 1024, us: 180, 215 and 50 with integer
 // Montgomery layers and a branch per gen_a candidate; 160, 175 and 42 with these transforms
