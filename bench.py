@@ -502,8 +502,8 @@ def fixed_rate_latency(rate, duration, keys=1024):
     for plain, graph in ((False, False), (False, True), (True, False)):
         # two slots (one batch on the GPU while the next fills) and batches closed
         # after 25 us, which kept batches near 600 requests on every box measured
-        # (50 us let some settle near 1000, doubling p50).  Batches of up to 8192
-        # decapsulations run the one-workgroup-per-request kernel.
+        # (50 us let some settle near 1000, doubling p50).  Batches of up to 1536
+        # decapsulations run the one-workgroup-per-request kernel, larger ones the stages.
         srv = Server(["kyber768"], keys_per_alg=keys, key_seed=0, max_batch=65536, slots=2,
                      arena_bytes=128 << 20, max_wait_us=25, plain=plain, graph=graph)
         ws = RequestSet.random(algs, ops, kid, rng)

@@ -1337,18 +1337,18 @@ static void launch_stream(pqc_ctx* c, const FrScratch& f, int ni, int with_f, co
 }
 
 // ---- batches under the loaded key, optionally cut into chunks over streams ------
-// One request's S'/E'/E'' stream is a serial chain of 231 permutations on a lane
-// pair (plus a pair for the F prefix), so a batch of 4096 keeps only a quarter of
-// the SIMDs busy while k_shake runs; 16384 requests put one wave on every SIMD.
-// Batches above tune.frodo_chunk requests are cut into chunks of that many, and
+// One request's S'/E'/E'' stream is a serial chain of 231 permutations (and 115 of the F
+// prefix beside it).  On 16 lanes per request a batch of 4096 puts two waves on every
+// SIMD, on lane pairs one of 16384 puts one there.  Batches above tune.frodo_chunk requests are cut into chunks of that many, and
 // chunk i runs its whole chain (w-decode, stream, sampling, shared-A GEMM, F) on
 // stream i mod 4: the caller's stream or one of the context's three side
 // streams, forked from and joined back to the caller's stream by events.  Every
 // chunk has scratch of its own (fr_scratch_at), so the bytes are those of the
-// unsplit batch.  Measured on MI355X, four concurrent 4096-request chains slow
-// each other's k_shake to 1.6-3.2 ms (1.1 ms alone), so one chain over the whole
-// batch is faster than chunks of 4096; the default therefore splits only above
-// 65536 requests, and the knob stays for the autotuner.
+// unsplit batch.  Measured on MI355X, 16384 decapsulations take 1.75 ms as one chain and
+// 3.4 ms in chunks of 4096 (3.5 to 4.2 where the process's hardware queues are fewer than
+// its streams): the four chains share the SIMDs and each needs a whole chain's time.  The
+// default therefore splits only above 65536 requests.  With lane pairs such chunks took 3.25
+// to 3.3 ms (4.0 to 4.4), with one wave of 16 lanes to a SIMD 3.75.
 constexpr size_t kFrPipeChunkDefault = 65536;
 static_assert(kFrPipeChunkDefault % 32 == 0, "chunks start on whole 256-row GEMM blocks");
 

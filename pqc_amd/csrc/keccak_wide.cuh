@@ -15,7 +15,8 @@
 // 180; a wave issues one every ~4.4 cycles, and the LDS round trip adds ~120 cycles.
 // Measured on MI355X, us per permutation at one wave per SIMD: 3.3, against 4.9 for an
 // unrolled interleaved lane pair, 6.3 for the rolled pair, 7.9 for one state per lane; at
-// two waves per SIMD 4.8.  Its throughput is a fifth of the one-state-per-lane form's.
+// two waves per SIMD 4.8.  Its throughput is about a fifth of the one-state-per-lane form's
+// (1.7 G permutations/s at two waves per SIMD, ~2.1 G at more, against 10.1 G).
 #pragma once
 #include <stddef.h>
 

@@ -812,10 +812,11 @@ int kyber_fused_mixed(pqc_ctx* c, int dec, size_t n, const pqc_kem_req* reqs, ui
 }
 
 // ---- allocation-free decapsulation ------------------------------------------------
-// pqc_kyber_dec_batch_noalloc runs the same kernels as crypto_kem_dec_batch on
-// the default tuning, with the tile kernel's PRF scratch and the status word in
-// `scratch`, a file-scope device array (one copy per GPU, held until the process
-// ends) instead of a context's allocation.  The host never names `scratch`
+// pqc_kyber_dec_batch_noalloc gives the bytes of crypto_kem_dec_batch by the two forms
+// that need no context's scratch: the per-request kernels up to 8192 requests, where the
+// context path has been in stages for long, and 64-request tiles above.  The tile
+// kernel's PRF rows and the status word are in `scratch`, a file-scope device array (one
+// copy per GPU, held until the process ends).  The host never names `scratch`
 // directly (in host code it is only a stand-in symbol): the device address is
 // looked up once per device with hipGetSymbolAddress and that address is what
 // the kernels receive.  Nothing in the scratch must start at zero: every PRF
@@ -861,8 +862,8 @@ template <int K>
 int noalloc_dec(const NoAllocDev& d, size_t n, uint8_t* ss, uint8_t* ct, const uint8_t* sk, uint32_t* status,
                 hipStream_t s) {
   using namespace kyber::fused;
-  // a workgroup per request up to where a 64-request tile launch (~1 ms for any batch)
-  // is faster: ~10.6 M decapsulations/s
+  // a workgroup per request up to 8192; a 64-request tile launch is as long for any batch:
+  // us at 8192 / in tiles 276 / 502, 666 / 853, 846 / 1255 for K = 2, 3, 4
   if (n <= 8192) {
     return kyber_lowlat_dec(K, n, ss, ct, sk, status, s);
   } else {

@@ -28,7 +28,7 @@
 //
 // Measured on MI355X, us per call, this path and the 32-request tiles (two waves per
 // SIMD, butterfly transforms) or per-request workgroups it replaced:
-//   Kyber-768 decapsulation, 65536 requests    600    712
+//   Kyber-768 decapsulation, 65536 requests    610    712  (596 to 675 across boxes, 712 to 793)
 //   Kyber-1024 decapsulation, 6000 requests    189    675 (a workgroup per request)
 // At 65536 the sponge stage takes ~370 us (53 permutations per request at 9.4 G/s, the
 // rate of the VALU on this mix), the product stages ~65 and ~140, the KDF ~15.
