@@ -170,7 +170,7 @@ struct Timer {
 constexpr float kWarmMs = 30.f;
 constexpr int kWarmRuns = 1000;
 
-// ms[i]: median time of cand[order[i]], i < n
+// ms[i]: median time of cand[order[i]], i < n; after an error, of those that have run
 static int measure(pqc_ctx* c, const std::vector<pqc_tuning>& cand, const std::vector<size_t>& order, size_t n,
                    pqc_workload_fn run, void* user, hipStream_t s, int reps, std::vector<float>& ms) {
   Timer t;
@@ -186,15 +186,15 @@ static int measure(pqc_ctx* c, const std::vector<pqc_tuning>& cand, const std::v
       c->tune = cand[order[i]];
       if (r == 0) rc = run(user, (void*)s);  // untimed: a configuration's first run
       if (!rc) rc = t.run(run, user, s, &e);
-      v[i].push_back(e);
+      if (!rc) v[i].push_back(e);
     }
-  if (rc) return rc;
   ms.clear();
   for (auto& x : v) {
+    if (x.empty()) break;
     std::sort(x.begin(), x.end());
     ms.push_back(x[x.size() / 2]);
   }
-  return PQC_OK;
+  return rc;
 }
 
 }  // namespace tuner
@@ -286,11 +286,7 @@ int pqc_autotune(pqc_ctx* c, const pqc_tune_request* r, pqc_workload_fn run, voi
   size_t best = order[0];
   std::vector<float> ms;
   int rc = measure(c, cand, order, budget, run, user, s, r->reps, ms);
-  if (rc) {
-    c->tune = start;
-    return rc;
-  }
-  for (size_t j = 0; j < budget; ++j) {
+  for (size_t j = 0; j < ms.size(); ++j) {
     float f[kFeatures];
     features(*r, cand[order[j]], f);
     S->x.insert(S->x.end(), f, f + kFeatures);
@@ -299,6 +295,10 @@ int pqc_autotune(pqc_ctx* c, const pqc_tune_request* r, pqc_workload_fn run, voi
       best_ms = ms[j];
       best = order[j];
     }
+  }
+  if (rc) {
+    c->tune = start;
+    return rc;
   }
   c->tune = cand[best];
   out->best = cand[best];

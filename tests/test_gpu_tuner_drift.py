@@ -34,3 +34,28 @@ def test_slow_first_runs_do_not_change_the_pick():
     assert res.best.fused_waves_per_cu == start
     assert T.get_tuning(ctx).fused_waves_per_cu == start
     ctx.close()
+
+
+def test_a_failing_run_keeps_the_samples_before_it():
+    """A workload that fails in the third candidate's first run: the error is reported, the
+    configuration in use stays, and the two candidates timed before it stay as samples."""
+    import pqc_amd as pqc
+    from pqc_amd import tuner as T
+    ctx, st = pqc.Context(["kyber768"], max_batch=1), pqc.Stream()
+    sk, ct, ss = (pqc.DeviceBuffer.from_array(np.zeros(b, np.uint8)) for b in (2400, 1088, 32))
+    start = T.get_tuning(ctx).as_dict()
+    seen = []
+
+    def run(s):
+        w = T.get_tuning(ctx).fused_waves_per_cu
+        if w not in seen:
+            seen.append(w)
+            if len(seen) == 3:
+                raise ValueError("no")
+        ctx.dec("kyber768", 1, ss, ct, sk, stream=s)
+
+    with pytest.raises(ValueError):
+        T.autotune(ctx, T.request("fused_kyber", 1, k=3, op=2, budget=0, reps=3), run, st)
+    assert len(T.samples(ctx)[1]) == 2
+    assert T.get_tuning(ctx).as_dict() == start
+    ctx.close()
